@@ -62,6 +62,7 @@ struct f2jk_ctx {
     // where B is nonzero for some P
     bool j_sparse = false;
     uint32_t* jlist[2] = {nullptr, nullptr};
+    int* jinv[2] = {nullptr, nullptr};   // lower-triangle element -> place in the list, or -1
     int jlist_vec[2] = {0, 0};
     int jlist_n[2] = {0, 0};
     size_t xchunk_bytes = kDefaultXChunkBytes;
@@ -102,6 +103,8 @@ struct Plan {
     // J
     int jvec = 1, nvec = 0, neg = 0, npc1 = 0, ppw2 = 0, npc2 = 0;
     const uint32_t* jlist = nullptr;  // element list of the J passes (null: every element)
+    const int* jinv = nullptr;        // element -> place in that list
+    int jdense = 0;                   // lower-triangle elements in all
     size_t jb = 8;             // bytes of a B element read by J
     // K
     int Pc = 0, nchunks = 0, ntile = 0, nlower = 0, nsplit = 0, ncolt = 0, kva = 1, nbw = 0, kx_waves = 4;
@@ -158,7 +161,9 @@ int scan_jlist(f2jk_ctx* ctx, const TB* B, unsigned char* flag) {
 
 void free_jlist(f2jk_ctx* ctx, int dtype) {
     if (ctx->jlist[dtype]) (void)hipFree(ctx->jlist[dtype]);
+    if (ctx->jinv[dtype]) (void)hipFree(ctx->jinv[dtype]);
     ctx->jlist[dtype] = nullptr;
+    ctx->jinv[dtype] = nullptr;
     ctx->jlist_vec[dtype] = ctx->jlist_n[dtype] = 0;
 }
 
@@ -186,13 +191,20 @@ int build_jlist(f2jk_ctx* ctx, int dtype) {
     if (rc) return rc;
     if (e != hipSuccess) return fail(F2JK_EHIP, std::string("j_scan flags: ") + hipGetErrorString(e));
     std::vector<uint32_t> list;
+    std::vector<int> inv(nvec, -1);
+    if (std::none_of(h.begin(), h.end(), [](unsigned char f) { return f != 0; }))
+        h[0] = 1;  // an all-zero B: one element keeps the launches non-empty
     int el = 0;
     for (int m = 0; m < N; ++m)
         for (int c = 0; c <= m; c += vec, ++el)
-            if (h[el]) list.push_back(((uint32_t)m << 16) | (uint32_t)c);
-    if (list.empty()) list.push_back(0u);  // an all-zero B: one element keeps the launches non-empty
+            if (h[el]) {
+                inv[el] = (int)list.size();
+                list.push_back(((uint32_t)m << 16) | (uint32_t)c);
+            }
     F2JK_HIP(hipMalloc(&ctx->jlist[dtype], list.size() * sizeof(uint32_t)));
     F2JK_HIP(hipMemcpy(ctx->jlist[dtype], list.data(), list.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    F2JK_HIP(hipMalloc(&ctx->jinv[dtype], inv.size() * sizeof(int)));
+    F2JK_HIP(hipMemcpy(ctx->jinv[dtype], inv.data(), inv.size() * sizeof(int), hipMemcpyHostToDevice));
     ctx->jlist_vec[dtype] = vec;
     ctx->jlist_n[dtype] = (int)list.size();
     return F2JK_OK;
@@ -264,8 +276,10 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         p.jvec = jvec_override ? jvec_override : j_vec_for(jdtype, N);
         int64_t nvec = 0;
         for (int64_t m = 0; m < N; ++m) nvec += (m + 1 + p.jvec - 1) / p.jvec;
+        p.jdense = (int)nvec;
         if (!grouped && ctx->jlist[jdtype] && ctx->jlist_vec[jdtype] == p.jvec) {
             p.jlist = ctx->jlist[jdtype];
+            p.jinv = ctx->jinv[jdtype];
             nvec = ctx->jlist_n[jdtype];
         }
         p.nvec = (int)nvec;
@@ -410,16 +424,8 @@ int launch_j(f2jk_ctx* ctx, const Plan& p, const TB* B, const double* const* D, 
     hipLaunchKernelGGL((j_accum_kernel<TB, VEC, kEPT, ND, NT>), dim3(p.neg, p.npc2), dim3(kJThreads), 0,
                        st, B, p.N, p.Q, gamma, rowoff, elist, p.nvec, p.ppw2, jpart);
     F2JK_LAUNCHED("j_accum");
-    if (elist) {
-        // elements outside the list are exactly zero (B is zero there for every P)
-        const int64_t NN = (int64_t)p.N * p.N;
-        for (int d = 0; d < ND; ++d) {
-            hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)cdiv(NN, 256)), dim3(256), 0, st, J[d], NN);
-            F2JK_LAUNCHED("fill_zero");
-        }
-    }
-    hipLaunchKernelGGL((j_reduce_kernel<VEC, ND>), dim3((unsigned)cdiv(p.nvec, 256)), dim3(256), 0,
-                       st, jpart, p.npc2, p.N, rowoff, elist, p.nvec, jp);
+    hipLaunchKernelGGL((j_reduce_kernel<VEC, ND>), dim3((unsigned)cdiv(p.jdense, kJRedElems)), dim3(kJThreads), 0,
+                       st, jpart, p.npc2, p.N, rowoff, p.jinv, p.nvec, p.jdense, jp);
     F2JK_LAUNCHED("j_reduce");
     TIM(F2JK_PH_JACC, false);
     return F2JK_OK;
@@ -514,7 +520,7 @@ int build_d(f2jk_ctx* ctx, const Plan& p, char* ws, hipStream_t st) {
         hipLaunchKernelGGL(ks_kernel<double>, dim3(nlower), dim3(kGThreads), 0, st, cp, p.N, p.OPAD,
                            p.ioff[d], p.width[d], 1, 1, nlower, dpart, 0);
         F2JK_LAUNCHED("ks(D)");
-        hipLaunchKernelGGL(k_reduce_kernel, dim3((unsigned)cdiv(p.N, 256), p.N), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st,
                            dpart, 1, p.N, dbuf + (size_t)d * p.N * p.N);
         F2JK_LAUNCHED("k_reduce(D)");
     }
@@ -579,7 +585,7 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipStr
     TIM(F2JK_PH_KRED, true);
     const int nsplit_used = std::min(p.nsplit, std::min(p.Pc, p.Q));
     for (int d = 0; d < p.nd; ++d) {
-        hipLaunchKernelGGL(k_reduce_kernel, dim3((unsigned)cdiv(p.N, 256), p.N), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st,
                            kpart + (size_t)d * p.nsplit * NN, nsplit_used, p.N, K[d]);
         F2JK_LAUNCHED("k_reduce");
     }
@@ -684,7 +690,7 @@ int run_k_bf16x3(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipSt
     TIM(F2JK_PH_KRED, true);
     const int nsplit_used = std::min(p.nsplit, std::min(p.Pc, p.Q));
     for (int d = 0; d < p.nd; ++d) {
-        hipLaunchKernelGGL(k_reduce_kernel, dim3((unsigned)cdiv(p.N, 256), p.N), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st,
                            kpart + (size_t)d * p.nsplit * NN, nsplit_used, p.N, K[d]);
         F2JK_LAUNCHED("k_reduce");
     }

@@ -75,26 +75,16 @@ __host__ __device__ inline int phase_blocks(const GJob& g, int phase) {
     switch (phase) {
         case GP_PAD: return gcdiv((long long)(PREC == F2JK_PREC_BF16X3 ? g.KP : g.N) * g.OPAD, 256);
         case GP_DKS: return j * g.nlower * g.nd;
-        case GP_DRED: return j * g.N * gcdiv(g.N, 256) * g.nd;
+        case GP_DRED: return j * k_reduce_blocks(g.N) * g.nd;
         case GP_GAMMA: return j * g.neg * g.npc1;
         case GP_GRED: return j * gcdiv((long long)g.nd * g.Q, 256);
         case GP_JACC: return j * g.neg * g.npc2;
-        case GP_JRED: return j * gcdiv(g.nvec, 256);
+        case GP_JRED: return j * gcdiv(g.nvec, kJRedElems);
         case GP_KX: return gcdiv((long long)g.Q * g.N, kTile) * g.ncolt;
         case GP_KS: return g.nlower * g.nsplit * g.nd;
-        case GP_KRED: return g.N * gcdiv(g.N, 256) * g.nd;
+        case GP_KRED: return k_reduce_blocks(g.N) * g.nd;
     }
     return 0;
-}
-
-// mirrored reduction of split partials: out[m][n] = out[n][m] = sum_s part[s][m][n]
-__device__ __forceinline__ void mirror_reduce(const double* part, int nsplit, int N, double* out, int m, int n) {
-    if (n > m || m >= N) return;
-    const long long NN = (long long)N * N;
-    double acc = 0.0;
-    for (int s = 0; s < nsplit; ++s) acc += part[s * NN + (long long)m * N + n];
-    out[(long long)m * N + n] = acc;
-    out[(long long)n * N + m] = acc;
 }
 
 // PREC: the group's precision; NBW, VA: tile width and load width of the
@@ -146,12 +136,16 @@ void grouped_kernel(const GArgs a) {
             const int d = local / g.nlower, b = local % g.nlower;
             ks_kernel_body<double>(g.Cp, g.N, g.OPAD, g.ioff[d], g.width[d], 1, 1, g.nlower,
                                    g.Dpart + (long long)d * g.N * g.N, 0, b, g.nlower);
-        } else if constexpr (PHASE == GP_DRED) {
-            const int per = g.N * gcdiv(g.N, 256);
-            const int d = local / per, r = local % per;
-            const int m = r / gcdiv(g.N, 256), n = (r % gcdiv(g.N, 256)) * 256 + tid;
+        } else if constexpr (PHASE == GP_DRED || PHASE == GP_KRED) {
+            const int per = k_reduce_blocks(g.N), nb = gcdiv(g.N, 16);
+            const int d = local / per, m4 = local % per / nb, n16 = local % per % nb;
             const long long NN = (long long)g.N * g.N;
-            mirror_reduce(g.Dpart + d * NN, 1, g.N, g.D + d * NN, m, n);
+            if (n16 * 16 <= m4 * 4 + 3) {
+                if constexpr (PHASE == GP_DRED)
+                    k_reduce_body(g.Dpart + d * NN, 1, g.N, g.D + d * NN, m4, n16);
+                else
+                    k_reduce_body(g.Kpart + d * g.nsplit * NN, g.nsplit, g.N, g.K[d], m4, n16);
+            }
         } else if constexpr (PHASE == GP_GAMMA) {
             const int bx = local % g.neg, by = local / g.neg;
             const long long NN = (long long)g.N * g.N;
@@ -179,25 +173,12 @@ void grouped_kernel(const GArgs a) {
             else
                 j_accum_kernel_body<TB, 2, 4, 1>(B, g.N, g.Q, g.gamma, g.rowoff, g.nvec, g.ppw2, g.jpart, bx, by);
         } else if constexpr (PHASE == GP_JRED) {
-            const int e = local * 256 + tid;
-            if (e < g.nvec) {
-                const int m = find_row(g.rowoff, g.N, e);
-                const int col = (e - g.rowoff[m]) * 2;
-                for (int dd = 0; dd < g.nd; ++dd) {
-                    double s0 = 0.0, s1 = 0.0;
-                    for (int c = 0; c < g.npc2; ++c) {
-                        const double* src = g.jpart + (((long long)c * g.nd + dd) * g.nvec + e) * 2;
-                        s0 += src[0];
-                        s1 += src[1];
-                    }
-                    double* Jd = g.J[dd];
-                    Jd[(long long)m * g.N + col] = s0;
-                    Jd[(long long)col * g.N + m] = s0;
-                    if (col + 1 <= m) {
-                        Jd[(long long)m * g.N + col + 1] = s1;
-                        Jd[(long long)(col + 1) * g.N + m] = s1;
-                    }
-                }
+            if (g.nd == 2) {
+                JPtrs<2> jp{{g.J[0], g.J[1]}};
+                j_reduce_body<2, 2>(g.jpart, g.npc2, g.N, g.rowoff, nullptr, g.nvec, g.nvec, jp, local);
+            } else {
+                JPtrs<1> jp{{g.J[0]}};
+                j_reduce_body<2, 1>(g.jpart, g.npc2, g.N, g.rowoff, nullptr, g.nvec, g.nvec, jp, local);
             }
         } else if constexpr (PHASE == GP_KX) {
             const int nb = phase_blocks<PREC>(g, GP_KX);
@@ -223,11 +204,6 @@ void grouped_kernel(const GArgs a) {
                 ks_kernel_body<TB>((const TB*)g.X, g.N, g.OPAD, g.ioff[d], g.width[d], g.Q, g.nsplit, g.nlower,
                                    kp, 0, b, per);
             }
-        } else if constexpr (PHASE == GP_KRED) {
-            const int per = g.N * gcdiv(g.N, 256);
-            const int d = local / per, r = local % per;
-            const int m = r / gcdiv(g.N, 256), n = (r % gcdiv(g.N, 256)) * 256 + tid;
-            mirror_reduce(g.Kpart + (long long)d * g.nsplit * g.N * g.N, g.nsplit, g.N, g.K[d], m, n);
         }
     }
 }

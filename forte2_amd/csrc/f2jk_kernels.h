@@ -349,33 +349,66 @@ __global__ __launch_bounds__(kJThreads) void j_accum_kernel(
 
 
 // J[dd][m][c] = J[dd][c][m] = sum_chunk jpart[chunk][dd][e][v]  (c = col+v <= m)
+// for every lower-triangle vector element; with a list of the elements that
+// the passes ran over, jinv[element] is its place in the list (-1: B is zero
+// there for every P, so is J).  A block holds 64 elements; its four waves sum
+// every fourth chunk each and are added in order: the chunks of a small nbf
+// are many (one per P or two), and one thread per element left the launch a
+// serial chain (33 us at nbf 24 with 139 chunks, 5 us with four waves).
+constexpr int kJRedElems = 64;
 template <int VEC, int ND>
-__global__ void j_reduce_kernel(const double* __restrict__ jpart, int nchunks, int N,
-                                const int* __restrict__ rowoff, const uint32_t* __restrict__ elist, int nvec,
-                                JPtrs<ND> J) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nvec) return;
-    int m, col;
-    j_element<VEC>(rowoff, elist, N, e, m, col);
+__device__ __forceinline__ void j_reduce_body(const double* __restrict__ jpart, int nchunks, int N,
+                                              const int* __restrict__ rowoff, const int* __restrict__ jinv,
+                                              int nlist, int nvec, const JPtrs<ND>& J, int b) {
+    __shared__ double red[3][kJRedElems][ND * VEC];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int e = b * kJRedElems + lane;
+    const int le = e < nvec ? (jinv ? jinv[e] : e) : -1;
+    double s[ND][VEC];
 #pragma unroll
-    for (int dd = 0; dd < ND; ++dd) {
-        double s[VEC];
+    for (int dd = 0; dd < ND; ++dd)
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) s[v] = 0.0;
-        for (int c = 0; c < nchunks; ++c) {
-            const double* src = jpart + (((int64_t)c * ND + dd) * nvec + e) * VEC;
+        for (int v = 0; v < VEC; ++v) s[dd][v] = 0.0;
+    if (le >= 0) {
+#pragma unroll 4
+        for (int c = w; c < nchunks; c += 4)
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) s[v] += src[v];
-        }
+            for (int dd = 0; dd < ND; ++dd) {
+                const Vec<double, VEC> x =
+                    load_vec<double, VEC>(jpart + (((int64_t)c * ND + dd) * nlist + le) * VEC);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-            const int cc = col + v;
-            if (cc <= m) {
-                J.p[dd][(int64_t)m * N + cc] = s[v];
-                J.p[dd][(int64_t)cc * N + m] = s[v];
+                for (int v = 0; v < VEC; ++v) s[dd][v] += x.v[v];
             }
-        }
     }
+    if (w > 0)
+#pragma unroll
+        for (int dd = 0; dd < ND; ++dd)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) red[w - 1][lane][dd * VEC + v] = s[dd][v];
+    __syncthreads();
+    if (w == 0 && e < nvec) {
+        const int m = find_row(rowoff, N, e);
+        const int col = (e - rowoff[m]) * VEC;
+#pragma unroll
+        for (int dd = 0; dd < ND; ++dd)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) {
+                const int i = dd * VEC + v, cc = col + v;
+                const double x = ((s[dd][v] + red[0][lane][i]) + red[1][lane][i]) + red[2][lane][i];
+                if (cc <= m) {
+                    J.p[dd][(int64_t)m * N + cc] = x;
+                    J.p[dd][(int64_t)cc * N + m] = x;
+                }
+            }
+    }
+    __syncthreads();  // red is free again (a persistent block goes on to its next 64 elements)
+}
+template <int VEC, int ND>
+__global__ __launch_bounds__(kJThreads) void j_reduce_kernel(const double* __restrict__ jpart, int nchunks, int N,
+                                                             const int* __restrict__ rowoff,
+                                                             const int* __restrict__ jinv, int nlist, int nvec,
+                                                             JPtrs<ND> J) {
+    j_reduce_body<VEC, ND>(jpart, nchunks, N, rowoff, jinv, nlist, nvec, J, blockIdx.x);
 }
 
 // flag[e] = 1 when B[P][m][c] != 0 for some P and some c <= m of vector
@@ -397,12 +430,6 @@ __global__ void j_scan_kernel(const TB* __restrict__ B, int N, int Q, const int*
         for (int v = 0; v < VEC; ++v) nz |= (col + v <= m) && (b.v[v] != TB(0));
     }
     flag[e] = (unsigned char)nz;
-}
-
-// x[i] = 0 for i < n
-__global__ void fill_zero_kernel(double* __restrict__ x, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = 0.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1663,17 +1690,39 @@ __global__ void x_copy_kernel(const double* __restrict__ X, int64_t R, int OPAD,
     out[r * ldx + c] = X[r * OPAD + c];
 }
 
-// K[m][n] = K[n][m] = sum_s Kpart[s][m][n] for m >= n (fixed order in s).
-__global__ void k_reduce_kernel(const double* __restrict__ Kpart, int nsplit, int N,
-                                double* __restrict__ K) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    const int m = blockIdx.y;
-    if (n > m || m >= N) return;
+// K[m][n] = K[n][m] = sum_s Kpart[s][m][n] for m >= n (fixed order in s).  A
+// block holds 4 rows x 16 columns; its four waves sum every fourth split each
+// and are added in order (one thread per element took 30-60 us below nbf 400,
+// a serial chain over the splits).
+__device__ __forceinline__ void k_reduce_body(const double* __restrict__ Kpart, int nsplit, int N,
+                                              double* __restrict__ K, int m4, int n16) {
+    __shared__ double red[3][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int m = m4 * 4 + (lane >> 4), n = n16 * 16 + (lane & 15);
+    const bool on = m < N && n <= m;
     const int64_t NN = (int64_t)N * N;
-    double acc = 0.0;
-    for (int s = 0; s < nsplit; ++s) acc += Kpart[s * NN + (int64_t)m * N + n];
-    K[(int64_t)m * N + n] = acc;
-    K[(int64_t)n * N + m] = acc;
+    double s = 0.0;
+    if (on) {
+        const double* p = Kpart + (int64_t)m * N + n;
+#pragma unroll 4
+        for (int c = w; c < nsplit; c += 4) s += p[c * NN];
+    }
+    if (w > 0) red[w - 1][lane] = s;
+    __syncthreads();
+    if (w == 0 && on) {
+        s = ((s + red[0][lane]) + red[1][lane]) + red[2][lane];
+        K[(int64_t)m * N + n] = s;
+        K[(int64_t)n * N + m] = s;
+    }
+    __syncthreads();
+}
+// blocks of the reduction of one N x N matrix (n16 past the diagonal: nothing to do)
+__host__ __device__ inline int k_reduce_blocks(int N) { return ((N + 3) / 4) * ((N + 15) / 16); }
+__global__ __launch_bounds__(256) void k_reduce_kernel(const double* __restrict__ Kpart, int nsplit, int N,
+                                                       double* __restrict__ K) {
+    const int nb = (N + 15) / 16, m4 = blockIdx.x / nb, n16 = blockIdx.x % nb;
+    if (n16 * 16 > m4 * 4 + 3) return;
+    k_reduce_body(Kpart, nsplit, N, K, m4, n16);
 }
 
 // Cp[n][ioff + i] = C[n][i] (i < nocc), zero for nocc <= i < width.
