@@ -11,6 +11,7 @@
 
 #include "f2jk.h"
 #include "f2jk_kernels.h"
+#include "f2jk_fp64.h"
 #include "f2jk_group.h"
 
 using namespace f2jk;
@@ -110,11 +111,13 @@ struct Plan {
     int Pc = 0, nchunks = 0, ntile = 0, nlower = 0, nsplit = 0, ncolt = 0, kva = 1, nbw = 0, kx_waves = 4;
     int ks_tile = 128;  // edge of the contraction's lower tiles (256: BF16x3 8-wave tiles)
     int kx_rows = 128;  // rows of a BF16x3 half-transform tile (256: the tall kernel)
-    bool kx_wide = false;  // FP64/FP32 half-transform in 320-column tiles (kx_wide_kernel)
+    bool kx_wide = false;  // FP32 half-transform in 320-column tiles (kx_wide_kernel)
+    int dnb = 0, dncolt = 0, dnks = 0;  // FP64 half-transform: column blocks of a tile, tiles, 16-k steps
+    size_t per_p = 0;      // bytes of X per P
     int ctrows = 0;     // rows of the padded bf16 coefficient planes (>= ncolt * tile columns)
     // workspace offsets
     int KP = 0;                // nbf rounded up to the bf16 k step
-    size_t off_cp32 = 0, off_cth = 0, off_ctl = 0;
+    size_t off_cp32 = 0, off_cth = 0, off_ctl = 0, off_cq = 0;
     size_t off_cp = 0, off_d = 0, off_dpart = 0, off_gpart = 0, off_gamma = 0, off_jpart = 0,
            off_x = 0, off_kpart = 0, total = 0;
     // sizes of the regions that scale with the launch-shape knobs
@@ -260,6 +263,15 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         off += align_up((size_t)N * p.OPAD * 8);
         p.off_cp32 = off;
         off += align_up((size_t)N * p.OPAD * 4);  // fp32 copy (FP32 K)
+        if (precision == F2JK_PREC_FP64 && p.want_k) {
+            // column tiles of equal width, at most 20 blocks of 16
+            const int nb = (int)cdiv(p.OPAD, 16);
+            p.dncolt = (int)cdiv(nb, kDMaxNB);
+            p.dnb = (int)cdiv(nb, p.dncolt);
+            p.dnks = (int)cdiv(N, kDK);
+            p.off_cq = off;
+            off += align_up((size_t)p.dncolt * p.dnks * p.dnb * 256 * 8);
+        }
         p.KP = (int)(cdiv(N, kBK16) * kBK16);
         if (precision == F2JK_PREC_BF16X3) {
             // transposed hi/lo bf16 copies (BF16X3 K), with zero rows up to a
@@ -306,6 +318,8 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         const size_t per_p = (size_t)N * p.OPAD * p.tk;
         int64_t pc = (int64_t)(xchunk_bytes / std::max<size_t>(per_p, 1));
         pc = std::max<int64_t>(1, std::min<int64_t>(pc, Q));
+        pc = std::min<int64_t>(pc, INT32_MAX / N);  // rows of a chunk are numbered in 32 bits
+        p.per_p = per_p;
         // as many chunks as the cap needs, of balanced size: no short last
         // chunk whose launches would be all set-up and Kpart traffic
         pc = cdiv(Q, cdiv(Q, pc));
@@ -349,7 +363,7 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
             p.nbw = best;
             p.kx_waves = ctx->kx_waves;
             p.ncolt = (int)cdiv(p.OPAD, 32 * p.nbw);
-        } else {
+        } else if (precision == F2JK_PREC_FP32) {
             // one 320-column tile reads each row block of B once (the
             // 128-column kernel once per column tile)
             p.kx_wide = !grouped && (ctx->kx_wide < 0 ? p.OPAD > kTile : ctx->kx_wide == 1);
@@ -471,10 +485,35 @@ int run_j(f2jk_ctx* ctx, const Plan& p, const double* const* D, int64_t ldd, dou
 }
 
 // --------------------------------------------------------------------------- C packing, D
+DCols dcols_of(const Plan& p, const int64_t* nocc) {
+    DCols dc{};
+    dc.nd = p.nd;
+    for (int d = 0; d < p.nd; ++d) {
+        dc.nocc[d] = (int)nocc[d];
+        dc.width[d] = p.width[d];
+        dc.ioff[d] = p.ioff[d];
+    }
+    return dc;
+}
+
 int pack_c(f2jk_ctx* ctx, const Plan& p, const double* const* C, const int64_t* nocc,
            const int64_t* ldc, char* ws, hipStream_t st, bool want_f32) {
     double* cp = (double*)(ws + p.off_cp);
     float* cp32 = (float*)(ws + p.off_cp32);
+    if (p.want_k && p.prec == F2JK_PREC_FP64) {
+        DCoef cs{};
+        for (int d = 0; d < p.nd; ++d) {
+            if (nocc[d] > 0 && (!C[d] || !ldc || ldc[d] < nocc[d]))
+                return fail(F2JK_EINVAL, "C pointer / ldc invalid");
+            cs.C[d] = C[d];
+            cs.ldc[d] = nocc[d] > 0 ? ldc[d] : 1;
+        }
+        const int64_t n = (int64_t)p.dncolt * p.dnks * p.dnb * 256;
+        hipLaunchKernelGGL(pack_cq_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, cs, dcols_of(p, nocc), p.N,
+                           p.OPAD, p.dnb, p.dnks, n, cp, (double*)(ws + p.off_cq));
+        F2JK_LAUNCHED("pack_cq");
+        return F2JK_OK;
+    }
     for (int d = 0; d < p.nd; ++d) {
         if (nocc[d] > 0 && (!C[d] || !ldc || ldc[d] < nocc[d]))
             return fail(F2JK_EINVAL, "C pointer / ldc invalid");
@@ -528,30 +567,60 @@ int build_d(f2jk_ctx* ctx, const Plan& p, char* ws, hipStream_t st) {
 }
 
 // --------------------------------------------------------------------------- K
-// X = A Cp over `grid` tiles: 128 x 320 tiles (kx_wide_kernel) or 128 x 128
+// X = A Cp (FP32) over `grid` tiles: 128 x 320 tiles (kx_wide_kernel) or 128 x 128
 // (kx_kernel), as the plan's column tiling says
-template <typename T>
-void launch_kx_typed(const Plan& p, unsigned grid, const T* A, int64_t R, const T* cp, T* X, hipStream_t st) {
-    constexpr int V4 = sizeof(T) == 4 ? 4 : 2;
+void launch_kx_fp32(const Plan& p, unsigned grid, const float* A, int64_t R, const float* cp, float* X,
+                    hipStream_t st) {
     if (p.kx_wide) {
         if (p.kva == 4)
-            hipLaunchKernelGGL((kx_wide_kernel<T, V4>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
+            hipLaunchKernelGGL((kx_wide_kernel<float, 4>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
                                p.OPAD, X, p.ncolt);
         else if (p.kva == 2)
-            hipLaunchKernelGGL((kx_wide_kernel<T, 2>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
+            hipLaunchKernelGGL((kx_wide_kernel<float, 2>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
                                p.OPAD, X, p.ncolt);
         else
-            hipLaunchKernelGGL((kx_wide_kernel<T, 1>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
+            hipLaunchKernelGGL((kx_wide_kernel<float, 1>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
                                p.OPAD, X, p.ncolt);
     } else if (p.kva == 4) {
-        hipLaunchKernelGGL((kx_kernel<T, V4>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
+        hipLaunchKernelGGL((kx_kernel<float, 4>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
                            p.ncolt);
     } else if (p.kva == 2) {
-        hipLaunchKernelGGL((kx_kernel<T, 2>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
+        hipLaunchKernelGGL((kx_kernel<float, 2>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
                            p.ncolt);
     } else {
-        hipLaunchKernelGGL((kx_kernel<T, 1>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
+        hipLaunchKernelGGL((kx_kernel<float, 1>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
                            p.ncolt);
+    }
+}
+
+// FP64 half-transform of R rows: kxd_ib row blocks per wave when that still
+// gives two workgroups to every CU, one otherwise (the products of an element
+// of X and their order do not depend on it).
+constexpr int kDSlots = 512;  // workgroups that run at once: two per CU
+
+template <int NB, int IB>
+void launch_kxd_ib(const Plan& p, const double* A, int64_t R, const double* cq, double* X, int64_t ldx, int ncol,
+                   hipStream_t st) {
+    const unsigned grid = (unsigned)(cdiv(R, 64 * IB) * p.dncolt);
+    hipLaunchKernelGGL((kxd_kernel<NB, IB>), dim3(grid), dim3(256), 0, st, A, R, p.N, cq, p.dnks, X, ldx, ncol,
+                       p.dncolt);
+}
+template <int NB>
+void launch_kxd_nb(const Plan& p, const double* A, int64_t R, const double* cq, double* X, int64_t ldx, int ncol,
+                   hipStream_t st) {
+    constexpr int IB = kxd_ib(NB);
+    if constexpr (IB >= 2) {
+        if (cdiv(R, 64 * IB) * p.dncolt >= kDSlots)
+            return launch_kxd_ib<NB, IB>(p, A, R, cq, X, ldx, ncol, st);
+    }
+    launch_kxd_ib<NB, 1>(p, A, R, cq, X, ldx, ncol, st);
+}
+template <int NB = 1>
+void launch_kxd(const Plan& p, const double* A, int64_t R, const double* cq, double* X, int64_t ldx, int ncol,
+                hipStream_t st) {
+    if constexpr (NB <= kDMaxNB) {
+        if (p.dnb == NB) return launch_kxd_nb<NB>(p, A, R, cq, X, ldx, ncol, st);
+        launch_kxd<NB + 1>(p, A, R, cq, X, ldx, ncol, st);
     }
 }
 
@@ -569,7 +638,10 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipStr
         const int64_t nrowt = cdiv(R, kTile);
         TIM(F2JK_PH_KX, true);
         const T* A = B + (int64_t)P0 * NN;
-        launch_kx_typed<T>(p, (unsigned)(nrowt * p.ncolt), A, R, cp, X, st);
+        if constexpr (sizeof(T) == 8)
+            launch_kxd(p, A, R, (const double*)(ws + p.off_cq), X, p.OPAD, p.OPAD, st);
+        else
+            launch_kx_fp32(p, (unsigned)(nrowt * p.ncolt), A, R, cp, X, st);
         F2JK_LAUNCHED("kx");
         TIM(F2JK_PH_KX, false);
         TIM(F2JK_PH_KS, true);
@@ -1183,6 +1255,10 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
         g.rowoff = want_j ? ctxs[j]->rowoff[p.jvec] : nullptr;
         g.Cp = (double*)(w + p.off_cp);
         g.Cp32 = (float*)(w + p.off_cp32);
+        g.Cq = (double*)(w + p.off_cq);
+        g.dnb = p.dnb;
+        g.dncolt = p.dncolt;
+        g.dnks = p.dnks;
         if (precision == F2JK_PREC_BF16X3) {
             g.Cth = (u16*)(w + p.off_cth);
             g.Ctl = (u16*)(w + p.off_ctl);
@@ -1264,25 +1340,13 @@ int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ld
     const int64_t lds[1] = {ldc};
     if ((rc = pack_c(ctx, p, Cs, &ncol, lds, w, st, false))) return rc;
     const double* B = (const double*)ctx->B[F2JK_F64];
-    const double* cp = (const double*)(w + p.off_cp);
-    double* Xc = (double*)(w + p.off_x);
+    const double* cq = (const double*)(w + p.off_cq);
     const int64_t NN = (int64_t)p.N * p.N;
-    // the kernel writes rows of OPAD columns: straight into the caller's X
-    // when its row stride is exactly that, through the workspace otherwise
-    const bool direct = (ldx == p.OPAD);
-    for (int64_t P0 = p0; P0 < p1; P0 += p.Pc) {
-        const int pc = (int)std::min<int64_t>(p.Pc, p1 - P0);
-        const int64_t R = (int64_t)pc * p.N;
-        const unsigned grid = (unsigned)(cdiv(R, kTile) * p.ncolt);
-        double* dst = X + (P0 - p0) * p.N * ldx;
-        double* Xo = direct ? dst : Xc;
-        launch_kx_typed<double>(p, grid, B + (int64_t)P0 * NN, R, cp, Xo, st);
+    const int64_t step = INT32_MAX / p.N;  // rows of a launch are numbered in 32 bits
+    for (int64_t P0 = p0; P0 < p1; P0 += step) {
+        const int64_t R = std::min<int64_t>(step, p1 - P0) * p.N;
+        launch_kxd(p, B + P0 * NN, R, cq, X + (P0 - p0) * p.N * ldx, ldx, (int)ncol, st);
         F2JK_LAUNCHED("kx");
-        if (!direct) {
-            hipLaunchKernelGGL(x_copy_kernel, dim3((unsigned)cdiv(R * ncol, 256)), dim3(256), 0, st, Xc, R,
-                               p.OPAD, (int)ncol, dst, ldx);
-            F2JK_LAUNCHED("x_copy");
-        }
     }
     g_last_error.clear();
     return F2JK_OK;

@@ -23,6 +23,7 @@
 
 #include "f2jk.h"
 #include "f2jk_kernels.h"
+#include "f2jk_fp64.h"
 
 namespace f2jk {
 
@@ -48,15 +49,17 @@ struct GJob {
     const int* rowoff;
     const double* C[2];
     double *Cp, *D, *Dpart, *gpart, *gamma, *jpart, *Kpart;
+    double* Cq;           // coefficients in the FP64 half-transform's order (FP64 K)
     float* Cp32;          // FP32 coefficients (FP32 K)
     u16 *Cth, *Ctl;       // transposed hi/lo coefficients (BF16x3 K)
     void* X;              // half-transformed chunk: FP64, FP32, or hi then lo bf16
     double* J[2];
     double* K[2];
-    long long ldc[2];
+    int64_t ldc[2];
     int N, Q, nd, nocc[2], width[2], ioff[2], OPAD, KP;
     int nvec, neg, npc1, npc2, ppw2;
     int nlower, nsplit, ncolt;
+    int dnb, dncolt, dnks;  // FP64 half-transform
     int want_j;
 };
 
@@ -73,18 +76,34 @@ template <int PREC>
 __host__ __device__ inline int phase_blocks(const GJob& g, int phase) {
     const int j = g.want_j ? 1 : 0;
     switch (phase) {
-        case GP_PAD: return gcdiv((long long)(PREC == F2JK_PREC_BF16X3 ? g.KP : g.N) * g.OPAD, 256);
+        case GP_PAD:
+            if (PREC == F2JK_PREC_FP64) return g.dncolt * g.dnks * g.dnb;
+            return gcdiv((long long)(PREC == F2JK_PREC_BF16X3 ? g.KP : g.N) * g.OPAD, 256);
         case GP_DKS: return j * g.nlower * g.nd;
         case GP_DRED: return j * k_reduce_blocks(g.N) * g.nd;
         case GP_GAMMA: return j * g.neg * g.npc1;
         case GP_GRED: return j * gcdiv((long long)g.nd * g.Q, 256);
         case GP_JACC: return j * g.neg * g.npc2;
         case GP_JRED: return j * gcdiv(g.nvec, kJRedElems);
-        case GP_KX: return gcdiv((long long)g.Q * g.N, kTile) * g.ncolt;
+        case GP_KX:
+            if (PREC == F2JK_PREC_FP64) return gcdiv((long long)g.Q * g.N, 64 * kxd_ib(g.dnb)) * g.dncolt;
+            return gcdiv((long long)g.Q * g.N, kTile) * g.ncolt;
         case GP_KS: return g.nlower * g.nsplit * g.nd;
         case GP_KRED: return k_reduce_blocks(g.N) * g.nd;
     }
     return 0;
+}
+
+// the FP64 half-transform of one job: the kernel of its width
+template <int NB = 1>
+__device__ __forceinline__ void grouped_kxd(char* lds, const GJob& g, int b, int nblocks) {
+    if constexpr (NB <= kDMaxNB) {
+        if (g.dnb == NB)
+            kxd_body<NB, kxd_ib(NB)>(lds, (const double*)g.B, (long long)g.Q * g.N, g.N, g.Cq, g.dnks, (double*)g.X,
+                                     g.OPAD, g.OPAD, g.dncolt, b, nblocks);
+        else
+            grouped_kxd<NB + 1>(lds, g, b, nblocks);
+    }
 }
 
 // PREC: the group's precision; NBW, VA: tile width and load width of the
@@ -124,13 +143,15 @@ void grouped_kernel(const GArgs a) {
                     g.Ctl[t] = __builtin_bit_cast(u16, l);
                     if (k < g.N) g.Cp[(long long)k * g.OPAD + c] = x;
                 }
+            } else if constexpr (PREC == F2JK_PREC_FP64) {
+                pack_cq_element(g.C, g.ldc, g.nd, g.nocc, g.ioff, g.N, g.OPAD, g.dnb, g.dnks, t, g.Cp, g.Cq);
             } else if (t < (long long)g.N * g.OPAD) {
                 const int n = (int)(t / g.OPAD), c = (int)(t % g.OPAD);
                 const int d = (g.nd == 2 && c >= g.ioff[1]) ? 1 : 0;
                 const int i = c - g.ioff[d];
                 const double x = (i < g.nocc[d]) ? g.C[d][(long long)n * g.ldc[d] + i] : 0.0;
                 g.Cp[t] = x;
-                if constexpr (PREC == F2JK_PREC_FP32) g.Cp32[t] = (float)x;
+                g.Cp32[t] = (float)x;
             }
         } else if constexpr (PHASE == GP_DKS) {
             const int d = local / g.nlower, b = local % g.nlower;
@@ -184,7 +205,8 @@ void grouped_kernel(const GArgs a) {
             const int nb = phase_blocks<PREC>(g, GP_KX);
             const long long R = (long long)g.Q * g.N;
             if constexpr (PREC == F2JK_PREC_FP64) {
-                kx_kernel_body<double, 2>((const double*)g.B, R, g.N, g.Cp, g.OPAD, (double*)g.X, g.ncolt, local, nb);
+                __shared__ __attribute__((aligned(16))) char lds[kDKxLds(kDMaxNB)];
+                grouped_kxd(lds, g, local, nb);
             } else if constexpr (PREC == F2JK_PREC_FP32) {
                 kx_kernel_body<float, 2>((const float*)g.B, R, g.N, g.Cp32, g.OPAD, (float*)g.X, g.ncolt, local, nb);
             } else {

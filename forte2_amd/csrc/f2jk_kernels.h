@@ -1679,17 +1679,6 @@ __global__ __launch_bounds__(64 * WR * WC, (TS == 128 ? 2 : 1)) void ks_bf16x3_d
                                    blockIdx.x, gridDim.x);
 }
 
-// out[r][c] = X[r][c] for r < R, c < ncol: a half-transformed chunk (row
-// stride OPAD) copied to a caller buffer with row stride ldx.
-__global__ void x_copy_kernel(const double* __restrict__ X, int64_t R, int OPAD, int ncol,
-                              double* __restrict__ out, int64_t ldx) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= R * ncol) return;
-    const int64_t r = t / ncol;
-    const int c = (int)(t % ncol);
-    out[r * ldx + c] = X[r * OPAD + c];
-}
-
 // K[m][n] = K[n][m] = sum_s Kpart[s][m][n] for m >= n (fixed order in s).  A
 // block holds 4 rows x 16 columns; its four waves sum every fourth split each
 // and are added in order (one thread per element took 30-60 us below nbf 400,
