@@ -114,6 +114,7 @@ struct Plan {
     bool kx_wide = false;  // FP32 half-transform in 320-column tiles (kx_wide_kernel)
     int dnb = 0, dncolt = 0, dnks = 0;  // FP64 half-transform: column blocks of a tile, tiles, 16-k steps
     size_t per_p = 0;      // bytes of X per P
+    DTiles dt{};           // FP64 contraction: tiles and their P splits
     int ctrows = 0;     // rows of the padded bf16 coefficient planes (>= ncolt * tile columns)
     // workspace offsets
     int KP = 0;                // nbf rounded up to the bf16 k step
@@ -213,6 +214,62 @@ int build_jlist(f2jk_ctx* ctx, int dtype) {
     return F2JK_OK;
 }
 
+constexpr int kDSlots = 512;  // workgroups of the FP64 K kernels that run at once: two per CU
+
+// Tiles of the FP64 contraction of an N x N matrix and the P splits of each
+// kind, in proportion to the cost of a tile: the blocks of its busiest wave,
+// 1.6 times that for a diagonal tile (its waves read two fragments per block
+// and lose the matrix pipe to full tiles on the same CU: workgroups of a
+// diagonal tile took 2.1 times their share of blocks).  All workgroups at
+// once (512) is best when the shares round well; a tile count that does not
+// fit runs in more, shorter workgroups that even out over several rounds, at
+// ~5 us a round and the traffic of their partials.  The estimate below orders
+// the measured times of nbf 318 (64.7 us at 512 workgroups, 71 at 1024, 85 at
+// 2048), 384 (491, 562, 529), 960 (6.2-7.1 ms, 5.6, 5.3, 4.9 at 4096) and 1152
+// (8.1-9.0 ms, 9.1, 8.6, 8.3).
+DTiles dtile_plan(int N, int64_t Pc, int width, int slots) {
+    DTiles m{};
+    m.nt = (int)cdiv(N, kTile);
+    m.rl = (int)cdiv(N - (m.nt - 1) * kTile, 16);
+    m.cnt[0] = (m.nt - 1) * (m.nt - 2) / 2;
+    m.cnt[1] = m.nt - 1;
+    m.cnt[2] = m.nt - 1;
+    m.cnt[3] = 1;
+    const double cost[4] = {16, 1.6 * 9, 4.0 * ((m.rl + 1) / 2), 1.6 * ((m.rl * (m.rl + 1) / 2 + 3) / 4)};
+    const double unit_us = 0.225 * (double)cdiv(width, kDK);  // one block for one P, two workgroups on the CU
+    double sum = 0;
+    for (int k = 0; k < 4; ++k) sum += m.cnt[k] * cost[k];
+    double best = -1;
+    for (int r : {1, 2, 4, 8})
+        for (int i = 0; i < 4; ++i) {
+            const double target = (double)slots * r * (1.0 - 0.04 * i);
+            int ns[4], total = 0, G = 1;
+            double work = 0, longest = 0;
+            for (int k = 0; k < 4; ++k) {
+                ns[k] = (int)std::max<int64_t>(1, std::min<int64_t>(Pc, (int64_t)(target * cost[k] / sum)));
+                total += m.cnt[k] * ns[k];
+                if (!m.cnt[k]) continue;
+                G = std::max(G, ns[k]);
+                longest = std::max(longest, cost[k] * (double)cdiv(Pc, ns[k]));
+            }
+            // the partials stay within the workspace the serving layer reserves for a job
+            if (G > 80 + (8 << 20) / ((int64_t)N * N) && best >= 0) continue;
+            work = sum * (double)Pc / slots;
+            const int rounds = (int)cdiv(total, slots);
+            // one round ends with its longest workgroup; several fill in behind each other
+            const double span = rounds == 1 ? longest : std::max(work, longest) + 0.6 * longest;
+            const double us = span * unit_us + 5.0 * rounds + (double)G * N * N * 8 / 8e6;
+            if (best < 0 || us < best) {
+                best = us;
+                for (int k = 0; k < 4; ++k) m.ns[k] = ns[k];
+                m.G = G;
+                m.total = total;
+            }
+            if ((int64_t)slots * r < 256) break;  // a small cap: no variants
+        }
+    return m;
+}
+
 // Limits of a plan that are otherwise the context's launch-shape knobs; the
 // no-alloc entry point lowers them until the plan fits its scratch array.
 struct PlanCaps {
@@ -257,7 +314,7 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
             p.ioff[d] = o;
             o += p.width[d];
         }
-        p.OPAD = o;
+        p.OPAD = (int)cdiv(o, 16) * 16;
         // the C copy used for D (always fp64) and the K copy (fp64 or fp32)
         p.off_cp = off;
         off += align_up((size_t)N * p.OPAD * 8);
@@ -376,6 +433,10 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         p.off_x = off;
         p.x_bytes = align_up((size_t)p.Pc * per_p);
         off += p.x_bytes;
+        if (precision == F2JK_PREC_FP64) {
+            p.dt = dtile_plan(N, pc, p.width[0], (int)std::min<int64_t>(kDSlots, target_blocks));
+            p.nsplit = p.dt.G;  // partials held per density
+        }
         p.off_kpart = off;
         p.kpart_bytes = align_up((size_t)p.nsplit * ndens * N * N * 8);
         off += p.kpart_bytes;
@@ -596,8 +657,6 @@ void launch_kx_fp32(const Plan& p, unsigned grid, const float* A, int64_t R, con
 // FP64 half-transform of R rows: kxd_ib row blocks per wave when that still
 // gives two workgroups to every CU, one otherwise (the products of an element
 // of X and their order do not depend on it).
-constexpr int kDSlots = 512;  // workgroups that run at once: two per CU
-
 template <int NB, int IB>
 void launch_kxd_ib(const Plan& p, const double* A, int64_t R, const double* cq, double* X, int64_t ldx, int ncol,
                    hipStream_t st) {
@@ -647,9 +706,13 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipStr
         TIM(F2JK_PH_KS, true);
         const int nsplit = std::min(p.nsplit, pc);
         for (int d = 0; d < p.nd; ++d) {
-            hipLaunchKernelGGL(ks_kernel<T>, dim3(p.nlower * nsplit), dim3(kGThreads), 0, st, X, p.N,
-                               p.OPAD, p.ioff[d], p.width[d], pc, nsplit, p.nlower,
-                               kpart + (size_t)d * p.nsplit * NN, c > 0 ? 1 : 0);
+            double* kp = kpart + (size_t)d * p.nsplit * NN;
+            if constexpr (sizeof(T) == 8)
+                hipLaunchKernelGGL(ksd_kernel, dim3(p.dt.total), dim3(256), 0, st, X, p.N, p.OPAD, p.ioff[d],
+                                   p.width[d], pc, p.dt, kp, c > 0 ? 1 : 0);
+            else
+                hipLaunchKernelGGL(ks_kernel<T>, dim3(p.nlower * nsplit), dim3(kGThreads), 0, st, X, p.N,
+                                   p.OPAD, p.ioff[d], p.width[d], pc, nsplit, p.nlower, kp, c > 0 ? 1 : 0);
             F2JK_LAUNCHED("ks");
         }
         TIM(F2JK_PH_KS, false);
@@ -657,8 +720,12 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipStr
     TIM(F2JK_PH_KRED, true);
     const int nsplit_used = std::min(p.nsplit, std::min(p.Pc, p.Q));
     for (int d = 0; d < p.nd; ++d) {
-        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st,
-                           kpart + (size_t)d * p.nsplit * NN, nsplit_used, p.N, K[d]);
+        double* kp = kpart + (size_t)d * p.nsplit * NN;
+        if constexpr (sizeof(T) == 8)
+            hipLaunchKernelGGL(kred_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st, kp, p.dt, p.N, K[d]);
+        else
+            hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st, kp, nsplit_used, p.N,
+                               K[d]);
         F2JK_LAUNCHED("k_reduce");
     }
     TIM(F2JK_PH_KRED, false);
@@ -1259,6 +1326,7 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
         g.dnb = p.dnb;
         g.dncolt = p.dncolt;
         g.dnks = p.dnks;
+        g.dt = p.dt;
         if (precision == F2JK_PREC_BF16X3) {
             g.Cth = (u16*)(w + p.off_cth);
             g.Ctl = (u16*)(w + p.off_ctl);

@@ -1,28 +1,36 @@
-// FP64 half-transform X = B C (gfx950) on v_mfma_f64_16x16x4.
+// FP64 exchange kernels (gfx950): the half-transform X = B C and the
+// contraction K = sum_P X_P X_P^T on v_mfma_f64_16x16x4.
 //
-// Rates (random B): 65 TFLOP/s at nbf 1152 with 240 and 320 columns, where the
-// same kernel without its loads of B reaches 67-68 (the clock under FP64 MFMA
-// load, not the 78.6 TFLOP/s of 2.4 GHz, is the ceiling) and the 128 x 320
-// tiles before it reached 46 (240 of 320 columns in use); 56 at nbf 384 with 80
-// columns (42 before: 80 of 128).  Below about 50 columns it is bound by
-// reading B: 4.2 TB/s of B and X at nbf 318.
+// One FP64 MFMA keeps a SIMD's matrix pipe busy for 64 cycles, so both are
+// bound by how evenly the 16 x 16 output blocks are spread over the SIMDs as
+// long as loads run a step ahead; LDS and L2 have room to spare.
 //
-// One FP64 MFMA keeps a SIMD's matrix pipe busy for 64 cycles, so the kernel
-// is bound by how evenly the 16 x 16 output blocks are spread over the SIMDs
-// as long as loads run a step ahead; LDS and L2 have room to spare.  So every
-// wave gets whole rows (16 * IB of them) and all the occupied columns of the
-// tile (NB blocks of 16, exactly the job's width): no wave holds padding
-// columns, and A = B(P|mn) goes from global memory straight into MFMA operands,
-// each element loaded once by one lane.
+// * The half-transform gives every wave whole rows (16 * IB of them) and all
+//   the occupied columns of the tile (NB blocks of 16, exactly the job's
+//   width): no wave holds padding columns, and A = B(P|mn) goes from global
+//   memory straight into MFMA operands, each element loaded once by one lane.
+//   Rates (random B): 65 TFLOP/s at nbf 1152 with 240 and 320 columns, where
+//   the same kernel without its loads of B reaches 67-68 (the clock under FP64
+//   MFMA load, not the 78.6 TFLOP/s of 2.4 GHz, is the ceiling) and the 128 x
+//   320 tiles before it reached 46 (240 of 320 columns in use); 56 at nbf 384
+//   with 80 columns (42 before: 80 of 128).  Below about 50 columns it is
+//   bound by reading B: 4.2 TB/s of B and X at nbf 318.
+// * The contraction splits the valid 16 x 16 blocks of a 128 x 128 tile over
+//   its four waves (a diagonal tile's 36 lower blocks as 9 per wave, an edge
+//   tile's rows in halves), and splits the P range of each kind of tile in
+//   proportion to its cost, so the workgroups of a launch take about as long.
+//   62 TFLOP/s of the lower triangle at nbf 1152 and 1536 (55 and 56 for the
+//   uniform splits of whole tiles before it), 53 at nbf 384 (43), where 60 is
+//   reached without any loads.
 //
 // Operand order.  A k step of 8 feeds two MFMAs: lane group g = lane / 16
 // holds k = 2g and 2g + 1 and supplies the first to MFMA 0 and the second to
 // MFMA 1.  The k sum is the same set of products in another order, and every
 // lane's operands are 16 contiguous bytes, in global memory and in LDS.
 //
-// The coefficients reach LDS by direct-to-LDS loads (lane l to slot l of 16
-// bytes) in the order in which the fragments are read: every LDS read is 1 KB
-// of consecutive bytes.  A load into LDS is not ordered with register loads, so a step ends
+// Tiles reach LDS by direct-to-LDS loads (lane l to slot l of 16 bytes) in the
+// order in which the fragments are read: every LDS read is 1 KB of consecutive
+// bytes.  A load into LDS is not ordered with register loads, so a step ends
 // with a full drain before its barrier; the loads have had the whole step.
 #pragma once
 #include "f2jk_kernels.h"
@@ -36,6 +44,7 @@ typedef double dx2u __attribute__((ext_vector_type(2), aligned(8)));
 constexpr int kDK = 16;         // k extent of one LDS stage
 constexpr int kDMaxNB = 20;     // 16-column blocks of the widest tile
 constexpr int kDMaxDens = 8;
+constexpr int kDKsLds = 2 * 2 * 16 * 1024;                // two stages of 8 + 8 row blocks, 2 KB each
 constexpr int kDKxLds(int nb) { return 2 * nb * 2048; }   // two stages of nb column blocks, 2 KB each
 
 // 16-row blocks per wave.  More than one block shares a coefficient fragment
@@ -217,6 +226,233 @@ __global__ __launch_bounds__(256, 2) void kxd_kernel(const double* __restrict__ 
                                                      int64_t ldx, int ncol, int ncolt) {
     __shared__ __attribute__((aligned(16))) char lds[kDKxLds(NB)];
     kxd_body<NB, IB>(lds, A, R, K, Cq, nks, X, ldx, ncol, ncolt, blockIdx.x, gridDim.x);
+}
+
+// ---------------------------------------------------------------------------
+// Contraction.  The lower triangle of K is cut into 128 x 128 tiles of 8 x 8
+// blocks; the last tile row has rl <= 8 blocks.  Four kinds of tiles, by the
+// blocks of their busiest wave (cost): 0 full (16), 1 diagonal (9), 2 last
+// row, 3 last diagonal.  Tiles of kind k split the P range in ns[k] parts.  Workgroups are numbered by the position
+// of their P range, so that those which read the same X run together.
+// ---------------------------------------------------------------------------
+struct DTiles {
+    int nt;        // tile rows
+    int rl;        // 16-row blocks of the last tile row
+    int cnt[4];    // tiles of each kind
+    int ns[4];     // P splits of each kind
+    int G;         // max ns of the kinds present
+    int total;     // workgroups: sum cnt * ns
+};
+__host__ __device__ inline int dtile_kind(const DTiles& m, int mt, int nt) {
+    return (mt == m.nt - 1 ? 2 : 0) + (mt == nt ? 1 : 0);
+}
+__host__ __device__ inline int dtile_cum(const DTiles& m, int g) {
+    int c = 0;
+    for (int k = 0; k < 4; ++k) c += m.cnt[k] * (int)((int64_t)m.ns[k] * g / m.G);
+    return c;
+}
+// workgroup b -> tile (mt, nt), split s of ns
+__host__ __device__ inline void dtile_decode(const DTiles& m, int b, int& mt, int& nt, int& s, int& ns) {
+    int g = (int)((int64_t)b * m.G / m.total);
+    while (dtile_cum(m, g + 1) <= b) ++g;
+    while (dtile_cum(m, g) > b) --g;
+    int x = b - dtile_cum(m, g);
+    for (int k = 0; k < 4; ++k) {
+        const int s0 = (int)((int64_t)m.ns[k] * g / m.G), s1 = (int)((int64_t)m.ns[k] * (g + 1) / m.G);
+        const int n = m.cnt[k] * (s1 - s0);
+        if (x >= n) {
+            x -= n;
+            continue;
+        }
+        const int q = x % m.cnt[k];
+        s = s0 + x / m.cnt[k];
+        ns = m.ns[k];
+        if (k == 0) {
+            mt = 1;
+            while (mt * (mt + 1) / 2 <= q) ++mt;
+            nt = q - mt * (mt - 1) / 2;
+        } else if (k == 1) {
+            mt = nt = q;
+        } else {
+            mt = m.nt - 1;
+            nt = k == 2 ? q : mt;
+        }
+        return;
+    }
+}
+
+__device__ __forceinline__ void ksd_body(char* lds, const double* __restrict__ X, int N, int OPAD, int ioff,
+                                         int width, int Pc, const DTiles& tm, double* __restrict__ Kpart,
+                                         int accumulate, int b) {
+    constexpr int STAGE = 32 * 1024;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int mt = 0, nt = 0, s = 0, ns = 1;
+    dtile_decode(tm, xcd_remap(b, tm.total), mt, nt, s, ns);
+    const bool diag = mt == nt;
+    const int rbn = mt == tm.nt - 1 ? tm.rl : 8;
+    const int m0 = mt * kTile, n0 = nt * kTile;
+    const int Pa = (int)((int64_t)Pc * s / ns), Pb = (int)((int64_t)Pc * (s + 1) / ns);
+    const int lr = lane & 15, lg = lane >> 4;
+
+    // this wave's loads: row block (wid + 4 q) / 2 (0-7 of the tile's rows,
+    // 8-15 of its columns), half (wid + 4 q) % 2 of the 16-k step
+    int qrow[8];
+    bool qon[8];
+    uint32_t qoff[8];
+    static_for<0, 8>([&](auto Q) {
+        constexpr int q = decltype(Q)::value;
+        const int rb = (wid + 4 * q) >> 1;
+        const int row = (rb < 8 ? m0 : n0 - 128) + rb * 16;
+        qon[q] = rb < 8 ? rb < rbn : !diag;
+        qrow[q] = qon[q] ? row : 0;
+        // rows past N are clamped onto row N - 1: they feed outputs that are never read
+        const int lrow = qrow[q] + lr < N ? lr : N - 1 - qrow[q];
+        qoff[q] = (uint32_t)(lrow * OPAD + 2 * lg) * 8;
+    });
+    const int h0 = wid & 1;
+    const int nkp = (width + kDK - 1) / kDK;  // steps per P; the last one is half when width % 16 == 8
+    const bool tail = width % kDK != 0;
+    auto load = [&](int P, int kt, int stg) {
+        if (tail && kt == nkp - 1 && h0) return;
+        const double* XP = X + (int64_t)P * N * OPAD + ioff + kt * kDK + 8 * h0;
+        const uint32_t l0 = lds_addr(lds) + stg * STAGE;
+        static_for<0, 8>([&](auto Q) {
+            constexpr int q = decltype(Q)::value;
+            if (qon[q]) lds_load16(uniform_ptr(XP + (int64_t)qrow[q] * OPAD), qoff[q], l0 + (wid + 4 * q) * 1024);
+        });
+    };
+
+    const int nsteps = (Pb - Pa) * nkp;
+    // the steps of the P range, one after the other: compute(LDS of the step at
+    // this lane's slot, halves of the step)
+    auto sweep = [&](auto&& compute) {
+        int kt = 0;           // the step being computed, of its P
+        int Pn = Pa, kn = 0;  // the step being loaded
+        if (nsteps > 0) load(Pa, 0, 0);
+        drain_and_barrier();
+        for (int st = 0; st < nsteps; ++st) {
+            const int cur = st & 1;
+            if (++kn == nkp) kn = 0, ++Pn;
+            if (st + 1 < nsteps) load(Pn, kn, cur ^ 1);
+            compute(lds + cur * STAGE + lane * 16, tail && kt == nkp - 1 ? 1 : 2);
+            kt = kn;
+            __builtin_amdgcn_sched_barrier(0);  // no MFMA moves past the drain
+            drain_and_barrier();
+        }
+    };
+    auto frag = [&](const char* L, int rb, int h) {
+        return *reinterpret_cast<const dx2*>(L + (2 * rb + h) * 1024);
+    };
+    double* Ks = Kpart + (int64_t)s * N * N;
+    auto put = [&](const dx4& v, int rb, int cb) {
+        const int col = n0 + cb * 16 + lr;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = m0 + rb * 16 + acc_row<double>(lane, r);
+            if (row < N && col < N) {
+                double* dst = Ks + (int64_t)row * N + col;
+                *dst = accumulate ? *dst + v[r] : v[r];
+            }
+        }
+    };
+    // NI x 4 blocks from row block i0 and column block j0
+    auto rect = [&](auto NI_, int i0, int j0) {
+        constexpr int NI = decltype(NI_)::value;
+        dx4 acc[NI > 0 ? NI : 1][4];
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = dx4{0, 0, 0, 0};
+        sweep([&](const char* L, int nh) {
+            for (int h = 0; h < nh; ++h) {
+                dx2 a[NI > 0 ? NI : 1], c[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) c[j] = frag(L, 8 + j0 + j, h);
+#pragma unroll
+                for (int i = 0; i < NI; ++i) a[i] = frag(L, i0 + i, h);
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[i][j] = mfma4(a[i].x, c[j].x, acc[i][j]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[i][j] = mfma4(a[i].y, c[j].y, acc[i][j]);
+                }
+            }
+        });
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) put(acc[i][j], i0 + i, j0 + j);
+    };
+    if (diag) {
+        // the lower blocks, numbered row after row, in quarters
+        const int nq = rbn * (rbn + 1) / 2;
+        const int qa = nq * wid / 4, qn = nq * (wid + 1) / 4 - qa;
+        int bi[9], bj[9];
+        {
+            int i = 0, q = qa;
+            while (q > i) q -= ++i;
+            static_for<0, 9>([&](auto T) {
+                constexpr int t = decltype(T)::value;
+                bi[t] = i < 8 ? i : 0;
+                bj[t] = i < 8 ? q : 0;
+                if (++q > i) q = 0, ++i;
+            });
+        }
+        dx4 acc[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) acc[i] = dx4{0, 0, 0, 0};
+        sweep([&](const char* L, int nh) {
+            for (int h = 0; h < nh; ++h) {
+                static_for<0, 3>([&](auto U) {  // three blocks at a time: consecutive MFMAs on different ones
+                    constexpr int u = 3 * decltype(U)::value;
+                    dx2 a[3], c[3];
+                    static_for<0, 3>([&](auto T) {
+                        a[T] = frag(L, bi[u + T], h);
+                        c[T] = frag(L, bj[u + T], h);
+                    });
+                    static_for<0, 3>([&](auto T) {
+                        if (u + T < qn) acc[u + T] = mfma4(a[T].x, c[T].x, acc[u + T]);
+                    });
+                    static_for<0, 3>([&](auto T) {
+                        if (u + T < qn) acc[u + T] = mfma4(a[T].y, c[T].y, acc[u + T]);
+                    });
+                });
+            }
+        });
+        static_for<0, 9>([&](auto T) {
+            if (T < qn) put(acc[T], bi[T], bj[T]);
+        });
+    } else {
+        // the rows in halves and the columns in halves, one quarter per wave
+        const int nr0 = (rbn + 1) / 2;
+        const int i0 = wid >> 1 ? nr0 : 0, ni = wid >> 1 ? rbn - nr0 : nr0, j0 = (wid & 1) * 4;
+        switch (ni) {
+            case 4: rect(std::integral_constant<int, 4>{}, i0, j0); break;
+            case 3: rect(std::integral_constant<int, 3>{}, i0, j0); break;
+            case 2: rect(std::integral_constant<int, 2>{}, i0, j0); break;
+            case 1: rect(std::integral_constant<int, 1>{}, i0, j0); break;
+            default: rect(std::integral_constant<int, 0>{}, i0, j0); break;
+        }
+    }
+}
+__global__ __launch_bounds__(256, 2) void ksd_kernel(const double* __restrict__ X, int N, int OPAD, int ioff,
+                                                     int width, int Pc, DTiles tm, double* __restrict__ Kpart,
+                                                     int accumulate) {
+    __shared__ __attribute__((aligned(16))) char lds[kDKsLds];
+    ksd_body(lds, X, N, OPAD, ioff, width, Pc, tm, Kpart, accumulate, blockIdx.x);
+}
+
+// the reduction over the splits of the element's tile
+__device__ __forceinline__ int dtile_splits(const DTiles& m, int m4, int n16) {
+    return m.ns[dtile_kind(m, m4 * 4 / kTile, n16 * 16 / kTile)];
+}
+__global__ __launch_bounds__(256) void kred_kernel(const double* __restrict__ Kpart, DTiles tm, int N,
+                                                   double* __restrict__ K) {
+    const int nb = (N + 15) / 16, m4 = blockIdx.x / nb, n16 = blockIdx.x % nb;
+    if (n16 * 16 > m4 * 4 + 3) return;
+    k_reduce_body(Kpart, dtile_splits(tm, m4, n16), N, K, m4, n16);
 }
 
 }  // namespace f2jk

@@ -60,6 +60,7 @@ struct GJob {
     int nvec, neg, npc1, npc2, ppw2;
     int nlower, nsplit, ncolt;
     int dnb, dncolt, dnks;  // FP64 half-transform
+    DTiles dt;              // FP64 contraction
     int want_j;
 };
 
@@ -88,7 +89,7 @@ __host__ __device__ inline int phase_blocks(const GJob& g, int phase) {
         case GP_KX:
             if (PREC == F2JK_PREC_FP64) return gcdiv((long long)g.Q * g.N, 64 * kxd_ib(g.dnb)) * g.dncolt;
             return gcdiv((long long)g.Q * g.N, kTile) * g.ncolt;
-        case GP_KS: return g.nlower * g.nsplit * g.nd;
+        case GP_KS: return (PREC == F2JK_PREC_FP64 ? g.dt.total : g.nlower * g.nsplit) * g.nd;
         case GP_KRED: return k_reduce_blocks(g.N) * g.nd;
     }
     return 0;
@@ -165,7 +166,9 @@ void grouped_kernel(const GArgs a) {
                 if constexpr (PHASE == GP_DRED)
                     k_reduce_body(g.Dpart + d * NN, 1, g.N, g.D + d * NN, m4, n16);
                 else
-                    k_reduce_body(g.Kpart + d * g.nsplit * NN, g.nsplit, g.N, g.K[d], m4, n16);
+                    k_reduce_body(g.Kpart + d * g.nsplit * NN,
+                                  PREC == F2JK_PREC_FP64 ? dtile_splits(g.dt, m4, n16) : g.nsplit, g.N, g.K[d], m4,
+                                  n16);
             }
         } else if constexpr (PHASE == GP_GAMMA) {
             const int bx = local % g.neg, by = local / g.neg;
@@ -215,13 +218,16 @@ void grouped_kernel(const GArgs a) {
                                                xh + R * g.OPAD, g.ncolt, local, nb);
             }
         } else if constexpr (PHASE == GP_KS) {
-            const int per = g.nlower * g.nsplit;
+            const int per = PREC == F2JK_PREC_FP64 ? g.dt.total : g.nlower * g.nsplit;
             const int d = local / per, b = local % per;
             double* kp = g.Kpart + (long long)d * g.nsplit * g.N * g.N;
             if constexpr (PREC == F2JK_PREC_BF16X3) {
                 const u16* xh = (const u16*)g.X;
                 ks_bf16x3_kernel_body<kTile, 2, 2>(xh, xh + (long long)g.Q * g.N * g.OPAD, g.N, g.OPAD, g.ioff[d], g.width[d],
                                       g.Q, g.nsplit, g.nlower, kp, 0, b, per);
+            } else if constexpr (PREC == F2JK_PREC_FP64) {
+                __shared__ __attribute__((aligned(16))) char lds[kDKsLds];
+                ksd_body(lds, (const double*)g.X, g.N, g.OPAD, g.ioff[d], g.width[d], g.Q, g.dt, kp, 0, b);
             } else {
                 ks_kernel_body<TB>((const TB*)g.X, g.N, g.OPAD, g.ioff[d], g.width[d], g.Q, g.nsplit, g.nlower,
                                    kp, 0, b, per);
