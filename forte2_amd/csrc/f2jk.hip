@@ -115,10 +115,12 @@ struct Plan {
     int dnb = 0, dncolt = 0, dnks = 0;  // FP64 half-transform: column blocks of a tile, tiles, 16-k steps
     size_t per_p = 0;      // bytes of X per P
     DTiles dt{};           // FP64 contraction: tiles and their P splits
+    bool gamma_x = false;  // gamma of J from the half-transform's row sums (FP64 J and K from C)
     int ctrows = 0;     // rows of the padded bf16 coefficient planes (>= ncolt * tile columns)
     // workspace offsets
     int KP = 0;                // nbf rounded up to the bf16 k step
     size_t off_cp32 = 0, off_cth = 0, off_ctl = 0, off_cq = 0;
+    size_t off_grow = 0;
     size_t off_cp = 0, off_d = 0, off_dpart = 0, off_gpart = 0, off_gamma = 0, off_jpart = 0,
            off_x = 0, off_kpart = 0, total = 0;
     // sizes of the regions that scale with the launch-shape knobs
@@ -216,6 +218,15 @@ int build_jlist(f2jk_ctx* ctx, int dtype) {
 
 constexpr int kDSlots = 512;  // workgroups of the FP64 K kernels that run at once: two per CU
 
+
+// the row sums of the half-transform's epilogue (grow null: none)
+struct KxdGamma {
+    const double* cp = nullptr;
+    double* grow = nullptr;
+    int64_t stride = 0;
+    DCols dc{};
+};
+
 // Tiles of the FP64 contraction of an N x N matrix and the P splits of each
 // kind, in proportion to the cost of a tile: the blocks of its busiest wave,
 // 1.6 times that for a diagonal tile (its waves read two fragments per block
@@ -294,6 +305,7 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
     p.want_j = flags & F2JK_WANT_J;
     p.want_k = flags & F2JK_WANT_K;
     p.need_c = p.want_k || (p.want_j && j_from_c);
+    p.gamma_x = precision == F2JK_PREC_FP64 && p.want_j && p.want_k && j_from_c;
     const int jdtype = (precision == F2JK_PREC_FP64) ? F2JK_F64 : F2JK_F32;
     const int kdtype = jdtype;
     if (p.want_j && !ctx->B[jdtype])
@@ -307,7 +319,8 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
     if (p.need_c) {
         if (!nocc) return fail(F2JK_EINVAL, "nocc is required");
         int o = 0;
-        const int kalign = (precision == F2JK_PREC_BF16X3) ? kBK16 : 16;
+        // the FP64 contraction takes k steps of 8, the others whole LDS stages
+        const int kalign = precision == F2JK_PREC_BF16X3 ? kBK16 : (precision == F2JK_PREC_FP64 && p.want_k) ? 8 : 16;
         for (int d = 0; d < ndens; ++d) {
             if (nocc[d] < 0 || nocc[d] > N) return fail(F2JK_EINVAL, "nocc out of range");
             p.width[d] = (int)(cdiv(std::max<int64_t>(nocc[d], 1), kalign) * kalign);
@@ -316,18 +329,23 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         }
         p.OPAD = (int)cdiv(o, 16) * 16;
         // the C copy used for D (always fp64) and the K copy (fp64 or fp32)
-        p.off_cp = off;
-        off += align_up((size_t)N * p.OPAD * 8);
-        p.off_cp32 = off;
-        off += align_up((size_t)N * p.OPAD * 4);  // fp32 copy (FP32 K)
         if (precision == F2JK_PREC_FP64 && p.want_k) {
             // column tiles of equal width, at most 20 blocks of 16
             const int nb = (int)cdiv(p.OPAD, 16);
             p.dncolt = (int)cdiv(nb, kDMaxNB);
             p.dnb = (int)cdiv(nb, p.dncolt);
             p.dnks = (int)cdiv(N, kDK);
+        }
+        p.off_cp = off;
+        off += align_up((size_t)N * std::max(p.OPAD, p.dncolt * p.dnb * 16) * 8);
+        p.off_cp32 = off;
+        off += align_up((size_t)N * p.OPAD * 4);  // fp32 copy (FP32 K)
+        if (precision == F2JK_PREC_FP64 && p.want_k) {
             p.off_cq = off;
-            off += align_up((size_t)p.dncolt * p.dnks * p.dnb * 256 * 8);
+            // where J and K come from C, D is not formed: Cq lies in the room of
+            // D and its partials (of which there is still as much as before)
+            const size_t cq = align_up((size_t)p.dncolt * p.dnks * p.dnb * 256 * 8);
+            off += p.gamma_x ? std::max(cq, align_up((size_t)ndens * N * N * 8) + align_up((size_t)N * N * 8)) : cq;
         }
         p.KP = (int)(cdiv(N, kBK16) * kBK16);
         if (precision == F2JK_PREC_BF16X3) {
@@ -357,14 +375,14 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         p.npc2 = (int)std::max<int64_t>(1, std::min<int64_t>(Q, cdiv(target_blocks, p.neg)));
         p.ppw2 = (int)cdiv(Q, p.npc2);
         p.npc2 = (int)cdiv(Q, p.ppw2);
-        if (j_from_c) {
+        if (j_from_c && !p.gamma_x) {
             p.off_d = off;
             off += align_up((size_t)ndens * N * N * 8);
             p.off_dpart = off;
             off += align_up((size_t)N * N * 8);
         }
         p.off_gpart = off;
-        off += align_up((size_t)p.neg * ndens * Q * 8);
+        if (!p.gamma_x) off += align_up((size_t)p.neg * ndens * Q * 8);
         p.off_gamma = off;
         off += align_up((size_t)ndens * Q * 8);
         p.off_jpart = off;
@@ -372,7 +390,8 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         off += p.jpart_bytes;
     }
     if (p.want_k) {
-        const size_t per_p = (size_t)N * p.OPAD * p.tk;
+        const size_t grow_p = p.gamma_x ? (size_t)p.dncolt * ndens * N * 8 : 0;
+        const size_t per_p = (size_t)N * p.OPAD * p.tk + grow_p;
         int64_t pc = (int64_t)(xchunk_bytes / std::max<size_t>(per_p, 1));
         pc = std::max<int64_t>(1, std::min<int64_t>(pc, Q));
         pc = std::min<int64_t>(pc, INT32_MAX / N);  // rows of a chunk are numbered in 32 bits
@@ -431,8 +450,10 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         else
             p.kva = (N % 4 == 0) ? 4 : ((N % 2 == 0) ? 2 : 1);
         p.off_x = off;
-        p.x_bytes = align_up((size_t)p.Pc * per_p);
+        p.x_bytes = align_up((size_t)p.Pc * (per_p - grow_p));
         off += p.x_bytes;
+        p.off_grow = off;
+        off += align_up((size_t)p.Pc * grow_p);
         if (precision == F2JK_PREC_FP64) {
             p.dt = dtile_plan(N, pc, p.width[0], (int)std::min<int64_t>(kDSlots, target_blocks));
             p.nsplit = p.dt.G;  // partials held per density
@@ -472,29 +493,32 @@ int tim_mark(f2jk_ctx* ctx, int phase, hipStream_t st, bool start) {
     } while (0)
 
 // --------------------------------------------------------------------------- J
+// densities d0 .. d0 + ND - 1; without D, gamma is there already
 template <typename TB, int VEC, int ND, bool NT>
-int launch_j(f2jk_ctx* ctx, const Plan& p, const TB* B, const double* const* D, int64_t ldd,
+int launch_j(f2jk_ctx* ctx, const Plan& p, const TB* B, int d0, const double* const* D, int64_t ldd,
              double* const* J, char* ws, hipStream_t st) {
     DPtrs<ND> dp;
     JPtrs<ND> jp;
     for (int d = 0; d < ND; ++d) {
-        dp.p[d] = D[d];
-        jp.p[d] = J[d];
+        dp.p[d] = D ? D[d0 + d] : nullptr;
+        jp.p[d] = J[d0 + d];
     }
     double* gpart = (double*)(ws + p.off_gpart);
-    double* gamma = (double*)(ws + p.off_gamma);
+    double* gamma = (double*)(ws + p.off_gamma) + (D ? 0 : (size_t)d0 * p.Q);
     double* jpart = (double*)(ws + p.off_jpart);
     const int* rowoff = ctx->rowoff[VEC];
     const uint32_t* elist = p.jlist;
-    TIM(F2JK_PH_JGAMMA, true);
-    hipLaunchKernelGGL((j_gamma_kernel<TB, VEC, kEPT, ND, NT>), dim3(p.neg, p.npc1), dim3(kJThreads), 0,
-                       st, B, p.N, p.Q, dp, ldd, rowoff, elist, p.nvec, kJ1PerBlock, gpart);
-    F2JK_LAUNCHED("j_gamma");
-    const int64_t ng = (int64_t)ND * p.Q;
-    hipLaunchKernelGGL(j_gamma_reduce_kernel, dim3((unsigned)cdiv(ng, 256)), dim3(256), 0, st,
-                       gpart, p.neg, ND, p.Q, gamma);
-    F2JK_LAUNCHED("j_gamma_reduce");
-    TIM(F2JK_PH_JGAMMA, false);
+    if (D) {
+        TIM(F2JK_PH_JGAMMA, true);
+        hipLaunchKernelGGL((j_gamma_kernel<TB, VEC, kEPT, ND, NT>), dim3(p.neg, p.npc1), dim3(kJThreads), 0,
+                           st, B, p.N, p.Q, dp, ldd, rowoff, elist, p.nvec, kJ1PerBlock, gpart);
+        F2JK_LAUNCHED("j_gamma");
+        const int64_t ng = (int64_t)ND * p.Q;
+        hipLaunchKernelGGL(j_gamma_reduce_kernel, dim3((unsigned)cdiv(ng, 256)), dim3(256), 0, st,
+                           gpart, p.neg, ND, p.Q, gamma);
+        F2JK_LAUNCHED("j_gamma_reduce");
+        TIM(F2JK_PH_JGAMMA, false);
+    }
     TIM(F2JK_PH_JACC, true);
     hipLaunchKernelGGL((j_accum_kernel<TB, VEC, kEPT, ND, NT>), dim3(p.neg, p.npc2), dim3(kJThreads), 0,
                        st, B, p.N, p.Q, gamma, rowoff, elist, p.nvec, p.ppw2, jpart);
@@ -515,12 +539,12 @@ int launch_j_nd(f2jk_ctx* ctx, const Plan& p, const TB* B, int nd, const double*
         int rc;
         const bool nt = ctx->j_nontemporal;
         if (nd - d >= 2) {
-            rc = nt ? launch_j<TB, VEC, 2, true>(ctx, p, B, D + d, ldd, J + d, ws, st)
-                    : launch_j<TB, VEC, 2, false>(ctx, p, B, D + d, ldd, J + d, ws, st);
+            rc = nt ? launch_j<TB, VEC, 2, true>(ctx, p, B, d, D, ldd, J, ws, st)
+                    : launch_j<TB, VEC, 2, false>(ctx, p, B, d, D, ldd, J, ws, st);
             d += 2;
         } else {
-            rc = nt ? launch_j<TB, VEC, 1, true>(ctx, p, B, D + d, ldd, J + d, ws, st)
-                    : launch_j<TB, VEC, 1, false>(ctx, p, B, D + d, ldd, J + d, ws, st);
+            rc = nt ? launch_j<TB, VEC, 1, true>(ctx, p, B, d, D, ldd, J, ws, st)
+                    : launch_j<TB, VEC, 1, false>(ctx, p, B, d, D, ldd, J, ws, st);
             d += 1;
         }
         if (rc) return rc;
@@ -571,7 +595,7 @@ int pack_c(f2jk_ctx* ctx, const Plan& p, const double* const* C, const int64_t* 
         }
         const int64_t n = (int64_t)p.dncolt * p.dnks * p.dnb * 256;
         hipLaunchKernelGGL(pack_cq_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, cs, dcols_of(p, nocc), p.N,
-                           p.OPAD, p.dnb, p.dnks, n, cp, (double*)(ws + p.off_cq));
+                           p.dncolt * p.dnb * 16, p.dnb, p.dnks, n, cp, (double*)(ws + p.off_cq));
         F2JK_LAUNCHED("pack_cq");
         return F2JK_OK;
     }
@@ -659,32 +683,34 @@ void launch_kx_fp32(const Plan& p, unsigned grid, const float* A, int64_t R, con
 // of X and their order do not depend on it).
 template <int NB, int IB>
 void launch_kxd_ib(const Plan& p, const double* A, int64_t R, const double* cq, double* X, int64_t ldx, int ncol,
-                   hipStream_t st) {
+                   const KxdGamma& g, hipStream_t st) {
     const unsigned grid = (unsigned)(cdiv(R, 64 * IB) * p.dncolt);
     hipLaunchKernelGGL((kxd_kernel<NB, IB>), dim3(grid), dim3(256), 0, st, A, R, p.N, cq, p.dnks, X, ldx, ncol,
-                       p.dncolt);
+                       p.dncolt, g.cp, g.dc, g.grow, g.stride);
 }
 template <int NB>
 void launch_kxd_nb(const Plan& p, const double* A, int64_t R, const double* cq, double* X, int64_t ldx, int ncol,
-                   hipStream_t st) {
+                   const KxdGamma& g, hipStream_t st) {
     constexpr int IB = kxd_ib(NB);
     if constexpr (IB >= 2) {
         if (cdiv(R, 64 * IB) * p.dncolt >= kDSlots)
-            return launch_kxd_ib<NB, IB>(p, A, R, cq, X, ldx, ncol, st);
+            return launch_kxd_ib<NB, IB>(p, A, R, cq, X, ldx, ncol, g, st);
     }
-    launch_kxd_ib<NB, 1>(p, A, R, cq, X, ldx, ncol, st);
+    launch_kxd_ib<NB, 1>(p, A, R, cq, X, ldx, ncol, g, st);
 }
 template <int NB = 1>
 void launch_kxd(const Plan& p, const double* A, int64_t R, const double* cq, double* X, int64_t ldx, int ncol,
-                hipStream_t st) {
+                const KxdGamma& g, hipStream_t st) {
     if constexpr (NB <= kDMaxNB) {
-        if (p.dnb == NB) return launch_kxd_nb<NB>(p, A, R, cq, X, ldx, ncol, st);
-        launch_kxd<NB + 1>(p, A, R, cq, X, ldx, ncol, st);
+        if (p.dnb == NB) return launch_kxd_nb<NB>(p, A, R, cq, X, ldx, ncol, g, st);
+        launch_kxd<NB + 1>(p, A, R, cq, X, ldx, ncol, g, st);
     }
 }
 
-template <typename T>
-int run_k_typed(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipStream_t st) {
+// `after_kx` runs once the last chunk's half-transform (and gamma) is queued
+template <typename T, typename F>
+int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const* K, char* ws, hipStream_t st,
+                F&& after_kx) {
     const T* B = (const T*)ctx->B[sizeof(T) == 8 ? F2JK_F64 : F2JK_F32];
     const T* cp = (sizeof(T) == 8) ? (const T*)(ws + p.off_cp) : (const T*)(ws + p.off_cp32);
     T* X = (T*)(ws + p.off_x);
@@ -697,12 +723,31 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipStr
         const int64_t nrowt = cdiv(R, kTile);
         TIM(F2JK_PH_KX, true);
         const T* A = B + (int64_t)P0 * NN;
-        if constexpr (sizeof(T) == 8)
-            launch_kxd(p, A, R, (const double*)(ws + p.off_cq), X, p.OPAD, p.OPAD, st);
-        else
+        if constexpr (sizeof(T) == 8) {
+            KxdGamma g;
+            if (p.gamma_x) {
+                g.cp = cp;
+                g.grow = (double*)(ws + p.off_grow);
+                g.stride = (int64_t)p.Pc * p.N;
+                g.dc = dcols_of(p, nocc);
+            }
+            launch_kxd(p, A, R, (const double*)(ws + p.off_cq), X, p.OPAD, p.OPAD, g, st);
+        } else
             launch_kx_fp32(p, (unsigned)(nrowt * p.ncolt), A, R, cp, X, st);
         F2JK_LAUNCHED("kx");
         TIM(F2JK_PH_KX, false);
+        if (p.gamma_x) {
+            TIM(F2JK_PH_JGAMMA, true);
+            hipLaunchKernelGGL(gamma_rows_kernel, dim3((unsigned)cdiv((int64_t)p.nd * pc, 4)), dim3(256), 0, st,
+                               (const double*)(ws + p.off_grow), (int64_t)p.Pc * p.N, p.nd, p.dncolt, p.N, pc,
+                               (double*)(ws + p.off_gamma) + P0, p.Q);
+            F2JK_LAUNCHED("gamma_rows");
+            TIM(F2JK_PH_JGAMMA, false);
+        }
+        if (c + 1 == p.nchunks) {
+            const int rc = after_kx();
+            if (rc) return rc;
+        }
         TIM(F2JK_PH_KS, true);
         const int nsplit = std::min(p.nsplit, pc);
         for (int d = 0; d < p.nd; ++d) {
@@ -869,31 +914,34 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
     if (p.need_c) {
         TIM(F2JK_PH_PREP, true);
         if ((rc = pack_c(ctx, p, C, nocc, ldc, w, st, p.want_k && p.prec == F2JK_PREC_FP32))) return rc;
-        if (p.want_j && j_from_c)
+        if (p.want_j && j_from_c && !p.gamma_x)
             if ((rc = build_d(ctx, p, w, st))) return rc;
         TIM(F2JK_PH_PREP, false);
     }
-    // fork: the J passes go to the side stream once the prepared inputs exist
+    // the J passes: on the side stream (forked once their inputs exist) when they
+    // run beside K
     const bool overlap = p.want_j && p.want_k && ctx->overlap_jk;
-    hipStream_t sj = st;
-    if (overlap) {
-        F2JK_HIP(hipEventRecord(ctx->ev_fork, st));
-        F2JK_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
-        sj = ctx->side;
-    }
-    if (p.want_j) {
+    hipStream_t sj = overlap ? ctx->side : st;
+    auto do_j = [&]() -> int {
+        if (!p.want_j) return F2JK_OK;
+        if (overlap) {
+            F2JK_HIP(hipEventRecord(ctx->ev_fork, st));
+            F2JK_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
+        }
+        if (p.gamma_x) return run_j(ctx, p, nullptr, 0, J, w, sj);
         std::vector<const double*> dptr(ndens);
-        int64_t lddu = ldd;
         for (int d = 0; d < ndens; ++d)
             dptr[d] = j_from_c ? (const double*)(w + p.off_d) + (size_t)d * p.N * p.N : Din[d];
-        if (j_from_c) lddu = p.N;
-        if ((rc = run_j(ctx, p, dptr.data(), lddu, J, w, sj))) return rc;
-    }
+        return run_j(ctx, p, dptr.data(), j_from_c ? p.N : ldd, J, w, sj);
+    };
+    if (!p.gamma_x && (rc = do_j())) return rc;
     if (p.want_k) {
         if (p.prec == F2JK_PREC_BF16X3)
             rc = run_k_bf16x3(ctx, p, K, w, st);
+        else if (p.tk == 8)
+            rc = run_k_typed<double>(ctx, p, nocc, K, w, st, [&] { return p.gamma_x ? do_j() : F2JK_OK; });
         else
-            rc = (p.tk == 8) ? run_k_typed<double>(ctx, p, K, w, st) : run_k_typed<float>(ctx, p, K, w, st);
+            rc = run_k_typed<float>(ctx, p, nocc, K, w, st, [] { return F2JK_OK; });
         if (rc) return rc;
     }
     // join: later work on the caller's stream sees J
@@ -941,7 +989,7 @@ int fit_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision,
         int rc = make_plan(ctx, ndens, nocc, precision, flags, true, p, 0, false, &caps);
         if (rc) return rc;
         if (p.total <= budget) return F2JK_OK;
-        const size_t per_p = p.want_k ? (size_t)p.N * p.OPAD * p.tk : 0;
+        const size_t per_p = p.per_p;
         if (p.want_k && p.Pc > 1 && p.x_bytes >= p.jpart_bytes + p.kpart_bytes)
             caps.xchunk_bytes = per_p * (size_t)(p.Pc / 2);
         else if (caps.target_blocks > 1)
@@ -1010,19 +1058,14 @@ int launch_group_kx_bf16(const GArgs& a, int nbw, hipStream_t st) {
 template <int PREC>
 int run_group(f2jk_ctx* ctx, const GArgs& a, int nbw, int va, hipStream_t st) {
     int rc;
+    constexpr bool gamma_x = PREC == F2JK_PREC_FP64;  // gamma comes with the half-transform
     TIM(F2JK_PH_PREP, true);
     if ((rc = launch_group_phase<GP_PAD, PREC>(a, st))) return rc;
-    if ((rc = launch_group_phase<GP_DKS, PREC>(a, st))) return rc;
-    if ((rc = launch_group_phase<GP_DRED, PREC>(a, st))) return rc;
+    if constexpr (!gamma_x) {
+        if ((rc = launch_group_phase<GP_DKS, PREC>(a, st))) return rc;
+        if ((rc = launch_group_phase<GP_DRED, PREC>(a, st))) return rc;
+    }
     TIM(F2JK_PH_PREP, false);
-    TIM(F2JK_PH_JGAMMA, true);
-    if ((rc = launch_group_phase<GP_GAMMA, PREC>(a, st))) return rc;
-    if ((rc = launch_group_phase<GP_GRED, PREC>(a, st))) return rc;
-    TIM(F2JK_PH_JGAMMA, false);
-    TIM(F2JK_PH_JACC, true);
-    if ((rc = launch_group_phase<GP_JACC, PREC>(a, st))) return rc;
-    if ((rc = launch_group_phase<GP_JRED, PREC>(a, st))) return rc;
-    TIM(F2JK_PH_JACC, false);
     TIM(F2JK_PH_KX, true);
     if constexpr (PREC == F2JK_PREC_BF16X3) {
         rc = (va == 4) ? launch_group_kx_bf16<4>(a, nbw, st) : launch_group_kx_bf16<2>(a, nbw, st);
@@ -1031,6 +1074,15 @@ int run_group(f2jk_ctx* ctx, const GArgs& a, int nbw, int va, hipStream_t st) {
         if ((rc = launch_group_phase<GP_KX, PREC>(a, st))) return rc;
     }
     TIM(F2JK_PH_KX, false);
+    TIM(F2JK_PH_JGAMMA, true);
+    if constexpr (!gamma_x)
+        if ((rc = launch_group_phase<GP_GAMMA, PREC>(a, st))) return rc;
+    if ((rc = launch_group_phase<GP_GRED, PREC>(a, st))) return rc;
+    TIM(F2JK_PH_JGAMMA, false);
+    TIM(F2JK_PH_JACC, true);
+    if ((rc = launch_group_phase<GP_JACC, PREC>(a, st))) return rc;
+    if ((rc = launch_group_phase<GP_JRED, PREC>(a, st))) return rc;
+    TIM(F2JK_PH_JACC, false);
     TIM(F2JK_PH_KS, true);
     if ((rc = launch_group_phase<GP_KS, PREC>(a, st))) return rc;
     TIM(F2JK_PH_KS, false);
@@ -1334,6 +1386,7 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
         g.X = (void*)(w + p.off_x);
         g.Kpart = (double*)(w + p.off_kpart);
         if (want_j) {
+            g.grow = (double*)(w + p.off_grow);
             g.D = (double*)(w + p.off_d);
             g.Dpart = (double*)(w + p.off_dpart);
             g.gpart = (double*)(w + p.off_gpart);
@@ -1413,7 +1466,7 @@ int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ld
     const int64_t step = INT32_MAX / p.N;  // rows of a launch are numbered in 32 bits
     for (int64_t P0 = p0; P0 < p1; P0 += step) {
         const int64_t R = std::min<int64_t>(step, p1 - P0) * p.N;
-        launch_kxd(p, B + P0 * NN, R, cq, X + (P0 - p0) * p.N * ldx, ldx, (int)ncol, st);
+        launch_kxd(p, B + P0 * NN, R, cq, X + (P0 - p0) * p.N * ldx, ldx, (int)ncol, KxdGamma{}, st);
         F2JK_LAUNCHED("kx");
     }
     g_last_error.clear();

@@ -72,7 +72,8 @@ struct DCols {
 
 // ---------------------------------------------------------------------------
 // Coefficients of all densities in the two forms the kernels read:
-//   Cp[n][c]  row-major, OPAD columns (D = C C^T);
+//   Cp[n][c]  row-major, the columns of all tiles (the gamma sums of the
+//             half-transform);
 //   Cq        [column tile][16-k step][block][k / 8 % 2][lane][2], the order
 //             of the half-transform's LDS tiles; zero outside N x nocc.
 // ---------------------------------------------------------------------------
@@ -81,7 +82,7 @@ struct DCoef {
     int64_t ldc[kDMaxDens];
 };
 __device__ __forceinline__ void pack_cq_element(const double* const* C, const int64_t* ldc, int nd,
-                                                const int* nocc, const int* ioff, int N, int OPAD, int nb, int nks,
+                                                const int* nocc, const int* ioff, int N, int ldcp, int nb, int nks,
                                                 int64_t t, double* __restrict__ Cp, double* __restrict__ Cq) {
     const int tt = (int)(t & 1), lane = (int)((t >> 1) & 63);
     const int64_t u = t >> 7;                       // (ct * nks + s) * 2 nb + 2 j + h
@@ -96,22 +97,29 @@ __device__ __forceinline__ void pack_cq_element(const double* const* C, const in
         if (i >= 0 && i < nocc[d] && k < N) x = C[d][(int64_t)k * ldc[d] + i];
     }
     Cq[t] = x;
-    if (k < N && c < OPAD) Cp[(int64_t)k * OPAD + c] = x;
+    if (k < N) Cp[(int64_t)k * ldcp + c] = x;
 }
-__global__ void pack_cq_kernel(DCoef cs, DCols dc, int N, int OPAD, int nb, int nks, int64_t total,
+__global__ void pack_cq_kernel(DCoef cs, DCols dc, int N, int ldcp, int nb, int nks, int64_t total,
                                double* __restrict__ Cp, double* __restrict__ Cq) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < total) pack_cq_element(cs.C, cs.ldc, dc.nd, dc.nocc, dc.ioff, N, OPAD, nb, nks, t, Cp, Cq);
+    if (t < total) pack_cq_element(cs.C, cs.ldc, dc.nd, dc.nocc, dc.ioff, N, ldcp, nb, nks, t, Cp, Cq);
 }
 
 // ---------------------------------------------------------------------------
 // Half-transform: X[r][c] = sum_k A[r][k] C[k][c], r < R, for a tile of
 // NB * 16 columns; 4 waves of 16 * IB rows each.
+// With grow, the epilogue also forms the row sums
+//   grow[ct * nd + d][r] = sum over the columns c of density d in the tile of X[r][c] C[r % N][c]
+// whose sum over the N rows of one P is gamma_P = sum_mn B_Pmn D_mn (D = C C^T):
+// the first J pass without another read of B and without D.  A row's sum does
+// not depend on how rows are cut into tiles or P into chunks.
 // ---------------------------------------------------------------------------
 template <int NB, int IB>
 __device__ __forceinline__ void kxd_body(char* lds, const double* __restrict__ A, int64_t R, int K,
                                          const double* __restrict__ Cq, int nks, double* __restrict__ X,
-                                         int64_t ldx, int ncol, int ncolt, int b, int nblocks) {
+                                         int64_t ldx, int ncol, int ncolt, const double* __restrict__ Cp, int nd,
+                                         const int* ioff, const int* width, double* __restrict__ grow,
+                                         int64_t gstride, int b, int nblocks) {
     constexpr int STAGE = NB * 2048;  // bytes
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -218,14 +226,64 @@ __device__ __forceinline__ void kxd_body(char* lds, const double* __restrict__ A
                     if (c0 + j * 16 < ncol) dst[j * 16] = acc[i][j][r];
             }
         }
+    if (!grow) return;
+    const int ldcp = ncolt * NB * 16;
+    auto row_sums = [&](int d, auto masked) {
+        const int lo = ioff[d], hi = lo + width[d];
+        double* gr = grow + (int64_t)(ct * nd + d) * gstride;
+#pragma unroll
+        for (int i = 0; i < IB; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t row = r0 + wr0 + i * 16 + acc_row<double>(lane, r);
+                const double* cr = Cp + (int64_t)((uint32_t)(row < R ? row : R - 1) % (uint32_t)K) * ldcp + c0;
+                double s = 0.0;
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    const double x = cr[j * 16];
+                    if constexpr (decltype(masked)::value)
+                        s = fma(acc[i][j][r], c0 + j * 16 >= lo && c0 + j * 16 < hi ? x : 0.0, s);
+                    else
+                        s = fma(acc[i][j][r], x, s);
+                }
+#pragma unroll
+                for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o);
+                if (lr == 0 && row < R) gr[row] = s;
+                __builtin_amdgcn_sched_barrier(0);  // one row's coefficients in registers at a time
+            }
+    };
+    if (nd == 1)
+        row_sums(0, std::false_type{});
+    else
+        for (int d = 0; d < nd; ++d) row_sums(d, std::true_type{});
 }
 
 template <int NB, int IB>
 __global__ __launch_bounds__(256, 2) void kxd_kernel(const double* __restrict__ A, int64_t R, int K,
                                                      const double* __restrict__ Cq, int nks, double* __restrict__ X,
-                                                     int64_t ldx, int ncol, int ncolt) {
+                                                     int64_t ldx, int ncol, int ncolt, const double* __restrict__ Cp,
+                                                     DCols dc, double* __restrict__ grow, int64_t gstride) {
     __shared__ __attribute__((aligned(16))) char lds[kDKxLds(NB)];
-    kxd_body<NB, IB>(lds, A, R, K, Cq, nks, X, ldx, ncol, ncolt, blockIdx.x, gridDim.x);
+    kxd_body<NB, IB>(lds, A, R, K, Cq, nks, X, ldx, ncol, ncolt, Cp, dc.nd, dc.ioff, dc.width, grow, gstride,
+                     blockIdx.x, gridDim.x);
+}
+
+// gamma[d][P] = sum over column tiles and rows m of grow[ct * nd + d][P * N + m], one wave per (d, P)
+__device__ __forceinline__ void gamma_rows_body(const double* __restrict__ grow, int64_t gstride, int nd, int ncolt,
+                                                int N, int pc, double* __restrict__ gamma, int Q, int64_t t) {
+    if (t >= (int64_t)nd * pc) return;
+    const int d = (int)(t / pc), P = (int)(t % pc), lane = threadIdx.x & 63;
+    double s = 0.0;
+    for (int ct = 0; ct < ncolt; ++ct) {
+        const double* g = grow + (int64_t)(ct * nd + d) * gstride + (int64_t)P * N;
+        for (int m = lane; m < N; m += 64) s += g[m];
+    }
+    s = wave_sum(s);
+    if (lane == 0) gamma[(int64_t)d * Q + P] = s;
+}
+__global__ __launch_bounds__(256) void gamma_rows_kernel(const double* __restrict__ grow, int64_t gstride, int nd,
+                                                         int ncolt, int N, int pc, double* __restrict__ gamma, int Q) {
+    gamma_rows_body(grow, gstride, nd, ncolt, N, pc, gamma, Q, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
 }
 
 // ---------------------------------------------------------------------------

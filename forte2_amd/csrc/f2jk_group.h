@@ -30,12 +30,12 @@ namespace f2jk {
 constexpr int kMaxGroup = 12;
 
 enum GroupPhase {
-    GP_PAD = 0,      // Cp[n][ioff+i] = C[n][i] (FP64; also the FP32 copy, or the
-                     // transposed hi/lo bf16 copies, of the precision forms)
-    GP_DKS = 1,      // Dpart[d] = Cp_d Cp_d^T (lower tiles)
-    GP_DRED = 2,     // D[d] mirrored from Dpart[d]
-    GP_GAMMA = 3,    // J pass 1
-    GP_GRED = 4,     // gamma reduction
+    GP_PAD = 0,      // Cp[n][ioff+i] = C[n][i] (FP64; also the half-transform's copy of
+                     // FP64 K, the FP32 copy, or the transposed hi/lo bf16 copies)
+    GP_DKS = 1,      // Dpart[d] = Cp_d Cp_d^T (lower tiles; precision forms)
+    GP_DRED = 2,     // D[d] mirrored from Dpart[d] (precision forms)
+    GP_GAMMA = 3,    // J pass 1 (precision forms)
+    GP_GRED = 4,     // gamma reduction (FP64: of the half-transform's row sums)
     GP_JACC = 5,     // J pass 2
     GP_JRED = 6,     // J reduction + mirror
     GP_KX = 7,       // half-transform (whole B: one chunk)
@@ -49,7 +49,7 @@ struct GJob {
     const int* rowoff;
     const double* C[2];
     double *Cp, *D, *Dpart, *gpart, *gamma, *jpart, *Kpart;
-    double* Cq;           // coefficients in the FP64 half-transform's order (FP64 K)
+    double *Cq, *grow;    // FP64: coefficients in the half-transform's order, its row sums
     float* Cp32;          // FP32 coefficients (FP32 K)
     u16 *Cth, *Ctl;       // transposed hi/lo coefficients (BF16x3 K)
     void* X;              // half-transformed chunk: FP64, FP32, or hi then lo bf16
@@ -83,7 +83,7 @@ __host__ __device__ inline int phase_blocks(const GJob& g, int phase) {
         case GP_DKS: return j * g.nlower * g.nd;
         case GP_DRED: return j * k_reduce_blocks(g.N) * g.nd;
         case GP_GAMMA: return j * g.neg * g.npc1;
-        case GP_GRED: return j * gcdiv((long long)g.nd * g.Q, 256);
+        case GP_GRED: return j * gcdiv((long long)g.nd * g.Q, PREC == F2JK_PREC_FP64 ? 4 : 256);
         case GP_JACC: return j * g.neg * g.npc2;
         case GP_JRED: return j * gcdiv(g.nvec, kJRedElems);
         case GP_KX:
@@ -101,7 +101,8 @@ __device__ __forceinline__ void grouped_kxd(char* lds, const GJob& g, int b, int
     if constexpr (NB <= kDMaxNB) {
         if (g.dnb == NB)
             kxd_body<NB, kxd_ib(NB)>(lds, (const double*)g.B, (long long)g.Q * g.N, g.N, g.Cq, g.dnks, (double*)g.X,
-                                     g.OPAD, g.OPAD, g.dncolt, b, nblocks);
+                                     g.OPAD, g.OPAD, g.dncolt, g.Cp, g.nd, g.ioff, g.width,
+                                     g.want_j ? g.grow : nullptr, (long long)g.Q * g.N, b, nblocks);
         else
             grouped_kxd<NB + 1>(lds, g, b, nblocks);
     }
@@ -145,7 +146,7 @@ void grouped_kernel(const GArgs a) {
                     if (k < g.N) g.Cp[(long long)k * g.OPAD + c] = x;
                 }
             } else if constexpr (PREC == F2JK_PREC_FP64) {
-                pack_cq_element(g.C, g.ldc, g.nd, g.nocc, g.ioff, g.N, g.OPAD, g.dnb, g.dnks, t, g.Cp, g.Cq);
+                pack_cq_element(g.C, g.ldc, g.nd, g.nocc, g.ioff, g.N, g.dncolt * g.dnb * 16, g.dnb, g.dnks, t, g.Cp, g.Cq);
             } else if (t < (long long)g.N * g.OPAD) {
                 const int n = (int)(t / g.OPAD), c = (int)(t % g.OPAD);
                 const int d = (g.nd == 2 && c >= g.ioff[1]) ? 1 : 0;
@@ -181,6 +182,9 @@ void grouped_kernel(const GArgs a) {
                 DPtrs<1> dp{{g.D}};
                 j_gamma_kernel_body<TB, 2, 4, 1>(B, g.N, g.Q, dp, g.N, g.rowoff, g.nvec, 32, g.gpart, bx, by);
             }
+        } else if constexpr (PHASE == GP_GRED && PREC == F2JK_PREC_FP64) {
+            gamma_rows_body(g.grow, (long long)g.Q * g.N, g.nd, g.dncolt, g.N, g.Q, g.gamma, g.Q,
+                            (long long)local * 4 + (tid >> 6));
         } else if constexpr (PHASE == GP_GRED) {
             const long long t = (long long)local * 256 + tid;
             if (t < (long long)g.nd * g.Q) {

@@ -62,8 +62,10 @@ enum f2jk_flags { F2JK_WANT_J = 1, F2JK_WANT_K = 2, F2JK_TIMING = 16 };
 
 /* phases reported by f2jk_last_timings (milliseconds, in this order) */
 enum f2jk_phase {
-    F2JK_PH_PREP = 0,      /* C padding, D = C C^T                           */
-    F2JK_PH_JGAMMA = 1,    /* J pass 1: gamma_P = sum_mn B_Pmn D_mn          */
+    F2JK_PH_PREP = 0,      /* C padding, D = C C^T (J without FP64 K)        */
+    F2JK_PH_JGAMMA = 1,    /* J pass 1: gamma_P = sum_mn B_Pmn D_mn (FP64 J
+                              and K from C: the sum of the half-transform's
+                              row sums, with no pass over B)                 */
     F2JK_PH_JACC = 2,      /* J pass 2: J_mn = sum_P gamma_P B_Pmn (+reduce) */
     F2JK_PH_KX = 3,        /* K half-transform X_Pmi = sum_n B_Pmn C_ni      */
     F2JK_PH_KS = 4,        /* K contraction K_mn += sum_Pi X_Pmi X_Pni       */
@@ -102,7 +104,7 @@ int f2jk_get_shape(const f2jk_ctx* ctx, int64_t* naux, int64_t* nbf);
  * 256 when nbf >= 768) is the lower-tile edge of the single-job BF16x3
  * contraction (256: one 8-wave workgroup per CU; grouped builds use 128);
  * "kx_wide" (-1, 0, 1; default -1 = above 128 occupied columns) runs the
- * FP64/FP32 half-transform in 128 x 320 tiles (8 waves), which read each
+ * FP32 half-transform in 128 x 320 tiles (8 waves), which read each
  * row block of B once instead of once per 128-column tile (the same products,
  * bitwise); "kx_rows" (0, 128, 256; default 0 = 256 when nbf >= 768 and nbf % 4 == 0)
  * is the row count of a single-job BF16x3 half-transform tile (256: 8 waves,
