@@ -69,8 +69,9 @@ struct f2jk_ctx {
     size_t xchunk_bytes = kDefaultXChunkBytes;
     bool j_nontemporal = true;
     int bf16_nbw_max = 10;          // widest BF16x3 half-transform tile: 32 * 10 columns
-    // J (HBM-bound) runs on a side stream concurrently with K (MFMA-bound)
-    bool overlap_jk = false;
+    // J (HBM-bound) runs on a side stream concurrently with K (MFMA-bound): 0, 1,
+    // -1 = FP64 builds whose J pass is long enough
+    int overlap_jk = -1;
     int kx_waves = 8;               // waves per BF16x3 half-transform workgroup (4 or 8)
     int ks_tile = 0;                // BF16x3 contraction tile edge: 128, 256, 0 = by nbf
     int kx_rows = 0;                // BF16x3 half-transform tile rows: 128, 256, 0 = by nbf
@@ -78,6 +79,7 @@ struct f2jk_ctx {
     int kx_wide = -1;               // FP64/FP32 half-transform in 320-column tiles: 0, 1, -1 = above 128 columns
     hipStream_t side = nullptr;     // default priority, created with the context
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    std::mutex ev_mu;               // an event is recorded and waited on in one piece
     int target_blocks = kTargetBlocks;
     // timing
     hipEvent_t ev[kMaxEvents];      // (start, end) pairs of non-nested phases
@@ -644,8 +646,9 @@ int build_d(f2jk_ctx* ctx, const Plan& p, char* ws, hipStream_t st) {
         hipLaunchKernelGGL(ks_kernel<double>, dim3(nlower), dim3(kGThreads), 0, st, cp, p.N, p.OPAD,
                            p.ioff[d], p.width[d], 1, 1, nlower, dpart, 0);
         F2JK_LAUNCHED("ks(D)");
-        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st,
-                           dpart, 1, p.N, dbuf + (size_t)d * p.N * p.N);
+        KPtrs dp{};
+        dp.p[0] = dbuf + (size_t)d * p.N * p.N;
+        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st, dpart, (int64_t)0, 1, p.N, dp);
         F2JK_LAUNCHED("k_reduce(D)");
     }
     return F2JK_OK;
@@ -750,29 +753,31 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const
         }
         TIM(F2JK_PH_KS, true);
         const int nsplit = std::min(p.nsplit, pc);
-        for (int d = 0; d < p.nd; ++d) {
-            double* kp = kpart + (size_t)d * p.nsplit * NN;
-            if constexpr (sizeof(T) == 8)
-                hipLaunchKernelGGL(ksd_kernel, dim3(p.dt.total), dim3(256), 0, st, X, p.N, p.OPAD, p.ioff[d],
-                                   p.width[d], pc, p.dt, kp, c > 0 ? 1 : 0);
-            else
-                hipLaunchKernelGGL(ks_kernel<T>, dim3(p.nlower * nsplit), dim3(kGThreads), 0, st, X, p.N,
-                                   p.OPAD, p.ioff[d], p.width[d], pc, nsplit, p.nlower, kp, c > 0 ? 1 : 0);
+        if constexpr (sizeof(T) == 8) {
+            hipLaunchKernelGGL(ksd_kernel, dim3(p.dt.total * p.nd), dim3(256), 0, st, X, p.N, p.OPAD, dcols_of(p, nocc),
+                               pc, p.dt, kpart, (int64_t)p.nsplit * NN, c > 0 ? 1 : 0);
             F2JK_LAUNCHED("ks");
+        } else {
+            for (int d = 0; d < p.nd; ++d) {
+                hipLaunchKernelGGL(ks_kernel<T>, dim3(p.nlower * nsplit), dim3(kGThreads), 0, st, X, p.N,
+                                   p.OPAD, p.ioff[d], p.width[d], pc, nsplit, p.nlower,
+                                   kpart + (size_t)d * p.nsplit * NN, c > 0 ? 1 : 0);
+                F2JK_LAUNCHED("ks");
+            }
         }
         TIM(F2JK_PH_KS, false);
     }
     TIM(F2JK_PH_KRED, true);
     const int nsplit_used = std::min(p.nsplit, std::min(p.Pc, p.Q));
-    for (int d = 0; d < p.nd; ++d) {
-        double* kp = kpart + (size_t)d * p.nsplit * NN;
-        if constexpr (sizeof(T) == 8)
-            hipLaunchKernelGGL(kred_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st, kp, p.dt, p.N, K[d]);
-        else
-            hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st, kp, nsplit_used, p.N,
-                               K[d]);
-        F2JK_LAUNCHED("k_reduce");
-    }
+    KPtrs kp{};
+    for (int d = 0; d < p.nd; ++d) kp.p[d] = K[d];
+    if constexpr (sizeof(T) == 8)
+        hipLaunchKernelGGL(kred_kernel, dim3(k_reduce_blocks(p.N), p.nd), dim3(256), 0, st, kpart,
+                           (int64_t)p.nsplit * NN, p.dt, p.N, kp);
+    else
+        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N), p.nd), dim3(256), 0, st, kpart,
+                           (int64_t)p.nsplit * NN, nsplit_used, p.N, kp);
+    F2JK_LAUNCHED("k_reduce");
     TIM(F2JK_PH_KRED, false);
     return F2JK_OK;
 }
@@ -873,14 +878,24 @@ int run_k_bf16x3(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipSt
     }
     TIM(F2JK_PH_KRED, true);
     const int nsplit_used = std::min(p.nsplit, std::min(p.Pc, p.Q));
-    for (int d = 0; d < p.nd; ++d) {
-        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st,
-                           kpart + (size_t)d * p.nsplit * NN, nsplit_used, p.N, K[d]);
-        F2JK_LAUNCHED("k_reduce");
-    }
+    KPtrs kp{};
+    for (int d = 0; d < p.nd; ++d) kp.p[d] = K[d];
+    hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N), p.nd), dim3(256), 0, st, kpart,
+                       (int64_t)p.nsplit * NN, nsplit_used, p.N, kp);
+    F2JK_LAUNCHED("k_reduce");
     TIM(F2JK_PH_KRED, false);
     return F2JK_OK;
 }
+
+// FP64 J beside K pays from a J pass of this many bytes on: the second pass then
+// reads B while the contraction (two waves of 182 registers and 64 KB of LDS
+// per workgroup, so J's waves fit beside it) keeps the matrix cores busy.
+// nbf 384 (B 1.3 GB in the pass) 1608 -> 1435 us per build, nbf 318 (0.3 GB)
+// 408 -> 376, nbf 1152 99.1 -> 97.5 ms; at nbf 115 (28 MB) the events cost more
+// than the 8 us pass (61 -> 73 us).  The kernels of the precision forms fill
+// the register file and gain 1%.
+constexpr double kOverlapBytes = 128e6;
+double j_pass_bytes(const Plan& p) { return (double)p.nvec * p.jvec * p.jb * p.Q; }
 
 int check_ws(const Plan& p, void* ws, size_t ws_bytes) {
     if (!ws) return fail(F2JK_EINVAL, "workspace pointer is NULL");
@@ -920,13 +935,18 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
     }
     // the J passes: on the side stream (forked once their inputs exist) when they
     // run beside K
-    const bool overlap = p.want_j && p.want_k && ctx->overlap_jk;
+    const bool overlap = p.want_j && p.want_k &&
+                         (ctx->overlap_jk < 0 ? p.gamma_x && !ctx->timing && j_pass_bytes(p) >= kOverlapBytes
+                                              : ctx->overlap_jk == 1);
     hipStream_t sj = overlap ? ctx->side : st;
+    bool forked = false;
     auto do_j = [&]() -> int {
         if (!p.want_j) return F2JK_OK;
         if (overlap) {
+            std::lock_guard<std::mutex> lock(ctx->ev_mu);
             F2JK_HIP(hipEventRecord(ctx->ev_fork, st));
             F2JK_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
+            forked = true;
         }
         if (p.gamma_x) return run_j(ctx, p, nullptr, 0, J, w, sj);
         std::vector<const double*> dptr(ndens);
@@ -934,21 +954,23 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
             dptr[d] = j_from_c ? (const double*)(w + p.off_d) + (size_t)d * p.N * p.N : Din[d];
         return run_j(ctx, p, dptr.data(), j_from_c ? p.N : ldd, J, w, sj);
     };
-    if (!p.gamma_x && (rc = do_j())) return rc;
-    if (p.want_k) {
+    if (!p.gamma_x) rc = do_j();
+    if (!rc && p.want_k) {
         if (p.prec == F2JK_PREC_BF16X3)
             rc = run_k_bf16x3(ctx, p, K, w, st);
         else if (p.tk == 8)
             rc = run_k_typed<double>(ctx, p, nocc, K, w, st, [&] { return p.gamma_x ? do_j() : F2JK_OK; });
         else
             rc = run_k_typed<float>(ctx, p, nocc, K, w, st, [] { return F2JK_OK; });
-        if (rc) return rc;
     }
-    // join: later work on the caller's stream sees J
-    if (overlap) {
+    // join, also after a failed launch: later work on the caller's stream comes
+    // after the side stream's
+    if (forked) {
+        std::lock_guard<std::mutex> lock(ctx->ev_mu);
         F2JK_HIP(hipEventRecord(ctx->ev_join, sj));
         F2JK_HIP(hipStreamWaitEvent(st, ctx->ev_join, 0));
     }
+    if (rc) return rc;
     TIM(F2JK_PH_TOTAL, false);
     g_last_error.clear();
     return F2JK_OK;
@@ -1215,7 +1237,7 @@ int f2jk_set_tuning(f2jk_ctx* ctx, const char* key, int64_t value) {
             return fail(F2JK_EINVAL, "bf16_nbw_max must be 2, 4, 5, 6, 8 or 10");
         ctx->bf16_nbw_max = (int)value;
     } else if (!strcmp(key, "overlap_jk")) {
-        ctx->overlap_jk = value != 0;
+        ctx->overlap_jk = value < 0 ? -1 : value != 0;
     } else if (!strcmp(key, "ks_tile")) {
         if (value != 0 && value != 128 && value != 256) return fail(F2JK_EINVAL, "ks_tile must be 0, 128 or 256");
         ctx->ks_tile = (int)value;

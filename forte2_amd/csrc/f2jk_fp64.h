@@ -495,22 +495,24 @@ __device__ __forceinline__ void ksd_body(char* lds, const double* __restrict__ X
         }
     }
 }
-__global__ __launch_bounds__(256, 2) void ksd_kernel(const double* __restrict__ X, int N, int OPAD, int ioff,
-                                                     int width, int Pc, DTiles tm, double* __restrict__ Kpart,
+// all densities in one launch (the partials of one are dstride doubles)
+__global__ __launch_bounds__(256, 2) void ksd_kernel(const double* __restrict__ X, int N, int OPAD, DCols dc, int Pc,
+                                                     DTiles tm, double* __restrict__ Kpart, int64_t dstride,
                                                      int accumulate) {
     __shared__ __attribute__((aligned(16))) char lds[kDKsLds];
-    ksd_body(lds, X, N, OPAD, ioff, width, Pc, tm, Kpart, accumulate, blockIdx.x);
+    const int d = blockIdx.x / tm.total;
+    ksd_body(lds, X, N, OPAD, dc.ioff[d], dc.width[d], Pc, tm, Kpart + d * dstride, accumulate, blockIdx.x % tm.total);
 }
 
 // the reduction over the splits of the element's tile
 __device__ __forceinline__ int dtile_splits(const DTiles& m, int m4, int n16) {
     return m.ns[dtile_kind(m, m4 * 4 / kTile, n16 * 16 / kTile)];
 }
-__global__ __launch_bounds__(256) void kred_kernel(const double* __restrict__ Kpart, DTiles tm, int N,
-                                                   double* __restrict__ K) {
+__global__ __launch_bounds__(256) void kred_kernel(const double* __restrict__ Kpart, int64_t dstride, DTiles tm,
+                                                   int N, KPtrs K) {
     const int nb = (N + 15) / 16, m4 = blockIdx.x / nb, n16 = blockIdx.x % nb;
     if (n16 * 16 > m4 * 4 + 3) return;
-    k_reduce_body(Kpart, dtile_splits(tm, m4, n16), N, K, m4, n16);
+    k_reduce_body(Kpart + blockIdx.y * dstride, dtile_splits(tm, m4, n16), N, K.p[blockIdx.y], m4, n16);
 }
 
 }  // namespace f2jk

@@ -1707,11 +1707,16 @@ __device__ __forceinline__ void k_reduce_body(const double* __restrict__ Kpart, 
 }
 // blocks of the reduction of one N x N matrix (n16 past the diagonal: nothing to do)
 __host__ __device__ inline int k_reduce_blocks(int N) { return ((N + 3) / 4) * ((N + 15) / 16); }
-__global__ __launch_bounds__(256) void k_reduce_kernel(const double* __restrict__ Kpart, int nsplit, int N,
-                                                       double* __restrict__ K) {
+// the K (or D) of every density of a call
+struct KPtrs {
+    double* p[8];
+};
+// grid (k_reduce_blocks(N), densities); the partials of one density are dstride doubles
+__global__ __launch_bounds__(256) void k_reduce_kernel(const double* __restrict__ Kpart, int64_t dstride, int nsplit,
+                                                       int N, KPtrs K) {
     const int nb = (N + 15) / 16, m4 = blockIdx.x / nb, n16 = blockIdx.x % nb;
     if (n16 * 16 > m4 * 4 + 3) return;
-    k_reduce_body(Kpart, nsplit, N, K, m4, n16);
+    k_reduce_body(Kpart + blockIdx.y * dstride, nsplit, N, K.p[blockIdx.y], m4, n16);
 }
 
 // Cp[n][ioff + i] = C[n][i] (i < nocc), zero for nocc <= i < width.

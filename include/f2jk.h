@@ -93,8 +93,9 @@ int f2jk_get_shape(const f2jk_ctx* ctx, int64_t* naux, int64_t* nbf);
  * none): "xchunk_bytes" caps the half-transformed chunk X held in the
  * workspace (default 4 GiB); "target_blocks" is the number of workgroups a
  * split launch aims for (default 2048); "j_nontemporal" (0/1, default 1)
- * streams B through non-temporal loads in the J passes; "overlap_jk" (0/1,
- * default 0) runs the J passes of a build_jk on the context's side stream
+ * streams B through non-temporal loads in the J passes; "overlap_jk" (0, 1,
+ * -1; default -1 = FP64 J and K from C with a J pass of 128 MB or more, unless
+ * F2JK_TIMING is asked for) runs the J passes of a build_jk on the context's side stream
  * concurrently with K (joined back before the call returns its work to the
  * caller's stream); "bf16_nbw_max" (2, 4, 5, 6, 8, 10) caps the BF16x3
  * half-transform tile at 32 * value occupied columns (tiles of up to 5 run two
