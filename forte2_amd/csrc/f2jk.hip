@@ -64,6 +64,10 @@ struct f2jk_ctx {
     bool j_sparse = false;
     uint32_t* jlist[2] = {nullptr, nullptr};
     int* jinv[2] = {nullptr, nullptr};   // lower-triangle element -> place in the list, or -1
+    // the listed elements of a copy one after the other (P-major), when asked for
+    // ("j_pack") and there is room: the J passes then read whole lines
+    bool j_pack = false;
+    void* jpacked[2] = {nullptr, nullptr};
     int jlist_vec[2] = {0, 0};
     int jlist_n[2] = {0, 0};
     size_t xchunk_bytes = kDefaultXChunkBytes;
@@ -107,6 +111,7 @@ struct Plan {
     int jvec = 1, nvec = 0, neg = 0, npc1 = 0, ppw2 = 0, npc2 = 0;
     const uint32_t* jlist = nullptr;  // element list of the J passes (null: every element)
     const int* jinv = nullptr;        // element -> place in that list
+    const void* jpacked = nullptr;    // the listed elements, packed
     int jdense = 0;                   // lower-triangle elements in all
     size_t jb = 8;             // bytes of a B element read by J
     // K
@@ -161,13 +166,58 @@ int ensure_rowoff(f2jk_ctx* ctx, int vec) {
 template <typename TB, int VEC>
 int scan_jlist(f2jk_ctx* ctx, const TB* B, unsigned char* flag) {
     const int nvec = ctx->nvec[VEC];
-    hipLaunchKernelGGL((j_scan_kernel<TB, VEC>), dim3((unsigned)cdiv(nvec, 256)), dim3(256), 0, nullptr, B,
+    hipLaunchKernelGGL(fill_bytes_kernel, dim3((unsigned)cdiv(nvec, 256)), dim3(256), 0, nullptr, flag, nvec);
+    F2JK_LAUNCHED("fill_bytes");
+    const unsigned ny = (unsigned)std::max<int64_t>(1, std::min<int64_t>(64, ctx->naux / 32));
+    hipLaunchKernelGGL((j_scan_kernel<TB, VEC>), dim3((unsigned)cdiv(nvec, 256), ny), dim3(256), 0, nullptr, B,
                        (int)ctx->nbf, (int)ctx->naux, ctx->rowoff[VEC], nvec, flag);
     F2JK_LAUNCHED("j_scan");
     return F2JK_OK;
 }
 
+template <typename TB, int VEC>
+int pack_jlist(f2jk_ctx* ctx, int dtype, const TB* B) {
+    const int n = ctx->jlist_n[dtype];
+    const unsigned ny = (unsigned)std::max<int64_t>(1, std::min<int64_t>(ctx->naux, 128));
+    hipLaunchKernelGGL((j_pack_kernel<TB, VEC>), dim3((unsigned)cdiv(n, 256), ny), dim3(256), 0, nullptr, B,
+                       (int)ctx->nbf, (int)ctx->naux, ctx->jlist[dtype], n, (TB*)ctx->jpacked[dtype]);
+    F2JK_LAUNCHED("j_pack");
+    return F2JK_OK;
+}
+
+// The packed elements of copy `dtype`, where they save bytes and a sixteenth of
+// the free memory holds them (a build that just fits the card keeps its room;
+// the passes give the same J, bitwise, either way).
+int build_jpacked(f2jk_ctx* ctx, int dtype) {
+    const int64_t N = ctx->nbf, n = ctx->jlist_n[dtype];
+    const int vec = ctx->jlist_vec[dtype];
+    const double esize = dtype == F2JK_F64 ? 8.0 : 4.0;
+    const double bytes = (double)n * vec * esize * (double)ctx->naux;
+    if ((double)n * vec > 0.85 * (double)N * (N + 1) / 2) return F2JK_OK;
+    size_t free_b = 0, total_b = 0;
+    F2JK_HIP(hipMemGetInfo(&free_b, &total_b));
+    if (bytes > (double)free_b / 16) return F2JK_OK;
+    if (hipMalloc(&ctx->jpacked[dtype], (size_t)bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->jpacked[dtype] = nullptr;
+        return F2JK_OK;
+    }
+    int rc;
+    if (dtype == F2JK_F64)
+        rc = vec == 2 ? pack_jlist<double, 2>(ctx, dtype, (const double*)ctx->B[dtype])
+                      : pack_jlist<double, 1>(ctx, dtype, (const double*)ctx->B[dtype]);
+    else
+        rc = vec == 4 ? pack_jlist<float, 4>(ctx, dtype, (const float*)ctx->B[dtype])
+           : vec == 2 ? pack_jlist<float, 2>(ctx, dtype, (const float*)ctx->B[dtype])
+                      : pack_jlist<float, 1>(ctx, dtype, (const float*)ctx->B[dtype]);
+    if (rc) return rc;
+    F2JK_HIP(hipStreamSynchronize(nullptr));  // builds on any stream read it
+    return F2JK_OK;
+}
+
 void free_jlist(f2jk_ctx* ctx, int dtype) {
+    if (ctx->jpacked[dtype]) (void)hipFree(ctx->jpacked[dtype]);
+    ctx->jpacked[dtype] = nullptr;
     if (ctx->jlist[dtype]) (void)hipFree(ctx->jlist[dtype]);
     if (ctx->jinv[dtype]) (void)hipFree(ctx->jinv[dtype]);
     ctx->jlist[dtype] = nullptr;
@@ -215,6 +265,7 @@ int build_jlist(f2jk_ctx* ctx, int dtype) {
     F2JK_HIP(hipMemcpy(ctx->jinv[dtype], inv.data(), inv.size() * sizeof(int), hipMemcpyHostToDevice));
     ctx->jlist_vec[dtype] = vec;
     ctx->jlist_n[dtype] = (int)list.size();
+    if (ctx->j_pack && dtype == F2JK_F32) return build_jpacked(ctx, dtype);
     return F2JK_OK;
 }
 
@@ -369,6 +420,7 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         if (!grouped && ctx->jlist[jdtype] && ctx->jlist_vec[jdtype] == p.jvec) {
             p.jlist = ctx->jlist[jdtype];
             p.jinv = ctx->jinv[jdtype];
+            p.jpacked = ctx->jpacked[jdtype];
             nvec = ctx->jlist_n[jdtype];
         }
         p.nvec = (int)nvec;
@@ -513,7 +565,8 @@ int launch_j(f2jk_ctx* ctx, const Plan& p, const TB* B, int d0, const double* co
     if (D) {
         TIM(F2JK_PH_JGAMMA, true);
         hipLaunchKernelGGL((j_gamma_kernel<TB, VEC, kEPT, ND, NT>), dim3(p.neg, p.npc1), dim3(kJThreads), 0,
-                           st, B, p.N, p.Q, dp, ldd, rowoff, elist, p.nvec, kJ1PerBlock, gpart);
+                           st, B, p.N, p.Q, dp, ldd, rowoff, elist, (const TB*)p.jpacked, p.nvec, kJ1PerBlock,
+                           gpart);
         F2JK_LAUNCHED("j_gamma");
         const int64_t ng = (int64_t)ND * p.Q;
         hipLaunchKernelGGL(j_gamma_reduce_kernel, dim3((unsigned)cdiv(ng, 256)), dim3(256), 0, st,
@@ -523,7 +576,7 @@ int launch_j(f2jk_ctx* ctx, const Plan& p, const TB* B, int d0, const double* co
     }
     TIM(F2JK_PH_JACC, true);
     hipLaunchKernelGGL((j_accum_kernel<TB, VEC, kEPT, ND, NT>), dim3(p.neg, p.npc2), dim3(kJThreads), 0,
-                       st, B, p.N, p.Q, gamma, rowoff, elist, p.nvec, p.ppw2, jpart);
+                       st, B, p.N, p.Q, gamma, rowoff, elist, (const TB*)p.jpacked, p.nvec, p.ppw2, jpart);
     F2JK_LAUNCHED("j_accum");
     hipLaunchKernelGGL((j_reduce_kernel<VEC, ND>), dim3((unsigned)cdiv(p.jdense, kJRedElems)), dim3(kJThreads), 0,
                        st, jpart, p.npc2, p.N, rowoff, p.jinv, p.nvec, p.jdense, jp);
@@ -815,7 +868,8 @@ void launch_kx_bf16_tall(const Plan& p, unsigned grid, const float* A, int64_t R
                        p.OPAD, xh, xl, p.ncolt);
 }
 
-int run_k_bf16x3(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipStream_t st) {
+template <typename F>
+int run_k_bf16x3(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipStream_t st, F&& after_kx) {
     const float* B = (const float*)ctx->B[F2JK_F32];
     const u16* th = (const u16*)(ws + p.off_cth);
     const u16* tl = (const u16*)(ws + p.off_ctl);
@@ -852,6 +906,10 @@ int run_k_bf16x3(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipSt
         }
         F2JK_LAUNCHED("kx_bf16x3");
         TIM(F2JK_PH_KX, false);
+        if (c + 1 == p.nchunks) {
+            const int rc = after_kx();
+            if (rc) return rc;
+        }
         TIM(F2JK_PH_KS, true);
         const int nsplit = std::min(p.nsplit, pc);
         const bool ks_dma = ctx->ks_dma < 0 ? p.ks_tile == 256 : ctx->ks_dma == 1;
@@ -892,8 +950,11 @@ int run_k_bf16x3(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipSt
 // per workgroup, so J's waves fit beside it) keeps the matrix cores busy.
 // nbf 384 (B 1.3 GB in the pass) 1608 -> 1435 us per build, nbf 318 (0.3 GB)
 // 408 -> 376, nbf 1152 99.1 -> 97.5 ms; at nbf 115 (28 MB) the events cost more
-// than the 8 us pass (61 -> 73 us).  The kernels of the precision forms fill
-// the register file and gain 1%.
+// than the 8 us pass (61 -> 73 us).  In the BF16x3 form both passes run beside
+// the last chunk's contraction (nbf 960: 11.84 -> 11.38 ms); beside the
+// half-transform, which fills the register file, they gained 1%, and beside the
+// contraction in 128-wide tiles, itself bound by reading X, nothing (nbf 384:
+// 769 and 775 us).
 constexpr double kOverlapBytes = 128e6;
 double j_pass_bytes(const Plan& p) { return (double)p.nvec * p.jvec * p.jb * p.Q; }
 
@@ -936,7 +997,8 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
     // the J passes: on the side stream (forked once their inputs exist) when they
     // run beside K
     const bool overlap = p.want_j && p.want_k &&
-                         (ctx->overlap_jk < 0 ? p.gamma_x && !ctx->timing && j_pass_bytes(p) >= kOverlapBytes
+                         (ctx->overlap_jk < 0 ? (p.gamma_x || (p.prec == F2JK_PREC_BF16X3 && p.ks_tile == 256)) &&
+                                                    !ctx->timing && j_pass_bytes(p) >= kOverlapBytes
                                               : ctx->overlap_jk == 1);
     hipStream_t sj = overlap ? ctx->side : st;
     bool forked = false;
@@ -954,10 +1016,12 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
             dptr[d] = j_from_c ? (const double*)(w + p.off_d) + (size_t)d * p.N * p.N : Din[d];
         return run_j(ctx, p, dptr.data(), j_from_c ? p.N : ldd, J, w, sj);
     };
-    if (!p.gamma_x) rc = do_j();
+    // J once the last half-transform is queued (FP64: its gamma comes with it)
+    const bool j_late = p.gamma_x || (overlap && p.prec == F2JK_PREC_BF16X3);
+    if (!j_late) rc = do_j();
     if (!rc && p.want_k) {
         if (p.prec == F2JK_PREC_BF16X3)
-            rc = run_k_bf16x3(ctx, p, K, w, st);
+            rc = run_k_bf16x3(ctx, p, K, w, st, [&] { return j_late ? do_j() : F2JK_OK; });
         else if (p.tk == 8)
             rc = run_k_typed<double>(ctx, p, nocc, K, w, st, [&] { return p.gamma_x ? do_j() : F2JK_OK; });
         else
@@ -1222,6 +1286,12 @@ int f2jk_set_tuning(f2jk_ctx* ctx, const char* key, int64_t value) {
             } else {
                 free_jlist(ctx, dt);
             }
+        }
+    } else if (!strcmp(key, "j_pack")) {
+        ctx->j_pack = value != 0;
+        if (ctx->j_sparse) {
+            int rc = build_jlist(ctx, F2JK_F32);
+            if (rc) return rc;
         }
     } else if (!strcmp(key, "ks_dma")) {
         if (value < -1 || value > 1) return fail(F2JK_EINVAL, "ks_dma must be -1, 0 or 1");

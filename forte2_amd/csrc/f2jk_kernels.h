@@ -132,10 +132,11 @@ template <typename TB, int VEC, int EPT, int ND, bool NT = false>
 __device__ __forceinline__ void j_gamma_kernel_body(
     const TB* __restrict__ B, int N, int Q, DPtrs<ND> D, int64_t ldd,
     const int* __restrict__ rowoff, int nvec, int ppw, double* __restrict__ gpart, int bx, int by,
-    const uint32_t* __restrict__ elist = nullptr) {
+    const uint32_t* __restrict__ elist = nullptr, const TB* __restrict__ packed = nullptr) {
     __shared__ double red[kJThreads / kWave][kJFlush][ND];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
-    const int64_t NN = (int64_t)N * N;
+    const int64_t NN = packed ? (int64_t)nvec * VEC : (int64_t)N * N;
+    if (packed) B = packed;
 
     int64_t off[EPT];
     double d[EPT][ND][VEC];
@@ -150,7 +151,7 @@ __device__ __forceinline__ void j_gamma_kernel_body(
         if (e < nvec) {
             int m, col;
             j_element<VEC>(rowoff, elist, N, e, m, col);
-            off[k] = (int64_t)m * N + col;
+            off[k] = packed ? (int64_t)e * VEC : (int64_t)m * N + col;
 #pragma unroll
             for (int v = 0; v < VEC; ++v) {
                 const int c = col + v;
@@ -236,10 +237,10 @@ __device__ __forceinline__ void j_gamma_kernel_body(
 template <typename TB, int VEC, int EPT, int ND, bool NT = false>
 __global__ __launch_bounds__(kJThreads) void j_gamma_kernel(
     const TB* __restrict__ B, int N, int Q, DPtrs<ND> D, int64_t ldd,
-    const int* __restrict__ rowoff, const uint32_t* __restrict__ elist, int nvec, int ppw,
-    double* __restrict__ gpart) {
+    const int* __restrict__ rowoff, const uint32_t* __restrict__ elist, const TB* __restrict__ packed, int nvec,
+    int ppw, double* __restrict__ gpart) {
     j_gamma_kernel_body<TB, VEC, EPT, ND, NT>(B, N, Q, D, ldd, rowoff, nvec, ppw, gpart, blockIdx.x, blockIdx.y,
-                                              elist);
+                                              elist, packed);
 }
 
 
@@ -262,9 +263,10 @@ template <typename TB, int VEC, int EPT, int ND, bool NT = false>
 __device__ __forceinline__ void j_accum_kernel_body(
     const TB* __restrict__ B, int N, int Q, const double* __restrict__ gamma,
     const int* __restrict__ rowoff, int nvec, int ppw, double* __restrict__ jpart, int bx, int by,
-    const uint32_t* __restrict__ elist = nullptr) {
+    const uint32_t* __restrict__ elist = nullptr, const TB* __restrict__ packed = nullptr) {
     const int tid = threadIdx.x;
-    const int64_t NN = (int64_t)N * N;
+    const int64_t NN = packed ? (int64_t)nvec * VEC : (int64_t)N * N;
+    if (packed) B = packed;
     int64_t off[EPT];
     int eidx[EPT];
 #pragma unroll
@@ -273,9 +275,13 @@ __device__ __forceinline__ void j_accum_kernel_body(
         eidx[k] = e;
         off[k] = 0;
         if (e < nvec) {
-            int m, col;
-            j_element<VEC>(rowoff, elist, N, e, m, col);
-            off[k] = (int64_t)m * N + col;
+            if (packed) {
+                off[k] = (int64_t)e * VEC;
+            } else {
+                int m, col;
+                j_element<VEC>(rowoff, elist, N, e, m, col);
+                off[k] = (int64_t)m * N + col;
+            }
         }
     }
     double acc[EPT][ND][VEC];
@@ -341,10 +347,10 @@ __device__ __forceinline__ void j_accum_kernel_body(
 template <typename TB, int VEC, int EPT, int ND, bool NT = false>
 __global__ __launch_bounds__(kJThreads) void j_accum_kernel(
     const TB* __restrict__ B, int N, int Q, const double* __restrict__ gamma,
-    const int* __restrict__ rowoff, const uint32_t* __restrict__ elist, int nvec, int ppw,
-    double* __restrict__ jpart) {
+    const int* __restrict__ rowoff, const uint32_t* __restrict__ elist, const TB* __restrict__ packed, int nvec,
+    int ppw, double* __restrict__ jpart) {
     j_accum_kernel_body<TB, VEC, EPT, ND, NT>(B, N, Q, gamma, rowoff, nvec, ppw, jpart, blockIdx.x, blockIdx.y,
-                                              elist);
+                                              elist, packed);
 }
 
 
@@ -413,23 +419,52 @@ __global__ __launch_bounds__(kJThreads) void j_reduce_kernel(const double* __res
 
 // flag[e] = 1 when B[P][m][c] != 0 for some P and some c <= m of vector
 // element e (lower triangle, numbered row after row): the elements the J
-// passes have to read.  One thread per element, all P.
+// passes have to read.  One thread per element and range of P (blockIdx.y);
+// flag starts at zero and a thread that finds its element flagged by another
+// range stops (one range over all P left most of the chip idle: 1.2 ms at nbf
+// 384, 2224 P).
 template <typename TB, int VEC>
 __global__ void j_scan_kernel(const TB* __restrict__ B, int N, int Q, const int* __restrict__ rowoff, int nvec,
-                              unsigned char* __restrict__ flag) {
+                              volatile unsigned char* flag) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= nvec) return;
     const int m = find_row(rowoff, N, e);
     const int col = (e - rowoff[m]) * VEC;
     const int64_t NN = (int64_t)N * N;
     const TB* p = B + (int64_t)m * N + col;
-    int nz = 0;
-    for (int P = 0; P < Q && !nz; ++P) {
-        const Vec<TB, VEC> b = load_vec<TB, VEC>(p + P * NN);
+    const int P0 = (int)((int64_t)Q * blockIdx.y / gridDim.y), P1 = (int)((int64_t)Q * (blockIdx.y + 1) / gridDim.y);
+    for (int P = P0; P < P1; P += 8) {
+        if (flag[e]) return;
+        int nz = 0;
+        const int np = min(8, P1 - P);
+        for (int i = 0; i < np; ++i) {
+            const Vec<TB, VEC> b = load_vec<TB, VEC>(p + (P + i) * NN);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) nz |= (col + v <= m) && (b.v[v] != TB(0));
+            for (int v = 0; v < VEC; ++v) nz |= (col + v <= m) && (b.v[v] != TB(0));
+        }
+        if (nz) {
+            flag[e] = 1;
+            return;
+        }
     }
-    flag[e] = (unsigned char)nz;
+}
+__global__ void fill_bytes_kernel(unsigned char* __restrict__ x, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) x[i] = 0;
+}
+// out[P][i] = the listed vector element i of B_P: what the J passes read, one
+// after the other.  In B the listed elements lie scattered in 16-byte pieces,
+// and whole 128-byte lines come from memory for them.
+template <typename TB, int VEC>
+__global__ void j_pack_kernel(const TB* __restrict__ B, int N, int Q, const uint32_t* __restrict__ elist, int n,
+                              TB* __restrict__ out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t x = elist[i];
+    const TB* p = B + (int64_t)(x >> 16) * N + (x & 0xffffu);
+    const int64_t NN = (int64_t)N * N;
+    for (int P = blockIdx.y; P < Q; P += gridDim.y)
+        *reinterpret_cast<Vec<TB, VEC>*>(out + ((int64_t)P * n + i) * VEC) = load_vec<TB, VEC>(p + P * NN);
 }
 
 // ---------------------------------------------------------------------------

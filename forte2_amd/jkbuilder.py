@@ -136,6 +136,8 @@ class FockBuilder:
             # fixed once formed; the scan happens here and when the FP32 copy
             # is registered)
             if self.j_sparse:
+                # the FP32 copy is this builder's own: its listed elements may be packed
+                self._tune("j_pack", 1)
                 self._tune("j_sparse", 1)
         return self._ctx
 

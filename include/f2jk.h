@@ -18,8 +18,8 @@
  *     given hipStream_t (NULL = default stream) and never synchronises.
  *   - Scratch memory is supplied by the caller (ws, ws_bytes); query its size
  *     with f2jk_workspace_size.  The library allocates device memory only in
- *     f2jk_ctx_create / f2jk_set_B / f2jk_set_tuning("j_sparse") (small
- *     index tables).
+ *     f2jk_ctx_create / f2jk_set_B / f2jk_set_tuning("j_sparse", "j_pack")
+ *     (small index tables; the packed elements of "j_pack").
  *   - Reductions are deterministic: a result depends only on the inputs and
  *     the context's shapes, never on concurrent work.
  *   - Return value: 0 on success, a negative f2jk_status otherwise; the
@@ -94,8 +94,8 @@ int f2jk_get_shape(const f2jk_ctx* ctx, int64_t* naux, int64_t* nbf);
  * workspace (default 4 GiB); "target_blocks" is the number of workgroups a
  * split launch aims for (default 2048); "j_nontemporal" (0/1, default 1)
  * streams B through non-temporal loads in the J passes; "overlap_jk" (0, 1,
- * -1; default -1 = FP64 J and K from C with a J pass of 128 MB or more, unless
- * F2JK_TIMING is asked for) runs the J passes of a build_jk on the context's side stream
+ * -1; default -1 = FP64 J and K from C, and BF16x3 with 256-wide contraction
+ * tiles, when a J pass reads 128 MB or more and F2JK_TIMING is not asked for) runs the J passes of a build_jk on the context's side stream
  * concurrently with K (joined back before the call returns its work to the
  * caller's stream); "bf16_nbw_max" (2, 4, 5, 6, 8, 10) caps the BF16x3
  * half-transform tile at 32 * value occupied columns (tiles of up to 5 run two
@@ -119,7 +119,12 @@ int f2jk_get_shape(const f2jk_ctx* ctx, int64_t* naux, int64_t* nbf);
  * its screened shell pairs: ~75% of the FP64 elements of (H2O)_64); J
  * elsewhere is exactly zero, as in the full sum.  B's zero pattern must not
  * change while registered (register it again to rescan).  The scan
- * synchronises the device.
+ * synchronises the device; "j_pack" (0/1, default 0): with j_sparse, the
+ * listed elements of the F32 copy are also kept one after the other in
+ * memory of the library (where they are less than 85% of the lower triangle
+ * and a sixteenth of the free device memory holds them), so that the J passes
+ * read whole lines; the same J, bitwise.  The copy's values must then not
+ * change while registered either.
  * Set by the autotuner. */
 int f2jk_set_tuning(f2jk_ctx* ctx, const char* key, int64_t value);
 

@@ -39,3 +39,20 @@ def test_zero_tensor(dev):
     for prec in ("fp64", "bf16x3"):
         J, K = fb.build_JK([C], precision=prec)
         assert float(J[0].abs().max()) == 0.0 and float(K[0].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("N,keep", [(7, 3), (36, 12), (64, 4), (130, 40)])
+def test_packed_elements_give_the_same_j(dev, N, keep):
+    # the J passes over the packed nonzero elements of the FP32 copy read the
+    # same elements in the same order: bitwise J, for J from C and from D
+    Q = 45
+    B = synthetic_B(Q, N, seed=N, device=dev)
+    i = torch.arange(N, device=dev)
+    B.mul_(((i[:, None] - i[None, :]).abs() < keep).to(B.dtype))
+    C = orthonormal_C(N, 3, seed=2, device=dev)
+    out = []
+    for pack in (0, 1):
+        fb = FockBuilder(B=B, device=dev, precision="bf16x3")
+        fb.set_tuning("j_pack", pack)
+        out.append(fb.build_JK([C])[0] + fb.build_J([C @ C.T]))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
