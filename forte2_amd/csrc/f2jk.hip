@@ -763,6 +763,18 @@ void launch_kxd(const Plan& p, const double* A, int64_t R, const double* cq, dou
     }
 }
 
+template <int NB = 1>
+void launch_kxt(int nb, const double* M, int64_t pstride, int ld, int K, int ncol, int64_t nP, const double* cq, int nks,
+                double* Y, int ni, int ncolt, hipStream_t st) {
+    if constexpr (NB <= kDMaxNB) {
+        if (nb != NB) return launch_kxt<NB + 1>(nb, M, pstride, ld, K, ncol, nP, cq, nks, Y, ni, ncolt, st);
+        constexpr int IB = kxd_ib(NB);
+        const int64_t nblocks = nP * cdiv(ncol, 16);
+        hipLaunchKernelGGL((kxt_kernel<NB, IB>), dim3((unsigned)(cdiv(nblocks, 4 * IB) * ncolt)), dim3(256), 0, st, M,
+                           pstride, ld, K, ncol, nblocks, cq, nks, Y, ni, ncolt);
+    }
+}
+
 // `after_kx` runs once the last chunk's half-transform (and gamma) is queued
 template <typename T, typename F>
 int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const* K, char* ws, hipStream_t st,
@@ -1560,6 +1572,94 @@ int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ld
         const int64_t R = std::min<int64_t>(step, p1 - P0) * p.N;
         launch_kxd(p, B + P0 * NN, R, cq, X + (P0 - p0) * p.N * ldx, ldx, (int)ncol, KxdGamma{}, st);
         F2JK_LAUNCHED("kx");
+    }
+    g_last_error.clear();
+    return F2JK_OK;
+}
+
+// Scratch of f2jk_mo_block: both coefficient sets, and the intermediate of one
+// block of P.  64 MB of it: what the first product writes the second one then
+// reads from the last-level cache.
+namespace {
+struct MoPlan {
+    Plan c[2];           // coefficient packing of C1 and C2
+    bool rows_first;     // C1 first (Y = C1^T B_P, then Y C2), or C2 first (X = B_P C2, then C1^T X)
+    int64_t step;        // P per block
+    size_t off_c[2], off_t, total;
+};
+constexpr size_t kMoBlockBytes = size_t(64) << 20;
+int mo_plan(const f2jk_ctx* ctx, int64_t n1, int64_t n2, MoPlan& m) {
+    const int64_t n[2] = {n1, n2};
+    size_t off = 0;
+    for (int i = 0; i < 2; ++i) {
+        Plan& p = m.c[i];
+        int rc = make_plan(ctx, 1, &n[i], F2JK_PREC_FP64, F2JK_WANT_K, false, p);
+        if (rc) return rc;
+        // only the packed coefficients of the plan are used
+        m.off_c[i] = off;
+        off += p.off_x;
+    }
+    const int64_t N = m.c[0].N, Q = m.c[0].Q;
+    m.rows_first = n1 < n2;  // the narrow set first: fewer products
+    const int64_t per_p = 8 * N * std::min(n1, n2);
+    m.step = std::max<int64_t>(1, std::min<int64_t>({Q, (int64_t)kMoBlockBytes / per_p, INT32_MAX / std::max(N, std::max(n1, n2))}));
+    m.off_t = off;
+    off += align_up((size_t)(m.step * per_p));
+    m.total = off;
+    return F2JK_OK;
+}
+}  // namespace
+
+int f2jk_mo_block_workspace_size(const f2jk_ctx* ctx, int64_t n1, int64_t n2, size_t* bytes) {
+    if (!ctx || !bytes) return fail(F2JK_EINVAL, "null argument");
+    if (n1 < 1 || n2 < 1) return fail(F2JK_EINVAL, "n1 and n2 must be >= 1");
+    MoPlan m;
+    int rc = mo_plan(ctx, n1, n2, m);
+    if (rc) return rc;
+    *bytes = m.total;
+    return F2JK_OK;
+}
+
+int f2jk_mo_block(f2jk_ctx* ctx, const double* C1, int64_t n1, int64_t ld1, const double* C2, int64_t n2, int64_t ld2,
+                  double* out, void* ws, size_t ws_bytes, void* stream) {
+    if (!ctx) return fail(F2JK_EINVAL, "null context");
+    if (!C1 || !C2 || !out) return fail(F2JK_EINVAL, "C1, C2 and out are required");
+    if (n1 < 1 || n2 < 1 || ld1 < n1 || ld2 < n2) return fail(F2JK_EINVAL, "n1, n2, ld1 or ld2 invalid");
+    MoPlan m;
+    int rc = mo_plan(ctx, n1, n2, m);
+    if (rc) return rc;
+    if (!ws) return fail(F2JK_EINVAL, "workspace pointer is NULL");
+    if (ws_bytes < m.total) return fail(F2JK_ENOMEM, "workspace too small");
+    if (((uintptr_t)ws) % 256) return fail(F2JK_EINVAL, "workspace must be 256-byte aligned");
+    F2JK_HIP(hipSetDevice(ctx->device));
+    hipStream_t st = (hipStream_t)stream;
+    const double* C[2] = {C1, C2};
+    const int64_t n[2] = {n1, n2}, ld[2] = {ld1, ld2};
+    const double* cq[2];
+    for (int i = 0; i < 2; ++i) {
+        char* w = (char*)ws + m.off_c[i];
+        if ((rc = pack_c(ctx, m.c[i], &C[i], &n[i], &ld[i], w, st, false))) return rc;
+        cq[i] = (const double*)(w + m.c[i].off_cq);
+    }
+    const Plan &p1 = m.c[0], &p2 = m.c[1];
+    const double* B = (const double*)ctx->B[F2JK_F64];
+    double* T = (double*)((char*)ws + m.off_t);
+    const int N = p1.N;
+    const int64_t NN = (int64_t)N * N;
+    for (int64_t P0 = 0; P0 < p1.Q; P0 += m.step) {
+        const int64_t nP = std::min<int64_t>(m.step, p1.Q - P0);
+        double* o = out + P0 * n1 * n2;
+        if (m.rows_first) {
+            launch_kxt(p1.dnb, B + P0 * NN, NN, N, N, N, nP, cq[0], p1.dnks, T, (int)n1, p1.dncolt, st);
+            F2JK_LAUNCHED("kxt");
+            launch_kxd(p2, T, nP * n1, cq[1], o, n2, (int)n2, KxdGamma{}, st);
+            F2JK_LAUNCHED("kx");
+        } else {
+            launch_kxd(p2, B + P0 * NN, nP * N, cq[1], T, n2, (int)n2, KxdGamma{}, st);
+            F2JK_LAUNCHED("kx");
+            launch_kxt(p1.dnb, T, N * n2, (int)n2, N, (int)n2, nP, cq[0], p1.dnks, o, (int)n1, p1.dncolt, st);
+            F2JK_LAUNCHED("kxt");
+        }
     }
     g_last_error.clear();
     return F2JK_OK;

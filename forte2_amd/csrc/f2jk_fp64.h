@@ -268,6 +268,126 @@ __global__ __launch_bounds__(256, 2) void kxd_kernel(const double* __restrict__ 
                      blockIdx.x, gridDim.x);
 }
 
+// ---------------------------------------------------------------------------
+// Transform of the row index: Y[P][i][n] = sum_k C[k][i] M[P][k][n], i < ni,
+// n < ncol, for matrices M[P] of K rows with row stride ld: the half-transform
+// with the operands exchanged (the coefficients of the same LDS tiles as A,
+// M's rows as B, 16 consecutive n of a row per lane group), so the sum runs
+// over M's rows and Y comes out with n contiguous, ready to be the A of
+// kxd_kernel.  A wave holds IB blocks of 16 n for all NB * 16 rows i of the
+// tile.
+// ---------------------------------------------------------------------------
+template <int NB, int IB>
+__global__ __launch_bounds__(256, 2) void kxt_kernel(const double* __restrict__ M, int64_t pstride, int ld, int K,
+                                                     int ncol, int64_t nblocks, const double* __restrict__ Cq, int nks,
+                                                     double* __restrict__ Y, int ni, int ncolt) {
+    __shared__ __attribute__((aligned(16))) char lds[kDKxLds(NB)];
+    constexpr int STAGE = NB * 2048;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t = xcd_remap(blockIdx.x, gridDim.x);
+    const int ct = t % ncolt;
+    const int64_t q0 = ((int64_t)(t / ncolt) * 4 + wid) * IB;  // first block of the wave
+    const int nblk = (ncol + 15) / 16;                         // blocks per P
+    const int lr = lane & 15, lg = lane >> 4;
+
+    const double* mp[IB];
+    int64_t P[IB];
+    int n[IB];
+#pragma unroll
+    for (int i = 0; i < IB; ++i) {
+        const int64_t q = q0 + i < nblocks ? q0 + i : nblocks - 1;  // past the end: computed, never stored
+        P[i] = q / nblk;
+        n[i] = (int)(q - P[i] * nblk) * 16 + lr;
+        mp[i] = M + P[i] * pstride + (int64_t)(2 * lg) * ld + (n[i] < ncol ? n[i] : ncol - 1);
+    }
+    dx2 an[IB][2];
+    auto load_m = [&](int s) {
+        if ((s + 1) * kDK <= K) {
+#pragma unroll
+            for (int i = 0; i < IB; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const double* p = mp[i] + (int64_t)(s * kDK + 8 * h) * ld;
+                    an[i][h].x = p[0];
+                    an[i][h].y = p[ld];
+                }
+        } else {  // the last step of a K that is not a multiple of 16: zeros past K
+#pragma unroll
+            for (int i = 0; i < IB; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int k = s * kDK + 8 * h + 2 * lg;
+                    const double* p = mp[i] + (int64_t)(s * kDK + 8 * h) * ld;
+                    an[i][h].x = k < K ? p[0] : 0.0;
+                    an[i][h].y = k + 1 < K ? p[ld] : 0.0;
+                }
+        }
+    };
+    const double* Ct = uniform_ptr(Cq + (int64_t)ct * nks * (NB * 256));
+    auto load_c = [&](int s, int stg) {
+        const double* base = Ct + (int64_t)s * (NB * 256);
+        const uint32_t l0 = lds_addr(lds) + stg * STAGE;
+        static_for<0, (2 * NB + 3) / 4>([&](auto Q) {
+            const int q = wid + 4 * decltype(Q)::value;
+            if (q < 2 * NB) lds_load16(base + q * 128, (uint32_t)lane * 16, l0 + q * 1024);
+        });
+    };
+    dx4 acc[IB][NB];
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = dx4{0, 0, 0, 0};
+    load_c(0, 0);
+    load_m(0);
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) asm volatile("" : "+v"(an[i][h]));
+    drain_and_barrier();
+    for (int s = 0; s < nks; ++s) {
+        const int cur = s & 1;
+        dx2 a[IB][2];
+#pragma unroll
+        for (int i = 0; i < IB; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) a[i][h] = an[i][h];
+        if (s + 1 < nks) {
+            load_c(s + 1, cur ^ 1);
+            load_m(s + 1);
+        }
+        const char* st = lds + cur * STAGE + lane * 16;
+        constexpr int NG = 2 * NB, AHEAD = NG > 3 ? 3 : NG - 1;
+        dx2 c[4];
+        auto frag = [&](auto G) {
+            constexpr int g = decltype(G)::value;
+            c[g & 3] = *reinterpret_cast<const dx2*>(st + (2 * (g % NB) + g / NB) * 1024);
+        };
+        static_for<0, AHEAD>(frag);
+        static_for<0, NG>([&](auto G) {
+            constexpr int g = decltype(G)::value, h = g / NB, j = g % NB;
+            if constexpr (g + AHEAD < NG) frag(std::integral_constant<int, g + AHEAD>{});
+#pragma unroll
+            for (int i = 0; i < IB; ++i) acc[i][j] = mfma4(c[g & 3].x, a[i][h].x, acc[i][j]);
+#pragma unroll
+            for (int i = 0; i < IB; ++i) acc[i][j] = mfma4(c[g & 3].y, a[i][h].y, acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        drain_and_barrier();
+    }
+#pragma unroll
+    for (int i = 0; i < IB; ++i) {
+        if (q0 + i >= nblocks || n[i] >= ncol) continue;
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = (ct * NB + j) * 16 + acc_row<double>(lane, r);
+                if (row < ni) Y[(P[i] * ni + row) * ncol + n[i]] = acc[i][j][r];
+            }
+    }
+}
+
 // gamma[d][P] = sum over column tiles and rows m of grow[ct * nd + d][P * N + m], one wave per (d, P)
 __device__ __forceinline__ void gamma_rows_body(const double* __restrict__ grow, int64_t gstride, int nd, int ncolt,
                                                 int N, int pc, double* __restrict__ gamma, int Q, int64_t t) {

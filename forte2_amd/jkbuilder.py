@@ -401,19 +401,30 @@ class FockBuilder:
 
     def B_tensor_gen_block(self, C1, C2):
         """B[P, i, j] = sum_mn B_Pmn C1_mi C2_nj: the MO-basis B tensor
-        (jkbuilder.py:521-552).  X = B C2 on MFMA, then C1^T X as a batched
-        GEMM, by blocks of P.  Real orbitals (conj is the identity)."""
+        (jkbuilder.py:521-552), both contractions on MFMA (f2jk_mo_block), the
+        narrower set first.  Real orbitals (conj is the identity)."""
         self.B_Pmn
         c1, to_np = self._as_dev(C1)
         c2, to_np2 = self._as_dev(C2)
         if c1.dim() != 2 or c2.dim() != 2 or c1.shape[0] != self.nbf or c2.shape[0] != self.nbf:
             raise ValueError(f"C1 and C2 must have {self.nbf} rows")
-        out = torch.empty((self.naux, c1.shape[1], c2.shape[1]), dtype=torch.float64, device=self.device)
-        if out.numel() == 0:
+        if c1.shape[1] > self.nbf:  # the kernels take at most nbf columns at a time
+            out = torch.cat([self.B_tensor_gen_block(c1[:, i:i + self.nbf], c2)
+                             for i in range(0, c1.shape[1], self.nbf)], 1)
             return out.cpu().numpy() if (to_np or to_np2) else out
-        c1t = c1.T.contiguous()
-        for P0, P1, X in self._x_blocks(c2):
-            out[P0:P1] = torch.matmul(c1t, X)
+        out = torch.empty((self.naux, c1.shape[1], c2.shape[1]), dtype=torch.float64, device=self.device)
+        if out.numel():
+            lib = nat.jk_lib()
+            c1, ld1 = self._rowmajor(c1)
+            c2, ld2 = self._rowmajor(c2)
+            n1, n2 = int(c1.shape[1]), int(c2.shape[1])
+            nbytes = ctypes.c_size_t()
+            nat.jk_check(lib.f2jk_mo_block_workspace_size(self.ctx, n1, n2, ctypes.byref(nbytes)), "workspace")
+            ws = self._workspace(nbytes.value)
+            nat.jk_check(lib.f2jk_mo_block(self.ctx, ctypes.c_void_p(c1.data_ptr()), n1, ld1,
+                                           ctypes.c_void_p(c2.data_ptr()), n2, ld2, ctypes.c_void_p(out.data_ptr()),
+                                           ctypes.c_void_p(ws.data_ptr()), ws.numel(), self._stream()),
+                         "f2jk_mo_block")
         return out.cpu().numpy() if (to_np or to_np2) else out
 
     def two_electron_integrals_gen_block(self, C1, C2, C3, C4):

@@ -216,13 +216,20 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens,
 /* Half-transform X[P-p0][m][i] = sum_n B[P][m][n] C[n][i] for p0 <= P < p1,
  * i < ncol, into the caller's X ((p1-p0)*nbf rows, row stride ldx), FP64.  The first step of
  * FockBuilder.B_tensor_gen_block (forte2/jkbuilder/jkbuilder.py:521-552),
- * whose einsum "Pmn,mi,nj->Pij" is finished by a GEMM with C1 on the caller's
- * side; two_electron_integrals_gen_block (:382-420) contracts two such blocks
+ * whose einsum "Pmn,mi,nj->Pij" f2jk_mo_block computes whole; two_electron_integrals_gen_block (:382-420) contracts two such blocks
  * over P.  Workspace: f2jk_workspace_size(ctx, 1, &ncol, FP64, F2JK_WANT_K).  With ldx equal
  * to ncol rounded up to 16 the kernel writes X in place (no copy). */
 int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ldc, int64_t p0,
                         int64_t p1, double* X, int64_t ldx, int precision, void* ws, size_t ws_bytes,
                         void* stream);
+
+/* MO-basis block out[P][i][j] = sum_mn B[P][m][n] C1[m][i] C2[n][j] for every
+ * P (naux x n1 x n2, dense), FP64: FockBuilder.B_tensor_gen_block
+ * (forte2/jkbuilder/jkbuilder.py:521-552).  The narrower of the two sets is
+ * contracted first.  Workspace: f2jk_mo_block_workspace_size. */
+int f2jk_mo_block_workspace_size(const f2jk_ctx* ctx, int64_t n1, int64_t n2, size_t* bytes);
+int f2jk_mo_block(f2jk_ctx* ctx, const double* C1, int64_t n1, int64_t ld1, const double* C2,
+                  int64_t n2, int64_t ld2, double* out, void* ws, size_t ws_bytes, void* stream);
 
 /* Message of the last failure on this thread ("" if none). */
 const char* f2jk_last_error(void);
