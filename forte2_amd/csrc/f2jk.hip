@@ -1131,11 +1131,16 @@ int group_plan(f2jk_ctx* const* ctxs, int njobs, const int* ndens, const int64_t
 
 template <int PH, int PREC, int NBW = 2, int VA = 2>
 int launch_group_phase(const GArgs& a, hipStream_t st) {
-    long long total = 0;
-    for (int j = 0; j < a.njobs; ++j) total += phase_blocks<PREC>(a.job[j], PH);
+    GArgs b = a;
+    int total = 0;
+    for (int j = 0; j < a.njobs; ++j) {
+        b.first[j] = total;
+        total += phase_blocks<PREC>(a.job[j], PH);
+    }
+    for (int j = a.njobs; j <= kMaxGroup; ++j) b.first[j] = total;
     if (total == 0) return F2JK_OK;
-    const unsigned grid = (unsigned)std::min<long long>(total, 4096);
-    hipLaunchKernelGGL((grouped_kernel<PH, PREC, NBW, VA>), dim3(grid), dim3(256), 0, st, a);
+    const unsigned grid = (unsigned)std::min(total, 4096);
+    hipLaunchKernelGGL((grouped_kernel<PH, PREC, NBW, VA>), dim3(grid), dim3(256), 0, st, b);
     F2JK_LAUNCHED("grouped phase " + std::to_string(PH));
     return F2JK_OK;
 }
@@ -1153,8 +1158,10 @@ int launch_group_kx_bf16(const GArgs& a, int nbw, hipStream_t st) {
     }
 }
 
+// `beside`: the second J pass of an FP64 group runs on the side stream, beside
+// the contraction (see kOverlapBytes); the caller joins it
 template <int PREC>
-int run_group(f2jk_ctx* ctx, const GArgs& a, int nbw, int va, hipStream_t st) {
+int run_group(f2jk_ctx* ctx, const GArgs& a, int nbw, int va, hipStream_t st, bool beside) {
     int rc;
     constexpr bool gamma_x = PREC == F2JK_PREC_FP64;  // gamma comes with the half-transform
     TIM(F2JK_PH_PREP, true);
@@ -1168,6 +1175,10 @@ int run_group(f2jk_ctx* ctx, const GArgs& a, int nbw, int va, hipStream_t st) {
     if constexpr (PREC == F2JK_PREC_BF16X3) {
         rc = (va == 4) ? launch_group_kx_bf16<4>(a, nbw, st) : launch_group_kx_bf16<2>(a, nbw, st);
         if (rc) return rc;
+    } else if constexpr (PREC == F2JK_PREC_FP64) {
+        rc = nbw <= kGroupNarrowNB ? launch_group_phase<GP_KX, PREC, kGroupNarrowNB>(a, st)
+                                   : launch_group_phase<GP_KX, PREC, kDMaxNB>(a, st);
+        if (rc) return rc;
     } else {
         if ((rc = launch_group_phase<GP_KX, PREC>(a, st))) return rc;
     }
@@ -1177,9 +1188,16 @@ int run_group(f2jk_ctx* ctx, const GArgs& a, int nbw, int va, hipStream_t st) {
         if ((rc = launch_group_phase<GP_GAMMA, PREC>(a, st))) return rc;
     if ((rc = launch_group_phase<GP_GRED, PREC>(a, st))) return rc;
     TIM(F2JK_PH_JGAMMA, false);
+    hipStream_t sj = st;
+    if (beside) {
+        std::lock_guard<std::mutex> lock(ctx->ev_mu);
+        F2JK_HIP(hipEventRecord(ctx->ev_fork, st));
+        F2JK_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
+        sj = ctx->side;
+    }
     TIM(F2JK_PH_JACC, true);
-    if ((rc = launch_group_phase<GP_JACC, PREC>(a, st))) return rc;
-    if ((rc = launch_group_phase<GP_JRED, PREC>(a, st))) return rc;
+    if ((rc = launch_group_phase<GP_JACC, PREC>(a, sj))) return rc;
+    if ((rc = launch_group_phase<GP_JRED, PREC>(a, sj))) return rc;
     TIM(F2JK_PH_JACC, false);
     TIM(F2JK_PH_KS, true);
     if ((rc = launch_group_phase<GP_KS, PREC>(a, st))) return rc;
@@ -1459,10 +1477,11 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
     if (want_j && !J) return fail(F2JK_EINVAL, "null argument");
     F2JK_HIP(hipSetDevice(ctxs[0]->device));
     hipStream_t st = (hipStream_t)stream;
-    // the group's BF16x3 tile width (widest job) and load width (4 when every nbf allows it)
-    int nbw = 2, va = 4;
+    // the group's tile width (widest job; FP64: column blocks) and the BF16x3 load
+    // width (4 when every nbf allows it)
+    int nbw = precision == F2JK_PREC_FP64 ? 1 : 2, va = 4;
     for (int j = 0; j < njobs; ++j) {
-        nbw = std::max(nbw, plans[j].nbw);
+        nbw = std::max(nbw, precision == F2JK_PREC_FP64 ? plans[j].dnb : plans[j].nbw);
         if (plans[j].N % 4) va = 2;
     }
     std::vector<GJob> jobs(njobs);
@@ -1483,6 +1502,7 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
         g.dncolt = p.dncolt;
         g.dnks = p.dnks;
         g.dt = p.dt;
+        g.drows = 64 * (nbw <= kGroupNarrowNB ? 1 : kxd_ib(std::max(1, p.dnb)));
         if (precision == F2JK_PREC_BF16X3) {
             g.Cth = (u16*)(w + p.off_cth);
             g.Ctl = (u16*)(w + p.off_ctl);
@@ -1526,22 +1546,37 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
         if (p.nlower != (int)(cdiv(p.N, kTile) * (cdiv(p.N, kTile) + 1) / 2))
             return fail(F2JK_EINVAL, "inconsistent tile plan");
     }
+    // the longest jobs first: a launch starts its blocks in this order and ends
+    // with short ones
+    std::stable_sort(jobs.begin(), jobs.end(), [](const GJob& x, const GJob& y) {
+        return (double)x.Q * x.N * x.N * x.OPAD > (double)y.Q * y.N * y.N * y.OPAD;
+    });
     f2jk_ctx* ctx = ctxs[0];  // timing events of the group
     tim_begin(ctx, flags & F2JK_TIMING);
     TIM(F2JK_PH_TOTAL, true);
+    double jbytes = 0.0;
+    for (const Plan& p : plans) jbytes += j_pass_bytes(p);
+    const bool beside = want_j && precision == F2JK_PREC_FP64 && !ctx->timing &&
+                        (ctx->overlap_jk < 0 ? jbytes >= kOverlapBytes : ctx->overlap_jk == 1);
     for (int j0 = 0; j0 < njobs; j0 += kMaxGroup) {
         GArgs a;
         std::memset(&a, 0, sizeof(a));
         a.njobs = std::min(kMaxGroup, njobs - j0);
         for (int j = 0; j < a.njobs; ++j) a.job[j] = jobs[j0 + j];
         if (precision == F2JK_PREC_FP64)
-            rc = run_group<F2JK_PREC_FP64>(ctx, a, nbw, va, st);
+            rc = run_group<F2JK_PREC_FP64>(ctx, a, nbw, va, st, beside);
         else if (precision == F2JK_PREC_FP32)
-            rc = run_group<F2JK_PREC_FP32>(ctx, a, nbw, va, st);
+            rc = run_group<F2JK_PREC_FP32>(ctx, a, nbw, va, st, false);
         else
-            rc = run_group<F2JK_PREC_BF16X3>(ctx, a, nbw, va, st);
-        if (rc) return rc;
+            rc = run_group<F2JK_PREC_BF16X3>(ctx, a, nbw, va, st, false);
+        if (rc) break;
     }
+    if (beside) {  // also after a failed launch: later work comes after the side stream's
+        std::lock_guard<std::mutex> lock(ctx->ev_mu);
+        F2JK_HIP(hipEventRecord(ctx->ev_join, ctx->side));
+        F2JK_HIP(hipStreamWaitEvent(st, ctx->ev_join, 0));
+    }
+    if (rc) return rc;
     TIM(F2JK_PH_TOTAL, false);
     g_last_error.clear();
     return F2JK_OK;

@@ -68,6 +68,16 @@ __device__ __forceinline__ const T* uniform_ptr(const T* p) {
 struct DCols {
     int nd;
     int nocc[kDMaxDens], width[kDMaxDens], ioff[kDMaxDens];
+    __device__ __forceinline__ int count() const { return nd; }
+    __device__ __forceinline__ int first(int d) const { return ioff[d]; }
+    __device__ __forceinline__ int end(int d) const { return ioff[d] + width[d]; }
+};
+// the same of one or two densities, in registers
+struct DCols2 {
+    int nd, ioff0, end0, ioff1, end1;
+    __device__ __forceinline__ int count() const { return nd; }
+    __device__ __forceinline__ int first(int d) const { return d ? ioff1 : ioff0; }
+    __device__ __forceinline__ int end(int d) const { return d ? end1 : end0; }
 };
 
 // ---------------------------------------------------------------------------
@@ -114,12 +124,12 @@ __global__ void pack_cq_kernel(DCoef cs, DCols dc, int N, int ldcp, int nb, int 
 // the first J pass without another read of B and without D.  A row's sum does
 // not depend on how rows are cut into tiles or P into chunks.
 // ---------------------------------------------------------------------------
-template <int NB, int IB>
+template <int NB, int IB, typename Cols>
 __device__ __forceinline__ void kxd_body(char* lds, const double* __restrict__ A, int64_t R, int K,
                                          const double* __restrict__ Cq, int nks, double* __restrict__ X,
-                                         int64_t ldx, int ncol, int ncolt, const double* __restrict__ Cp, int nd,
-                                         const int* ioff, const int* width, double* __restrict__ grow,
-                                         int64_t gstride, int b, int nblocks) {
+                                         int64_t ldx, int ncol, int ncolt, const double* __restrict__ Cp,
+                                         const Cols& dc, double* __restrict__ grow, int64_t gstride, int b,
+                                         int nblocks) {
     constexpr int STAGE = NB * 2048;  // bytes
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -227,9 +237,9 @@ __device__ __forceinline__ void kxd_body(char* lds, const double* __restrict__ A
             }
         }
     if (!grow) return;
-    const int ldcp = ncolt * NB * 16;
+    const int ldcp = ncolt * NB * 16, nd = dc.count();
     auto row_sums = [&](int d, auto masked) {
-        const int lo = ioff[d], hi = lo + width[d];
+        const int lo = dc.first(d), hi = dc.end(d);
         double* gr = grow + (int64_t)(ct * nd + d) * gstride;
 #pragma unroll
         for (int i = 0; i < IB; ++i)
@@ -264,7 +274,7 @@ __global__ __launch_bounds__(256, 2) void kxd_kernel(const double* __restrict__ 
                                                      int64_t ldx, int ncol, int ncolt, const double* __restrict__ Cp,
                                                      DCols dc, double* __restrict__ grow, int64_t gstride) {
     __shared__ __attribute__((aligned(16))) char lds[kDKxLds(NB)];
-    kxd_body<NB, IB>(lds, A, R, K, Cq, nks, X, ldx, ncol, ncolt, Cp, dc.nd, dc.ioff, dc.width, grow, gstride,
+    kxd_body<NB, IB>(lds, A, R, K, Cq, nks, X, ldx, ncol, ncolt, Cp, dc, grow, gstride,
                      blockIdx.x, gridDim.x);
 }
 

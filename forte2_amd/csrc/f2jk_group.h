@@ -2,8 +2,8 @@
 //
 // One persistent launch per phase covers the blocks of every job in the
 // group.  A block walks the concatenated block index space with a stride of
-// gridDim.x, finds its job from the per-phase block counts (a short uniform
-// scan, at most kMaxGroup jobs) and runs the same device body as the
+// gridDim.x, finds its job from the launch's table of first blocks (a short
+// uniform scan, at most kMaxGroup jobs) and runs the same device body as the
 // single-job kernels with the job's own plan.  The decomposition of a job
 // (element groups, P chunks, K splits) is its own plan, independent of the
 // other jobs; the tile width of the BF16x3 half-transform is the group's
@@ -59,13 +59,14 @@ struct GJob {
     int N, Q, nd, nocc[2], width[2], ioff[2], OPAD, KP;
     int nvec, neg, npc1, npc2, ppw2;
     int nlower, nsplit, ncolt;
-    int dnb, dncolt, dnks;  // FP64 half-transform
+    int dnb, dncolt, dnks, drows;  // FP64 half-transform; rows of a workgroup
     DTiles dt;              // FP64 contraction
     int want_j;
 };
 
 struct GArgs {
     int njobs;
+    int first[kMaxGroup + 1];  // first block of each job in the launch's phase, then the total
     GJob job[kMaxGroup];
 };
 static_assert(sizeof(GArgs) <= 4096, "the job table must fit the kernel argument limit");
@@ -87,7 +88,7 @@ __host__ __device__ inline int phase_blocks(const GJob& g, int phase) {
         case GP_JACC: return j * g.neg * g.npc2;
         case GP_JRED: return j * gcdiv(g.nvec, kJRedElems);
         case GP_KX:
-            if (PREC == F2JK_PREC_FP64) return gcdiv((long long)g.Q * g.N, 64 * kxd_ib(g.dnb)) * g.dncolt;
+            if (PREC == F2JK_PREC_FP64) return gcdiv((long long)g.Q * g.N, g.drows) * g.dncolt;
             return gcdiv((long long)g.Q * g.N, kTile) * g.ncolt;
         case GP_KS: return (PREC == F2JK_PREC_FP64 ? g.dt.total : g.nlower * g.nsplit) * g.nd;
         case GP_KRED: return k_reduce_blocks(g.N) * g.nd;
@@ -95,39 +96,46 @@ __host__ __device__ inline int phase_blocks(const GJob& g, int phase) {
     return 0;
 }
 
-// the FP64 half-transform of one job: the kernel of its width
-template <int NB = 1>
-__device__ __forceinline__ void grouped_kxd(char* lds, const GJob& g, int b, int nblocks) {
-    if constexpr (NB <= kDMaxNB) {
-        if (g.dnb == NB)
-            kxd_body<NB, kxd_ib(NB)>(lds, (const double*)g.B, (long long)g.Q * g.N, g.N, g.Cq, g.dnks, (double*)g.X,
-                                     g.OPAD, g.OPAD, g.dncolt, g.Cp, g.nd, g.ioff, g.width,
-                                     g.want_j ? g.grow : nullptr, (long long)g.Q * g.N, b, nblocks);
+// the FP64 half-transform of one job: the body of its width.  The job's fields
+// are read once, before the choice: with a use in every body the compiler
+// would copy the whole job table to scratch memory.
+struct GKxd {
+    const double *B, *Cq, *Cp;
+    double *X, *grow;
+    int64_t R;
+    int N, nks, OPAD, ncolt;
+    DCols2 dc;
+};
+// MAXNB 8: narrow jobs only, one row block per wave (114 registers and 32 KB
+// of LDS: four workgroups per CU); 20: every width (256 registers, two).
+constexpr int kGroupNarrowNB = 8;
+constexpr int grouped_kxd_ib(int maxnb, int nb) { return maxnb == kGroupNarrowNB ? 1 : kxd_ib(nb); }
+template <int MAXNB, int NB = 1>
+__device__ __forceinline__ void grouped_kxd(char* lds, int nb, const GKxd& k, int b, int nblocks) {
+    if constexpr (NB <= MAXNB) {
+        if (nb == NB)
+            kxd_body<NB, grouped_kxd_ib(MAXNB, NB)>(lds, k.B, k.R, k.N, k.Cq, k.nks, k.X, k.OPAD, k.OPAD, k.ncolt, k.Cp, k.dc, k.grow,
+                                     k.R, b, nblocks);
         else
-            grouped_kxd<NB + 1>(lds, g, b, nblocks);
+            grouped_kxd<MAXNB, NB + 1>(lds, nb, k, b, nblocks);
     }
 }
 
 // PREC: the group's precision; NBW, VA: tile width and load width of the
-// BF16x3 half-transform (unused otherwise).
+// BF16x3 half-transform; NBW of the FP64 one: its widest column tile, in blocks.
 template <int PHASE, int PREC, int NBW = 2, int VA = 2>
-__global__ __launch_bounds__(256, PREC != F2JK_PREC_BF16X3 ? (PHASE == GP_KX || PHASE == GP_KS ? 2 : 1)
+__global__ __launch_bounds__(256, PREC == F2JK_PREC_FP64 && PHASE == GP_KX && NBW == kGroupNarrowNB ? 4
+                                  : PREC != F2JK_PREC_BF16X3 ? (PHASE == GP_KX || PHASE == GP_KS ? 2 : 1)
                                   : PHASE == GP_KX ? kx_bf16_waves_per_eu<NBW>()
                                   : PHASE == GP_KS ? 2 : 1)
 void grouped_kernel(const GArgs a) {
     using TB = typename std::conditional<PREC == F2JK_PREC_FP64, double, float>::type;
-    int total = 0;
-    for (int j = 0; j < a.njobs; ++j) total += phase_blocks<PREC>(a.job[j], PHASE);
+    const int total = a.first[a.njobs];
     for (int lb = blockIdx.x; lb < total; lb += gridDim.x) {
-        int j = 0, base = 0;
-        for (;;) {
-            const int nb = phase_blocks<PREC>(a.job[j], PHASE);
-            if (lb < base + nb) break;
-            base += nb;
-            ++j;
-        }
+        int j = 0;
+        while (lb >= a.first[j + 1]) ++j;
         const GJob& g = a.job[j];
-        const int local = lb - base;
+        const int local = lb - a.first[j], nblocks = a.first[j + 1] - a.first[j];
         const int tid = threadIdx.x;
         if constexpr (PHASE == GP_PAD) {
             const long long t = (long long)local * 256 + tid;
@@ -177,10 +185,10 @@ void grouped_kernel(const GArgs a) {
             const TB* B = (const TB*)g.B;
             if (g.nd == 2) {
                 DPtrs<2> dp{{g.D, g.D + NN}};
-                j_gamma_kernel_body<TB, 2, 4, 2>(B, g.N, g.Q, dp, g.N, g.rowoff, g.nvec, 32, g.gpart, bx, by);
+                j_gamma_kernel_body<TB, 2, 4, 2, true>(B, g.N, g.Q, dp, g.N, g.rowoff, g.nvec, 32, g.gpart, bx, by);
             } else {
                 DPtrs<1> dp{{g.D}};
-                j_gamma_kernel_body<TB, 2, 4, 1>(B, g.N, g.Q, dp, g.N, g.rowoff, g.nvec, 32, g.gpart, bx, by);
+                j_gamma_kernel_body<TB, 2, 4, 1, true>(B, g.N, g.Q, dp, g.N, g.rowoff, g.nvec, 32, g.gpart, bx, by);
             }
         } else if constexpr (PHASE == GP_GRED && PREC == F2JK_PREC_FP64) {
             gamma_rows_body(g.grow, (long long)g.Q * g.N, g.nd, g.dncolt, g.N, g.Q, g.gamma, g.Q,
@@ -197,9 +205,9 @@ void grouped_kernel(const GArgs a) {
             const int bx = local % g.neg, by = local / g.neg;
             const TB* B = (const TB*)g.B;
             if (g.nd == 2)
-                j_accum_kernel_body<TB, 2, 4, 2>(B, g.N, g.Q, g.gamma, g.rowoff, g.nvec, g.ppw2, g.jpart, bx, by);
+                j_accum_kernel_body<TB, 2, 4, 2, true>(B, g.N, g.Q, g.gamma, g.rowoff, g.nvec, g.ppw2, g.jpart, bx, by);
             else
-                j_accum_kernel_body<TB, 2, 4, 1>(B, g.N, g.Q, g.gamma, g.rowoff, g.nvec, g.ppw2, g.jpart, bx, by);
+                j_accum_kernel_body<TB, 2, 4, 1, true>(B, g.N, g.Q, g.gamma, g.rowoff, g.nvec, g.ppw2, g.jpart, bx, by);
         } else if constexpr (PHASE == GP_JRED) {
             if (g.nd == 2) {
                 JPtrs<2> jp{{g.J[0], g.J[1]}};
@@ -209,11 +217,14 @@ void grouped_kernel(const GArgs a) {
                 j_reduce_body<2, 1>(g.jpart, g.npc2, g.N, g.rowoff, nullptr, g.nvec, g.nvec, jp, local);
             }
         } else if constexpr (PHASE == GP_KX) {
-            const int nb = phase_blocks<PREC>(g, GP_KX);
+            const int nb = nblocks;
             const long long R = (long long)g.Q * g.N;
             if constexpr (PREC == F2JK_PREC_FP64) {
-                __shared__ __attribute__((aligned(16))) char lds[kDKxLds(kDMaxNB)];
-                grouped_kxd(lds, g, local, nb);
+                __shared__ __attribute__((aligned(16))) char lds[kDKxLds(NBW)];
+                const GKxd k{(const double*)g.B, g.Cq, g.Cp, (double*)g.X, g.want_j ? g.grow : nullptr, R, g.N, g.dnks,
+                             g.OPAD, g.dncolt,
+                             DCols2{g.nd, g.ioff[0], g.ioff[0] + g.width[0], g.ioff[1], g.ioff[1] + g.width[1]}};
+                grouped_kxd<NBW>(lds, g.dnb, k, local, nb);
             } else if constexpr (PREC == F2JK_PREC_FP32) {
                 kx_kernel_body<float, 2>((const float*)g.B, R, g.N, g.Cp32, g.OPAD, (float*)g.X, g.ncolt, local, nb);
             } else {
