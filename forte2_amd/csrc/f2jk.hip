@@ -468,27 +468,21 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         const int64_t wg_target = p.ks_tile == 256 ? target_blocks / 4 : target_blocks / 2;
         p.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(pc, wg_target / p.nlower));
         if (precision == F2JK_PREC_BF16X3) {
-            // single-job builds of large nbf run the tall (256-row) half-transform
+            // single-job builds run the tall (256-row) half-transform: build
+            // times with 128 and 256 rows at nbf 192 175 / 171 us, 288 381 / 369,
+            // 384 798 / 788, 576 2524 / 2437, 700 4379 / 4169, 960 12.5 / 11.1 ms
             p.kx_rows = 128;
-            if (!grouped) p.kx_rows = ctx->kx_rows ? ctx->kx_rows : (N >= 768 ? 256 : 128);
+            if (!grouped) p.kx_rows = ctx->kx_rows ? ctx->kx_rows : (N >= 192 ? 256 : 128);
             if (N % 4 || N < 32) p.kx_rows = 128;  // the tall kernel loads A rows 16 bytes at a time
             // the tile width (in 32-column units) within the cap that computes
-            // the fewest column blocks; ties go to the wider tile.  The tall
-            // kernel's 2 x 4 waves take even widths only.
+            // the fewest column blocks; ties go to the wider tile
             const int need = (int)cdiv(p.OPAD, 32);
             int best = 0, cost = 0;
-            for (int w : {10, 8, 6, 5, 4, 2}) {
-                if (w > ctx->bf16_nbw_max || (p.kx_rows == 256 && w % 2)) continue;
+            for (int w : {10, 8, 7, 6, 5, 4, 3, 2, 1}) {
+                if (w > ctx->bf16_nbw_max) continue;
+                if (p.kx_rows == 128 && (w == 7 || w == 3 || w == 1)) continue;
                 const int c = (int)cdiv(need, w) * w;
                 if (best == 0 || c < cost) best = w, cost = c;
-            }
-            if (best == 0) {  // a cap of 5 leaves no even width: the 128-row kernel
-                p.kx_rows = 128;
-                for (int w : {10, 8, 6, 5, 4, 2}) {
-                    if (w > ctx->bf16_nbw_max) continue;
-                    const int c = (int)cdiv(need, w) * w;
-                    if (best == 0 || c < cost) best = w, cost = c;
-                }
             }
             p.nbw = best;
             p.kx_waves = ctx->kx_waves;
@@ -872,12 +866,20 @@ void launch_kx_bf16(const Plan& p, unsigned grid, const float* A, int64_t R, con
     launch_kx_bf16_w<NBW, 4>(p, grid, A, R, th, tl, xh, xl, st);
 }
 
-// the tall (256-row, 2 x 4 waves) half-transform; even widths only
-template <int NBW>
+// The tall (256-row) half-transform: 2 x 4 waves at even widths (in 32-column
+// units), 4 x 2 at odd ones, which 2 x 4 cannot split.  Widths that fit the
+// job: at 224 columns (nbf 960) 7 units take 3.31 ms per chunk where 8 took
+// 3.44; 4 x 2 waves at 6 units took 5.12 ms where 2 x 4 take 5.02 (nbf 1188).
+// 9 units would spill.
+template <int NBW = 1>
 void launch_kx_bf16_tall(const Plan& p, unsigned grid, const float* A, int64_t R, const u16* th,
                          const u16* tl, u16* xh, u16* xl, hipStream_t st) {
-    hipLaunchKernelGGL((kx_bf16x3_tall_kernel<NBW, 2, 4>), dim3(grid), dim3(512), 0, st, A, R, p.N, p.KP, th, tl,
-                       p.OPAD, xh, xl, p.ncolt);
+    if constexpr (NBW <= 10) {
+        if (p.nbw != NBW) return launch_kx_bf16_tall<NBW == 8 ? 10 : NBW + 1>(p, grid, A, R, th, tl, xh, xl, st);
+        constexpr int WR = NBW % 2 ? 4 : 2;
+        hipLaunchKernelGGL((kx_bf16x3_tall_kernel<NBW, WR, 8 / WR>), dim3(grid), dim3(512), 0, st, A, R, p.N, p.KP, th,
+                           tl, p.OPAD, xh, xl, p.ncolt);
+    }
 }
 
 template <typename F>
@@ -898,13 +900,7 @@ int run_k_bf16x3(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipSt
         TIM(F2JK_PH_KX, true);
         if (p.kx_rows == 256) {
             const unsigned grid = (unsigned)(cdiv(R, kTallRows) * p.ncolt);
-            switch (p.nbw) {
-                case 2: launch_kx_bf16_tall<2>(p, grid, A, R, th, tl, xh, xl, st); break;
-                case 4: launch_kx_bf16_tall<4>(p, grid, A, R, th, tl, xh, xl, st); break;
-                case 6: launch_kx_bf16_tall<6>(p, grid, A, R, th, tl, xh, xl, st); break;
-                case 8: launch_kx_bf16_tall<8>(p, grid, A, R, th, tl, xh, xl, st); break;
-                default: launch_kx_bf16_tall<10>(p, grid, A, R, th, tl, xh, xl, st); break;
-            }
+            launch_kx_bf16_tall(p, grid, A, R, th, tl, xh, xl, st);
         } else {
         const unsigned grid = (unsigned)(cdiv(R, kTile) * p.ncolt);
         switch (p.nbw) {

@@ -1254,8 +1254,7 @@ __device__ __forceinline__ void kx_bf16x3_tall_body(
     static_assert(A_LD * T == TM * 8 && A_LD <= 15, "A tile must split evenly");
     // coefficient tile: 2 planes x BN rows x 4 chunks, in wave instructions of 16 rows
     constexpr int B_INS = 2 * BN / 16;
-    constexpr int B_LD = B_INS / NW;
-    static_assert(B_LD * NW == B_INS, "coefficient tile must split over the waves");
+    constexpr int B_LD = (B_INS + NW - 1) / NW;
     __shared__ __attribute__((aligned(16))) __bf16 Ah[2][TM][kBK16];
     __shared__ __attribute__((aligned(16))) __bf16 Al[2][TM][kBK16];
     __shared__ __attribute__((aligned(16))) __bf16 Bt[2][2][BN][kBK16];  // [stage][hi, lo][row][k]
@@ -1310,9 +1309,11 @@ __device__ __forceinline__ void kx_bf16x3_tall_body(
         static_for<0, B_LD>([&](auto Q) {
             constexpr int q = decltype(Q)::value;
             const int g = wid + NW * q;                // wave instruction index (wave-uniform)
-            const int plane = g / (BN / 16), grp = g % (BN / 16);
-            const u16* base = (plane ? Ctl : Cth) + (int64_t)(c0 + grp * 16) * KP + k0;
-            lds_load16(base, boff, lds_addr(&Bt[stg][plane][grp * 16][0]));
+            if (B_INS % NW == 0 || g < B_INS) {
+                const int plane = g / (BN / 16), grp = g % (BN / 16);
+                const u16* base = (plane ? Ctl : Cth) + (int64_t)(c0 + grp * 16) * KP + k0;
+                lds_load16(base, boff, __builtin_amdgcn_readfirstlane(lds_addr(&Bt[stg][plane][grp * 16][0])));
+            }
         });
     };
 
@@ -1654,12 +1655,16 @@ __device__ __forceinline__ void ks_bf16x3_dma_body(
     drain_and_barrier();
     const int fr = lane & 15, fc = lane >> 4;
     const int ra0 = wr * (TS / WR), rb0w = wc * (TS / WC);
+    // a wave whose block lies above the diagonal or past row N loads its share
+    // and multiplies nothing
+    const bool active = m0 + ra0 < N && n0 + rb0w <= m0 + ra0 + TS / WR - 1;
     int st = 0;
     for (int P = Pa; P < Pb; ++P) {
     for (int kt = 0; kt < nkp; ++kt, ++st) {
         const int cur = st & 1, nxt = cur ^ 1;
         const int sp = min(st + 1, nsteps - 1);  // clamped: the last loads are harmless repeats
         load(Pa + sp / nkp, (sp % nkp) * kBK16, nxt);
+        if (active) {
         bf16x8 ah[IB], al[IB], bh[2], bl[2];
         const int rb0 = rb0w + fr;
         bh[0] = *reinterpret_cast<const bf16x8*>(&Xt[cur][2][rb0][swz16(rb0, fc)]);
@@ -1686,9 +1691,11 @@ __device__ __forceinline__ void ks_bf16x3_dma_body(
             static_for<0, IB>([&](auto I) { acc[I][j] = mfma_bf16(ah[I], bh[j & 1], acc[I][j]); });
             __builtin_amdgcn_sched_barrier(0);
         });
+        }
         drain_and_barrier();
     }
     }
+    if (!active) return;
     double* Ks = Kpart + (int64_t)s * N * N;
 #pragma unroll
     for (int i = 0; i < IB; ++i)

@@ -107,9 +107,9 @@ int f2jk_get_shape(const f2jk_ctx* ctx, int64_t* naux, int64_t* nbf);
  * "kx_wide" (-1, 0, 1; default -1 = above 128 occupied columns) runs the
  * FP32 half-transform in 128 x 320 tiles (8 waves), which read each
  * row block of B once instead of once per 128-column tile (the same products,
- * bitwise); "kx_rows" (0, 128, 256; default 0 = 256 when nbf >= 768 and nbf % 4 == 0)
+ * bitwise); "kx_rows" (0, 128, 256; default 0 = 256 when nbf >= 192 and nbf % 4 == 0)
  * is the row count of a single-job BF16x3 half-transform tile (256: 8 waves,
- * even widths, coefficient tiles loaded straight into LDS); "ks_dma" (-1, 0,
+ * coefficient tiles loaded straight into LDS); "ks_dma" (-1, 0,
  * 1; default -1 = with 256-wide tiles) loads the BF16x3 contraction's X
  * tiles straight into LDS instead of staging them through registers (the same
  * products, bitwise); "j_sparse" (0/1, default 0): when 1, every registered B
