@@ -123,6 +123,7 @@ struct Plan {
     size_t per_p = 0;      // bytes of X per P
     DTiles dt{};           // FP64 contraction: tiles and their P splits
     bool gamma_x = false;  // gamma of J from the half-transform's row sums (FP64 J and K from C)
+    bool small = false;    // ... by the blocks of the second J pass, and both reductions in one launch
     int ctrows = 0;     // rows of the padded bf16 coefficient planes (>= ncolt * tile columns)
     // workspace offsets
     int KP = 0;                // nbf rounded up to the bf16 k step
@@ -287,7 +288,8 @@ struct KxdGamma {
 // diagonal tile took 2.1 times their share of blocks).  All workgroups at
 // once (512) is best when the shares round well; a tile count that does not
 // fit runs in more, shorter workgroups that even out over several rounds, at
-// ~5 us a round and the traffic of their partials.  The estimate below orders
+// ~5 us a round, the traffic of their partials and the reduction's chain of
+// loads (~0.03 us per split).  The estimate below orders
 // the measured times of nbf 318 (64.7 us at 512 workgroups, 71 at 1024, 85 at
 // 2048), 384 (491, 562, 529), 960 (6.2-7.1 ms, 5.6, 5.3, 4.9 at 4096) and 1152
 // (8.1-9.0 ms, 9.1, 8.6, 8.3).
@@ -304,7 +306,7 @@ DTiles dtile_plan(int N, int64_t Pc, int width, int slots) {
     double sum = 0;
     for (int k = 0; k < 4; ++k) sum += m.cnt[k] * cost[k];
     double best = -1;
-    for (int r : {1, 2, 4, 8})
+    for (double r : {0.25, 0.5, 1.0, 2.0, 4.0, 8.0})
         for (int i = 0; i < 4; ++i) {
             const double target = (double)slots * r * (1.0 - 0.04 * i);
             int ns[4], total = 0, G = 1;
@@ -322,14 +324,16 @@ DTiles dtile_plan(int N, int64_t Pc, int width, int slots) {
             const int rounds = (int)cdiv(total, slots);
             // one round ends with its longest workgroup; several fill in behind each other
             const double span = rounds == 1 ? longest : std::max(work, longest) + 0.6 * longest;
-            const double us = span * unit_us + 5.0 * rounds + (double)G * N * N * 8 / 8e6;
+            // up to one workgroup per CU has the matrix pipes to itself
+            const double us = span * unit_us * (total <= slots / 2 ? 0.55 : 1.0) + 5.0 * rounds +
+                              (double)G * N * N * 8 / 4e6 + 0.03 * G;
             if (best < 0 || us < best) {
                 best = us;
                 for (int k = 0; k < 4; ++k) m.ns[k] = ns[k];
                 m.G = G;
                 m.total = total;
             }
-            if ((int64_t)slots * r < 256) break;  // a small cap: no variants
+            if (slots < 256) break;  // a small cap: no variants
         }
     return m;
 }
@@ -428,6 +432,14 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         p.npc1 = (int)cdiv(Q, kJ1PerBlock);
         p.npc2 = (int)std::max<int64_t>(1, std::min<int64_t>(Q, cdiv(target_blocks, p.neg)));
         p.ppw2 = (int)cdiv(Q, p.npc2);
+        // FP64 builds of up to 8 element groups (nbf ~180) are bound by their
+        // launches: fewer of them, and (grouped too, for the same sums) no more
+        // partials than two rounds of the reduction's loads (64 chunks), as long
+        // as a block can form the gamma of its own P
+        if (p.gamma_x && p.neg <= 8 && ndens <= 2) {
+            p.ppw2 = std::max(p.ppw2, std::min<int>(kGBlock, (int)cdiv(Q, 64)));
+            p.small = !grouped && p.ppw2 <= kGBlock;
+        }
         p.npc2 = (int)cdiv(Q, p.ppw2);
         if (j_from_c && !p.gamma_x) {
             p.off_d = off;
@@ -502,6 +514,7 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         off += p.x_bytes;
         p.off_grow = off;
         off += align_up((size_t)p.Pc * grow_p);
+        if (p.nchunks > 1) p.small = false;  // the row sums of the last chunk only are there
         if (precision == F2JK_PREC_FP64) {
             p.dt = dtile_plan(N, pc, p.width[0], (int)std::min<int64_t>(kDSlots, target_blocks));
             p.nsplit = p.dt.G;  // partials held per density
@@ -569,6 +582,16 @@ int launch_j(f2jk_ctx* ctx, const Plan& p, const TB* B, int d0, const double* co
         TIM(F2JK_PH_JGAMMA, false);
     }
     TIM(F2JK_PH_JACC, true);
+    if constexpr (sizeof(TB) == 8 && VEC <= 2) {
+        if (p.small) {
+            hipLaunchKernelGGL((j_accum_rows_kernel<VEC, kEPT, ND>), dim3(p.neg, p.npc2), dim3(kJThreads), 0, st, B,
+                               p.N, p.Q, (const double*)(ws + p.off_grow), (int64_t)p.Pc * p.N, p.dncolt, rowoff, elist,
+                               p.nvec, p.ppw2, jpart);
+            F2JK_LAUNCHED("j_accum_rows");
+            TIM(F2JK_PH_JACC, false);
+            return F2JK_OK;  // reduced together with K
+        }
+    }
     hipLaunchKernelGGL((j_accum_kernel<TB, VEC, kEPT, ND, NT>), dim3(p.neg, p.npc2), dim3(kJThreads), 0,
                        st, B, p.N, p.Q, gamma, rowoff, elist, (const TB*)p.jpacked, p.nvec, p.ppw2, jpart);
     F2JK_LAUNCHED("j_accum");
@@ -769,10 +792,20 @@ void launch_kxt(int nb, const double* M, int64_t pstride, int ld, int K, int nco
     }
 }
 
+template <int VEC, int ND>
+void launch_jkred(const f2jk_ctx* ctx, const Plan& p, const double* jpart, double* const* J, const double* kpart,
+                  int64_t dstride, const KPtrs& kp, hipStream_t st) {
+    JPtrs<ND> jp;
+    for (int d = 0; d < ND; ++d) jp.p[d] = J[d];
+    const int nbj = (int)cdiv(p.jdense, kJRedElems);
+    hipLaunchKernelGGL((jkred_kernel<VEC, ND>), dim3(nbj + k_reduce_blocks(p.N) * ND), dim3(256), 0, st, jpart, p.npc2,
+                       p.N, ctx->rowoff[VEC], p.jinv, p.nvec, p.jdense, jp, nbj, kpart, dstride, p.dt, kp);
+}
+
 // `after_kx` runs once the last chunk's half-transform (and gamma) is queued
 template <typename T, typename F>
-int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const* K, char* ws, hipStream_t st,
-                F&& after_kx) {
+int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const* J, double* const* K, char* ws,
+                hipStream_t st, F&& after_kx) {
     const T* B = (const T*)ctx->B[sizeof(T) == 8 ? F2JK_F64 : F2JK_F32];
     const T* cp = (sizeof(T) == 8) ? (const T*)(ws + p.off_cp) : (const T*)(ws + p.off_cp32);
     T* X = (T*)(ws + p.off_x);
@@ -798,7 +831,7 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const
             launch_kx_fp32(p, (unsigned)(nrowt * p.ncolt), A, R, cp, X, st);
         F2JK_LAUNCHED("kx");
         TIM(F2JK_PH_KX, false);
-        if (p.gamma_x) {
+        if (p.gamma_x && !p.small) {
             TIM(F2JK_PH_JGAMMA, true);
             hipLaunchKernelGGL(gamma_rows_kernel, dim3((unsigned)cdiv((int64_t)p.nd * pc, 4)), dim3(256), 0, st,
                                (const double*)(ws + p.off_grow), (int64_t)p.Pc * p.N, p.nd, p.dncolt, p.N, pc,
@@ -830,10 +863,17 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const
     const int nsplit_used = std::min(p.nsplit, std::min(p.Pc, p.Q));
     KPtrs kp{};
     for (int d = 0; d < p.nd; ++d) kp.p[d] = K[d];
-    if constexpr (sizeof(T) == 8)
-        hipLaunchKernelGGL(kred_kernel, dim3(k_reduce_blocks(p.N), p.nd), dim3(256), 0, st, kpart,
-                           (int64_t)p.nsplit * NN, p.dt, p.N, kp);
-    else
+    if constexpr (sizeof(T) == 8) {
+        if (p.small) {
+            const bool v2 = p.jvec == 2;
+            const auto red = p.nd == 2 ? (v2 ? launch_jkred<2, 2> : launch_jkred<1, 2>)
+                                       : (v2 ? launch_jkred<2, 1> : launch_jkred<1, 1>);
+            red(ctx, p, (const double*)(ws + p.off_jpart), J, kpart, (int64_t)p.nsplit * NN, kp, st);
+        } else {
+            hipLaunchKernelGGL(kred_kernel, dim3(k_reduce_blocks(p.N), p.nd), dim3(256), 0, st, kpart,
+                               (int64_t)p.nsplit * NN, p.dt, p.N, kp);
+        }
+    } else
         hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N), p.nd), dim3(256), 0, st, kpart,
                            (int64_t)p.nsplit * NN, nsplit_used, p.N, kp);
     F2JK_LAUNCHED("k_reduce");
@@ -1004,7 +1044,7 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
     }
     // the J passes: on the side stream (forked once their inputs exist) when they
     // run beside K
-    const bool overlap = p.want_j && p.want_k &&
+    const bool overlap = p.want_j && p.want_k && !p.small &&
                          (ctx->overlap_jk < 0 ? (p.gamma_x || (p.prec == F2JK_PREC_BF16X3 && p.ks_tile == 256)) &&
                                                     !ctx->timing && j_pass_bytes(p) >= kOverlapBytes
                                               : ctx->overlap_jk == 1);
@@ -1031,9 +1071,9 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
         if (p.prec == F2JK_PREC_BF16X3)
             rc = run_k_bf16x3(ctx, p, K, w, st, [&] { return j_late ? do_j() : F2JK_OK; });
         else if (p.tk == 8)
-            rc = run_k_typed<double>(ctx, p, nocc, K, w, st, [&] { return p.gamma_x ? do_j() : F2JK_OK; });
+            rc = run_k_typed<double>(ctx, p, nocc, J, K, w, st, [&] { return p.gamma_x ? do_j() : F2JK_OK; });
         else
-            rc = run_k_typed<float>(ctx, p, nocc, K, w, st, [] { return F2JK_OK; });
+            rc = run_k_typed<float>(ctx, p, nocc, J, K, w, st, [] { return F2JK_OK; });
     }
     // join, also after a failed launch: later work on the caller's stream comes
     // after the side stream's

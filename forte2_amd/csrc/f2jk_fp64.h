@@ -645,4 +645,49 @@ __global__ __launch_bounds__(256) void kred_kernel(const double* __restrict__ Kp
     k_reduce_body(Kpart + blockIdx.y * dstride, dtile_splits(tm, m4, n16), N, K.p[blockIdx.y], m4, n16);
 }
 
+// both reductions of a small build in one launch: nbj blocks of J, the rest K
+template <int VEC, int ND>
+__global__ __launch_bounds__(256) void jkred_kernel(const double* __restrict__ jpart, int nchunks, int N,
+                                                    const int* __restrict__ rowoff, const int* __restrict__ jinv,
+                                                    int nlist, int nvec, JPtrs<ND> J, int nbj,
+                                                    const double* __restrict__ Kpart, int64_t dstride, DTiles tm,
+                                                    KPtrs K) {
+    if ((int)blockIdx.x < nbj) {
+        j_reduce_body<VEC, ND>(jpart, nchunks, N, rowoff, jinv, nlist, nvec, J, blockIdx.x);
+        return;
+    }
+    const int per = k_reduce_blocks(N), b = blockIdx.x - nbj, d = b / per;
+    const int nb = (N + 15) / 16, m4 = b % per / nb, n16 = b % per % nb;
+    if (n16 * 16 > m4 * 4 + 3) return;
+    k_reduce_body(Kpart + d * dstride, dtile_splits(tm, m4, n16), N, K.p[d], m4, n16);
+}
+
+// The second J pass of a small build with gamma formed by its own blocks from
+// the half-transform's row sums (gamma_rows_kernel's sums in the same order),
+// which saves a launch; a block has at most kGBlock values of P.
+template <int VEC, int EPT, int ND>
+__global__ __launch_bounds__(kJThreads) void j_accum_rows_kernel(const double* __restrict__ B, int N, int Q,
+                                                                 const double* __restrict__ grow, int64_t gstride,
+                                                                 int ncolt, const int* __restrict__ rowoff,
+                                                                 const uint32_t* __restrict__ elist, int nvec, int ppw,
+                                                                 double* __restrict__ jpart) {
+    __shared__ double g[ND * kGBlock];
+    const int P0 = blockIdx.y * ppw, np = min(Q, P0 + ppw) - P0;
+    const int lane = threadIdx.x & 63;
+    for (int t = threadIdx.x >> 6; t < ND * np; t += kJThreads / 64) {
+        const int d = t / np, p = t % np;
+        double s = 0.0;
+        for (int ct = 0; ct < ncolt; ++ct) {
+            const double* r = grow + (int64_t)(ct * ND + d) * gstride + (int64_t)(P0 + p) * N;
+            for (int m = lane; m < N; m += 64) s += r[m];
+        }
+        s = wave_sum(s);
+        if (lane == 0) g[d * kGBlock + p] = s;
+    }
+    __syncthreads();
+    const auto gamma = [&](int d, int P) { return g[d * kGBlock + P - P0]; };
+    j_accum_kernel_body<double, VEC, EPT, ND, true>(B, N, Q, gamma, rowoff, nvec, ppw, jpart, blockIdx.x, blockIdx.y,
+                                                    elist);
+}
+
 }  // namespace f2jk

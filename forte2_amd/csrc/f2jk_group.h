@@ -205,9 +205,9 @@ void grouped_kernel(const GArgs a) {
             const int bx = local % g.neg, by = local / g.neg;
             const TB* B = (const TB*)g.B;
             if (g.nd == 2)
-                j_accum_kernel_body<TB, 2, 4, 2, true>(B, g.N, g.Q, g.gamma, g.rowoff, g.nvec, g.ppw2, g.jpart, bx, by);
+                j_accum_kernel_body<TB, 2, 4, 2, true>(B, g.N, g.Q, GammaAll{g.gamma, g.Q}, g.rowoff, g.nvec, g.ppw2, g.jpart, bx, by);
             else
-                j_accum_kernel_body<TB, 2, 4, 1, true>(B, g.N, g.Q, g.gamma, g.rowoff, g.nvec, g.ppw2, g.jpart, bx, by);
+                j_accum_kernel_body<TB, 2, 4, 1, true>(B, g.N, g.Q, GammaAll{g.gamma, g.Q}, g.rowoff, g.nvec, g.ppw2, g.jpart, bx, by);
         } else if constexpr (PHASE == GP_JRED) {
             if (g.nd == 2) {
                 JPtrs<2> jp{{g.J[0], g.J[1]}};

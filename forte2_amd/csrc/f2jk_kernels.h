@@ -255,18 +255,27 @@ __global__ void j_gamma_reduce_kernel(const double* __restrict__ gpart, int ngro
     gamma[t] = s;
 }
 
+constexpr int kGBlock = 16;  // most P values of a block that forms its own gamma
 // ---------------------------------------------------------------------------
 // J pass 2: partial J per (P chunk, density, element).
 // grid = (n_element_groups, n_p_chunks), block = 256.
 // ---------------------------------------------------------------------------
-template <typename TB, int VEC, int EPT, int ND, bool NT = false>
+// gamma(d, P): gamma of every P in global memory, or a block's own in LDS
+struct GammaAll {
+    const double* g;
+    int Q;
+    __device__ __forceinline__ double operator()(int d, int P) const { return g[(int64_t)d * Q + P]; }
+};
+template <typename TB, int VEC, int EPT, int ND, bool NT = false, typename Gamma>
 __device__ __forceinline__ void j_accum_kernel_body(
-    const TB* __restrict__ B, int N, int Q, const double* __restrict__ gamma,
+    const TB* __restrict__ B, int N, int Q, const Gamma& gamma,
     const int* __restrict__ rowoff, int nvec, int ppw, double* __restrict__ jpart, int bx, int by,
     const uint32_t* __restrict__ elist = nullptr, const TB* __restrict__ packed = nullptr) {
     const int tid = threadIdx.x;
     const int64_t NN = packed ? (int64_t)nvec * VEC : (int64_t)N * N;
     if (packed) B = packed;
+    const int P0 = by * ppw;
+    const int P1 = min(Q, P0 + ppw);
     int64_t off[EPT];
     int eidx[EPT];
 #pragma unroll
@@ -292,8 +301,6 @@ __device__ __forceinline__ void j_accum_kernel_body(
 #pragma unroll
             for (int v = 0; v < VEC; ++v) acc[k][dd][v] = 0.0;
 
-    const int P0 = by * ppw;
-    const int P1 = min(Q, P0 + ppw);
     int P = P0;
     for (; P + 1 < P1; P += 2) {
         const TB* B0 = B + (int64_t)P * NN;
@@ -307,8 +314,8 @@ __device__ __forceinline__ void j_accum_kernel_body(
         double g0[ND], g1[ND];
 #pragma unroll
         for (int dd = 0; dd < ND; ++dd) {
-            g0[dd] = gamma[(int64_t)dd * Q + P];
-            g1[dd] = gamma[(int64_t)dd * Q + P + 1];
+            g0[dd] = gamma(dd, P);
+            g1[dd] = gamma(dd, P + 1);
         }
 #pragma unroll
         for (int k = 0; k < EPT; ++k)
@@ -327,7 +334,7 @@ __device__ __forceinline__ void j_accum_kernel_body(
             Vec<TB, VEC> b0 = stream_vec<TB, VEC, NT>(B0 + off[k]);
 #pragma unroll
             for (int dd = 0; dd < ND; ++dd) {
-                const double g = gamma[(int64_t)dd * Q + P];
+                const double g = gamma(dd, P);
 #pragma unroll
                 for (int v = 0; v < VEC; ++v) acc[k][dd][v] = fma(g, (double)b0.v[v], acc[k][dd][v]);
             }
@@ -349,7 +356,7 @@ __global__ __launch_bounds__(kJThreads) void j_accum_kernel(
     const TB* __restrict__ B, int N, int Q, const double* __restrict__ gamma,
     const int* __restrict__ rowoff, const uint32_t* __restrict__ elist, const TB* __restrict__ packed, int nvec,
     int ppw, double* __restrict__ jpart) {
-    j_accum_kernel_body<TB, VEC, EPT, ND, NT>(B, N, Q, gamma, rowoff, nvec, ppw, jpart, blockIdx.x, blockIdx.y,
+    j_accum_kernel_body<TB, VEC, EPT, ND, NT>(B, N, Q, GammaAll{gamma, Q}, rowoff, nvec, ppw, jpart, blockIdx.x, blockIdx.y,
                                               elist, packed);
 }
 
@@ -376,7 +383,7 @@ __device__ __forceinline__ void j_reduce_body(const double* __restrict__ jpart, 
 #pragma unroll
         for (int v = 0; v < VEC; ++v) s[dd][v] = 0.0;
     if (le >= 0) {
-#pragma unroll 4
+#pragma unroll 8
         for (int c = w; c < nchunks; c += 4)
 #pragma unroll
             for (int dd = 0; dd < ND; ++dd) {
@@ -1735,7 +1742,7 @@ __device__ __forceinline__ void k_reduce_body(const double* __restrict__ Kpart, 
     double s = 0.0;
     if (on) {
         const double* p = Kpart + (int64_t)m * N + n;
-#pragma unroll 4
+#pragma unroll 8
         for (int c = w; c < nsplit; c += 4) s += p[c * NN];
     }
     if (w > 0) red[w - 1][lane] = s;
