@@ -393,10 +393,13 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
             p.dnb = (int)cdiv(nb, p.dncolt);
             p.dnks = (int)cdiv(N, kDK);
         }
+        // FP64 K alone reads neither of them, and with J no fp32 copy: K-only builds
+        // that fitted the no-alloc scratch array before Cq came still do
+        const bool dk = precision == F2JK_PREC_FP64 && p.want_k;
         p.off_cp = off;
-        off += align_up((size_t)N * std::max(p.OPAD, p.dncolt * p.dnb * 16) * 8);
+        if (!dk || p.gamma_x) off += align_up((size_t)N * std::max(p.OPAD, p.dncolt * p.dnb * 16) * 8);
         p.off_cp32 = off;
-        off += align_up((size_t)N * p.OPAD * 4);  // fp32 copy (FP32 K)
+        if (!dk) off += align_up((size_t)N * p.OPAD * 4);  // fp32 copy (FP32 K)
         if (precision == F2JK_PREC_FP64 && p.want_k) {
             p.off_cq = off;
             // where J and K come from C, D is not formed: Cq lies in the room of
@@ -667,7 +670,7 @@ int pack_c(f2jk_ctx* ctx, const Plan& p, const double* const* C, const int64_t* 
         }
         const int64_t n = (int64_t)p.dncolt * p.dnks * p.dnb * 256;
         hipLaunchKernelGGL(pack_cq_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, cs, dcols_of(p, nocc), p.N,
-                           p.dncolt * p.dnb * 16, p.dnb, p.dnks, n, cp, (double*)(ws + p.off_cq));
+                           p.dncolt * p.dnb * 16, p.dnb, p.dnks, n, p.gamma_x ? cp : nullptr, (double*)(ws + p.off_cq));
         F2JK_LAUNCHED("pack_cq");
         return F2JK_OK;
     }
@@ -1531,7 +1534,7 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
         std::memset(&g, 0, sizeof(g));
         g.B = ctxs[j]->B[precision == F2JK_PREC_FP64 ? F2JK_F64 : F2JK_F32];
         g.rowoff = want_j ? ctxs[j]->rowoff[p.jvec] : nullptr;
-        g.Cp = (double*)(w + p.off_cp);
+        g.Cp = precision != F2JK_PREC_FP64 || p.gamma_x ? (double*)(w + p.off_cp) : nullptr;
         g.Cp32 = (float*)(w + p.off_cp32);
         g.Cq = (double*)(w + p.off_cq);
         g.dnb = p.dnb;

@@ -83,7 +83,7 @@ struct DCols2 {
 // ---------------------------------------------------------------------------
 // Coefficients of all densities in the two forms the kernels read:
 //   Cp[n][c]  row-major, the columns of all tiles (the gamma sums of the
-//             half-transform);
+//             half-transform; null without them);
 //   Cq        [column tile][16-k step][block][k / 8 % 2][lane][2], the order
 //             of the half-transform's LDS tiles; zero outside N x nocc.
 // ---------------------------------------------------------------------------
@@ -107,7 +107,7 @@ __device__ __forceinline__ void pack_cq_element(const double* const* C, const in
         if (i >= 0 && i < nocc[d] && k < N) x = C[d][(int64_t)k * ldc[d] + i];
     }
     Cq[t] = x;
-    if (k < N) Cp[(int64_t)k * ldcp + c] = x;
+    if (Cp && k < N) Cp[(int64_t)k * ldcp + c] = x;
 }
 __global__ void pack_cq_kernel(DCoef cs, DCols dc, int N, int ldcp, int nb, int nks, int64_t total,
                                double* __restrict__ Cp, double* __restrict__ Cq) {
