@@ -1009,6 +1009,16 @@ int run_k_bf16x3(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipSt
 constexpr double kOverlapBytes = 128e6;
 double j_pass_bytes(const Plan& p) { return (double)p.nvec * p.jvec * p.jb * p.Q; }
 
+// A stream that joins a capture stays in it until the capture ends, and another
+// stream's build on the same context meanwhile would be drawn in: a build being
+// captured keeps to its own stream unless "overlap_jk" asks for the side stream.
+bool capturing(hipStream_t st) {
+    if (!st) return false;  // the default stream cannot be captured
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();
+    return status != hipStreamCaptureStatusNone;
+}
+
 int check_ws(const Plan& p, void* ws, size_t ws_bytes) {
     if (!ws) return fail(F2JK_EINVAL, "workspace pointer is NULL");
     if (ws_bytes < p.total)
@@ -1049,7 +1059,7 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
     // run beside K
     const bool overlap = p.want_j && p.want_k && !p.small &&
                          (ctx->overlap_jk < 0 ? (p.gamma_x || (p.prec == F2JK_PREC_BF16X3 && p.ks_tile == 256)) &&
-                                                    !ctx->timing && j_pass_bytes(p) >= kOverlapBytes
+                                                    !ctx->timing && j_pass_bytes(p) >= kOverlapBytes && !capturing(st)
                                               : ctx->overlap_jk == 1);
     hipStream_t sj = overlap ? ctx->side : st;
     bool forked = false;
@@ -1596,7 +1606,7 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
     double jbytes = 0.0;
     for (const Plan& p : plans) jbytes += j_pass_bytes(p);
     const bool beside = want_j && precision == F2JK_PREC_FP64 && !ctx->timing &&
-                        (ctx->overlap_jk < 0 ? jbytes >= kOverlapBytes : ctx->overlap_jk == 1);
+                        (ctx->overlap_jk < 0 ? jbytes >= kOverlapBytes && !capturing(st) : ctx->overlap_jk == 1);
     for (int j0 = 0; j0 < njobs; j0 += kMaxGroup) {
         GArgs a;
         std::memset(&a, 0, sizeof(a));

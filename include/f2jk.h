@@ -95,8 +95,9 @@ int f2jk_get_shape(const f2jk_ctx* ctx, int64_t* naux, int64_t* nbf);
  * split launch aims for (default 2048); "j_nontemporal" (0/1, default 1)
  * streams B through non-temporal loads in the J passes; "overlap_jk" (0, 1,
  * -1; default -1 = FP64 J and K from C, and BF16x3 with 256-wide contraction
- * tiles, when a J pass reads 128 MB or more and F2JK_TIMING is not asked for) runs the J passes of a build_jk on the context's side stream
- * concurrently with K (joined back before the call returns its work to the
+ * tiles, when a J pass reads 128 MB or more, F2JK_TIMING is not asked for and
+ * the stream is not being captured) runs the J passes of a build_jk on the
+ * context's side stream concurrently with K (joined back before the call returns its work to the
  * caller's stream); "bf16_nbw_max" (2, 4, 5, 6, 8, 10) caps the BF16x3
  * half-transform tile at 32 * value occupied columns (tiles of up to 5 run two
  * workgroups per CU); "kx_waves" (4 or 8, default 8) is the number of waves of

@@ -68,3 +68,36 @@ def test_k_alone_in_the_scratch_array(dev, N, o, nd):
             ref += x @ x.T
         assert (K.cpu() - ref).abs().max().item() <= 1e-10
     nat.jk_lib().f2jk_ctx_destroy(h)
+
+
+def test_captured_build_beside_an_eager_one(dev):
+    # J reads 158 MB: the eager build runs it on the context's side stream, which
+    # must not have joined the capture
+    N, Q = 256, 600
+    print(f"[capture] N={N} Q={Q}", flush=True)
+    B = synthetic_B(Q, N, seed=3, device=dev)
+    C = orthonormal_C(N, 40, seed=1, device=dev)
+    flags = nat.F2JK_WANT_J | nat.F2JK_WANT_K
+    h = _ctx(dev, B)
+    ws = _workspace(h, [C], flags, dev)
+    eager, graphed = _Build(h, [C], flags, ws), _Build(h, [C], flags, None)
+    eager(), graphed()
+    torch.cuda.synchronize()
+    ref_e, ref_g = eager.out(), graphed.out()
+    other = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode="relaxed"):
+        graphed()
+        with torch.cuda.stream(other):
+            eager()
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(eager.out(), ref_e))
+    for _ in range(3):
+        for x in graphed.J + graphed.K:
+            x.zero_()
+        graph.replay()
+        eager()  # eager work behind the replay
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(graphed.out(), ref_g))
+        assert all(torch.equal(a, b) for a, b in zip(eager.out(), ref_e))
+    nat.jk_lib().f2jk_ctx_destroy(h)
