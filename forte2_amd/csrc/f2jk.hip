@@ -129,7 +129,7 @@ struct Plan {
     int KP = 0;                // nbf rounded up to the bf16 k step
     size_t off_cp32 = 0, off_cth = 0, off_ctl = 0, off_cq = 0;
     size_t off_grow = 0;
-    size_t off_cp = 0, off_d = 0, off_dpart = 0, off_gpart = 0, off_gamma = 0, off_jpart = 0,
+    size_t off_cp = 0, off_d = 0, off_gpart = 0, off_gamma = 0, off_jpart = 0,
            off_x = 0, off_kpart = 0, total = 0;
     // sizes of the regions that scale with the launch-shape knobs
     size_t jpart_bytes = 0, x_bytes = 0, kpart_bytes = 0;
@@ -447,8 +447,6 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         if (j_from_c && !p.gamma_x) {
             p.off_d = off;
             off += align_up((size_t)ndens * N * N * 8);
-            p.off_dpart = off;
-            off += align_up((size_t)N * N * 8);
         }
         p.off_gpart = off;
         if (!p.gamma_x) off += align_up((size_t)p.neg * ndens * Q * 8);
@@ -657,73 +655,46 @@ DCols dcols_of(const Plan& p, const int64_t* nocc) {
 }
 
 int pack_c(f2jk_ctx* ctx, const Plan& p, const double* const* C, const int64_t* nocc,
-           const int64_t* ldc, char* ws, hipStream_t st, bool want_f32) {
+           const int64_t* ldc, char* ws, hipStream_t st) {
     double* cp = (double*)(ws + p.off_cp);
-    float* cp32 = (float*)(ws + p.off_cp32);
+    DCoef cs{};
+    for (int d = 0; d < p.nd; ++d) {
+        if (nocc[d] > 0 && (!C[d] || !ldc || ldc[d] < nocc[d]))
+            return fail(F2JK_EINVAL, "C pointer / ldc invalid");
+        cs.C[d] = C[d];
+        cs.ldc[d] = nocc[d] > 0 ? ldc[d] : 1;
+    }
     if (p.want_k && p.prec == F2JK_PREC_FP64) {
-        DCoef cs{};
-        for (int d = 0; d < p.nd; ++d) {
-            if (nocc[d] > 0 && (!C[d] || !ldc || ldc[d] < nocc[d]))
-                return fail(F2JK_EINVAL, "C pointer / ldc invalid");
-            cs.C[d] = C[d];
-            cs.ldc[d] = nocc[d] > 0 ? ldc[d] : 1;
-        }
         const int64_t n = (int64_t)p.dncolt * p.dnks * p.dnb * 256;
         hipLaunchKernelGGL(pack_cq_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, cs, dcols_of(p, nocc), p.N,
                            p.dncolt * p.dnb * 16, p.dnb, p.dnks, n, p.gamma_x ? cp : nullptr, (double*)(ws + p.off_cq));
         F2JK_LAUNCHED("pack_cq");
         return F2JK_OK;
     }
-    for (int d = 0; d < p.nd; ++d) {
-        if (nocc[d] > 0 && (!C[d] || !ldc || ldc[d] < nocc[d]))
-            return fail(F2JK_EINVAL, "C pointer / ldc invalid");
-        const int64_t n = (int64_t)p.N * p.width[d];
-        hipLaunchKernelGGL(pad_c_kernel<double>, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st,
-                           C[d], nocc[d] > 0 ? ldc[d] : 1, p.N, (int)nocc[d], p.width[d], p.ioff[d],
-                           p.OPAD, cp);
-        F2JK_LAUNCHED("pad_c");
-        if (want_f32) {
-            hipLaunchKernelGGL(pad_c_kernel<float>, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st,
-                               C[d], nocc[d] > 0 ? ldc[d] : 1, p.N, (int)nocc[d], p.width[d],
-                               p.ioff[d], p.OPAD, cp32);
-            F2JK_LAUNCHED("pad_c32");
-        }
-        if (p.want_k && p.prec == F2JK_PREC_BF16X3) {
-            const int64_t nt = (int64_t)p.width[d] * p.KP;
-            hipLaunchKernelGGL(pad_ct_bf16_kernel, dim3((unsigned)cdiv(nt, 256)), dim3(256), 0, st,
-                               C[d], nocc[d] > 0 ? ldc[d] : 1, p.N, (int)nocc[d], p.width[d],
-                               p.ioff[d], p.KP, (u16*)(ws + p.off_cth), (u16*)(ws + p.off_ctl));
-            F2JK_LAUNCHED("pad_ct_bf16");
-        }
-    }
+    PackOut out{};
+    if (p.want_j) out.Cp = cp;
+    if (p.want_k && p.prec == F2JK_PREC_FP32) out.Cp32 = (float*)(ws + p.off_cp32);
+    int64_t n = (int64_t)p.N * p.OPAD;
     if (p.want_k && p.prec == F2JK_PREC_BF16X3) {
-        // zero rows past the occupied columns: the tall half-transform loads
+        // with zero rows past the occupied columns: the tall half-transform loads
         // whole column tiles without clamping
-        const int zr = p.ctrows - p.OPAD;
-        const int64_t nt = (int64_t)zr * p.KP;
-        hipLaunchKernelGGL(pad_ct_bf16_kernel, dim3((unsigned)cdiv(nt, 256)), dim3(256), 0, st, C[0], 1, p.N, 0,
-                           zr, p.OPAD, p.KP, (u16*)(ws + p.off_cth), (u16*)(ws + p.off_ctl));
-        F2JK_LAUNCHED("pad_ct_bf16 zero rows");
+        out.Th = (u16*)(ws + p.off_cth);
+        out.Tl = (u16*)(ws + p.off_ctl);
+        out.rows = p.ctrows;
+        out.KP = p.KP;
+        n = (int64_t)p.ctrows * p.KP;
     }
+    hipLaunchKernelGGL(pack_c_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, cs, dcols_of(p, nocc), p.N, p.OPAD,
+                       out);
+    F2JK_LAUNCHED("pack_c");
     return F2JK_OK;
 }
 
-// D_d = Cp_d Cp_d^T via the contraction kernel with a single "P".
-int build_d(f2jk_ctx* ctx, const Plan& p, char* ws, hipStream_t st) {
-    const double* cp = (const double*)(ws + p.off_cp);
-    double* dbuf = (double*)(ws + p.off_d);
-    double* dpart = (double*)(ws + p.off_dpart);
-    const int nt = (int)cdiv(p.N, kTile);
-    const int nlower = nt * (nt + 1) / 2;
-    for (int d = 0; d < p.nd; ++d) {
-        hipLaunchKernelGGL(ks_kernel<double>, dim3(nlower), dim3(kGThreads), 0, st, cp, p.N, p.OPAD,
-                           p.ioff[d], p.width[d], 1, 1, nlower, dpart, 0);
-        F2JK_LAUNCHED("ks(D)");
-        KPtrs dp{};
-        dp.p[0] = dbuf + (size_t)d * p.N * p.N;
-        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N)), dim3(256), 0, st, dpart, (int64_t)0, 1, p.N, dp);
-        F2JK_LAUNCHED("k_reduce(D)");
-    }
+// D_d = Cp_d Cp_d^T
+int build_d(const Plan& p, const int64_t* nocc, char* ws, hipStream_t st) {
+    hipLaunchKernelGGL(d_kernel, dim3(d_blocks(p.N), p.nd), dim3(256), 0, st, (const double*)(ws + p.off_cp), p.N, p.OPAD,
+                       dcols_of(p, nocc), (double*)(ws + p.off_d));
+    F2JK_LAUNCHED("d");
     return F2JK_OK;
 }
 
@@ -1050,9 +1021,9 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
     TIM(F2JK_PH_TOTAL, true);
     if (p.need_c) {
         TIM(F2JK_PH_PREP, true);
-        if ((rc = pack_c(ctx, p, C, nocc, ldc, w, st, p.want_k && p.prec == F2JK_PREC_FP32))) return rc;
+        if ((rc = pack_c(ctx, p, C, nocc, ldc, w, st))) return rc;
         if (p.want_j && j_from_c && !p.gamma_x)
-            if ((rc = build_d(ctx, p, w, st))) return rc;
+            if ((rc = build_d(p, nocc, w, st))) return rc;
         TIM(F2JK_PH_PREP, false);
     }
     // the J passes: on the side stream (forked once their inputs exist) when they
@@ -1215,10 +1186,8 @@ int run_group(f2jk_ctx* ctx, const GArgs& a, int nbw, int va, hipStream_t st, bo
     constexpr bool gamma_x = PREC == F2JK_PREC_FP64;  // gamma comes with the half-transform
     TIM(F2JK_PH_PREP, true);
     if ((rc = launch_group_phase<GP_PAD, PREC>(a, st))) return rc;
-    if constexpr (!gamma_x) {
-        if ((rc = launch_group_phase<GP_DKS, PREC>(a, st))) return rc;
-        if ((rc = launch_group_phase<GP_DRED, PREC>(a, st))) return rc;
-    }
+    if constexpr (!gamma_x)
+        if ((rc = launch_group_phase<GP_D, PREC>(a, st))) return rc;
     TIM(F2JK_PH_PREP, false);
     TIM(F2JK_PH_KX, true);
     if constexpr (PREC == F2JK_PREC_BF16X3) {
@@ -1561,7 +1530,6 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
         if (want_j) {
             g.grow = (double*)(w + p.off_grow);
             g.D = (double*)(w + p.off_d);
-            g.Dpart = (double*)(w + p.off_dpart);
             g.gpart = (double*)(w + p.off_gpart);
             g.gamma = (double*)(w + p.off_gamma);
             g.jpart = (double*)(w + p.off_jpart);
@@ -1647,7 +1615,7 @@ int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ld
     char* w = (char*)ws;
     const double* Cs[1] = {C};
     const int64_t lds[1] = {ldc};
-    if ((rc = pack_c(ctx, p, Cs, &ncol, lds, w, st, false))) return rc;
+    if ((rc = pack_c(ctx, p, Cs, &ncol, lds, w, st))) return rc;
     const double* B = (const double*)ctx->B[F2JK_F64];
     const double* cq = (const double*)(w + p.off_cq);
     const int64_t NN = (int64_t)p.N * p.N;
@@ -1722,7 +1690,7 @@ int f2jk_mo_block(f2jk_ctx* ctx, const double* C1, int64_t n1, int64_t ld1, cons
     const double* cq[2];
     for (int i = 0; i < 2; ++i) {
         char* w = (char*)ws + m.off_c[i];
-        if ((rc = pack_c(ctx, m.c[i], &C[i], &n[i], &ld[i], w, st, false))) return rc;
+        if ((rc = pack_c(ctx, m.c[i], &C[i], &n[i], &ld[i], w, st))) return rc;
         cq[i] = (const double*)(w + m.c[i].off_cq);
     }
     const Plan &p1 = m.c[0], &p2 = m.c[1];

@@ -690,4 +690,122 @@ __global__ __launch_bounds__(kJThreads) void j_accum_rows_kernel(const double* _
                                                     elist);
 }
 
+// ---------------------------------------------------------------------------
+// Coefficients and D of the builds whose J needs D (FP32 and BF16x3 forms, J
+// alone from C): one launch for every copy and density, and one for D.
+// Rounds of launches bound both: at nbf 384 with 80 columns in BF16x3 five
+// launches took 43 us (D's 128 x 128 tiles, six workgroups: 23 us, and its
+// mirror); with these two the build went from 751 to 735 us, builds of 90 us
+// lost 9 (one density) and 26 us (two).
+// ---------------------------------------------------------------------------
+struct PackOut {
+    double* Cp;     // N x OPAD, or null
+    float* Cp32;    // the same in FP32, or null
+    u16 *Th, *Tl;   // transposed hi/lo bf16 planes, rows x KP with zeros past nocc and N, or null
+    int rows, KP;
+};
+__global__ void pack_c_kernel(DCoef cs, DCols dc, int N, int OPAD, PackOut out) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int c, k;
+    if (out.Th) {
+        if (t >= (int64_t)out.rows * out.KP) return;
+        c = (int)(t / out.KP), k = (int)(t % out.KP);
+    } else {
+        if (t >= (int64_t)N * OPAD) return;
+        k = (int)(t / OPAD), c = (int)(t % OPAD);
+    }
+    double x = 0.0;
+    for (int d = 0; d < dc.nd; ++d) {
+        const int i = c - dc.ioff[d];
+        if (i >= 0 && i < dc.nocc[d] && k < N) x = cs.C[d][(int64_t)k * cs.ldc[d] + i];
+    }
+    if (out.Th) {
+        __bf16 h, l;
+        split_bf16_from_double(x, h, l);
+        out.Th[t] = __builtin_bit_cast(u16, h);
+        out.Tl[t] = __builtin_bit_cast(u16, l);
+    }
+    if (k < N && c < OPAD) {
+        if (out.Cp) out.Cp[(int64_t)k * OPAD + c] = x;
+        if (out.Cp32) out.Cp32[(int64_t)k * OPAD + c] = (float)x;
+    }
+}
+
+// D = Cp Cp^T over the columns [ioff, ioff + width) (a multiple of 16): one
+// 32 x 32 tile of the lower triangle per wave, operands from global memory
+// (Cp is small enough for L2), a 16-k step ahead.  No mirror: J reads the lower
+// triangle only.
+constexpr int kDTile = 32;
+__host__ __device__ inline int d_blocks(int N) {  // of four waves
+    const int nt = (N + kDTile - 1) / kDTile;
+    return (nt * (nt + 1) / 2 + 3) / 4;
+}
+__device__ __forceinline__ void d_body(const double* __restrict__ Cp, int N, int OPAD, int ioff, int width,
+                                       double* __restrict__ D, int b) {
+    const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+    const int t = b * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int nt = (N + kDTile - 1) / kDTile;
+    if (t >= nt * (nt + 1) / 2) return;
+    int mt = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+    while (mt * (mt + 1) / 2 > t) --mt;
+    while ((mt + 1) * (mt + 2) / 2 <= t) ++mt;
+    const int m0 = mt * kDTile, n0 = (t - mt * (mt + 1) / 2) * kDTile;
+    const double *ap[2], *bp[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {  // rows past N are clamped onto the last and never stored
+        const int r = m0 + i * 16 + lr, c = n0 + i * 16 + lr;
+        ap[i] = Cp + (int64_t)(r < N ? r : N - 1) * OPAD + ioff + 2 * lg;
+        bp[i] = Cp + (int64_t)(c < N ? c : N - 1) * OPAD + ioff + 2 * lg;
+    }
+    dx4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = dx4{0, 0, 0, 0};
+    dx2 an[2][2], bn[2][2];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                an[i][h] = *reinterpret_cast<const dx2*>(ap[i] + k0 + 8 * h);
+                bn[i][h] = *reinterpret_cast<const dx2*>(bp[i] + k0 + 8 * h);
+            }
+    };
+    load(0);
+    for (int k0 = 0; k0 < width; k0 += 16) {
+        dx2 a[2][2], c[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) a[i][h] = an[i][h], c[i][h] = bn[i][h];
+        if (k0 + 16 < width) load(k0 + 16);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma4(a[i][h].x, c[j][h].x, acc[i][j]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma4(a[i][h].y, c[j][h].y, acc[i][j]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = m0 + i * 16 + acc_row<double>(lane, r), n = n0 + j * 16 + lr;
+                if (m < N && n < N) D[(int64_t)m * N + n] = acc[i][j][r];
+            }
+}
+__global__ __launch_bounds__(256) void d_kernel(const double* __restrict__ Cp, int N, int OPAD, DCols dc,
+                                                double* __restrict__ D) {
+    const int d = blockIdx.y;
+    d_body(Cp, N, OPAD, dc.ioff[d], dc.width[d], D + (int64_t)d * N * N, blockIdx.x);
+}
+
 }  // namespace f2jk

@@ -32,23 +32,22 @@ constexpr int kMaxGroup = 12;
 enum GroupPhase {
     GP_PAD = 0,      // Cp[n][ioff+i] = C[n][i] (FP64; also the half-transform's copy of
                      // FP64 K, the FP32 copy, or the transposed hi/lo bf16 copies)
-    GP_DKS = 1,      // Dpart[d] = Cp_d Cp_d^T (lower tiles; precision forms)
-    GP_DRED = 2,     // D[d] mirrored from Dpart[d] (precision forms)
-    GP_GAMMA = 3,    // J pass 1 (precision forms)
-    GP_GRED = 4,     // gamma reduction (FP64: of the half-transform's row sums)
-    GP_JACC = 5,     // J pass 2
-    GP_JRED = 6,     // J reduction + mirror
-    GP_KX = 7,       // half-transform (whole B: one chunk)
-    GP_KS = 8,       // contraction, splits of P
-    GP_KRED = 9,     // K reduction + mirror
-    GP_NPHASE = 10
+    GP_D = 1,        // D[d] = Cp_d Cp_d^T, lower tiles (precision forms)
+    GP_GAMMA = 2,    // J pass 1 (precision forms)
+    GP_GRED = 3,     // gamma reduction (FP64: of the half-transform's row sums)
+    GP_JACC = 4,     // J pass 2
+    GP_JRED = 5,     // J reduction + mirror
+    GP_KX = 6,       // half-transform (whole B: one chunk)
+    GP_KS = 7,       // contraction, splits of P
+    GP_KRED = 8,     // K reduction + mirror
+    GP_NPHASE = 9
 };
 
 struct GJob {
     const void* B;        // FP64 B (FP64 groups) or the FP32 copy (FP32 / BF16x3 groups)
     const int* rowoff;
     const double* C[2];
-    double *Cp, *D, *Dpart, *gpart, *gamma, *jpart, *Kpart;
+    double *Cp, *D, *gpart, *gamma, *jpart, *Kpart;
     double *Cq, *grow;    // FP64: coefficients in the half-transform's order, its row sums
     float* Cp32;          // FP32 coefficients (FP32 K)
     u16 *Cth, *Ctl;       // transposed hi/lo coefficients (BF16x3 K)
@@ -81,8 +80,7 @@ __host__ __device__ inline int phase_blocks(const GJob& g, int phase) {
         case GP_PAD:
             if (PREC == F2JK_PREC_FP64) return g.dncolt * g.dnks * g.dnb;
             return gcdiv((long long)(PREC == F2JK_PREC_BF16X3 ? g.KP : g.N) * g.OPAD, 256);
-        case GP_DKS: return j * g.nlower * g.nd;
-        case GP_DRED: return j * k_reduce_blocks(g.N) * g.nd;
+        case GP_D: return j * d_blocks(g.N) * g.nd;
         case GP_GAMMA: return j * g.neg * g.npc1;
         case GP_GRED: return j * gcdiv((long long)g.nd * g.Q, PREC == F2JK_PREC_FP64 ? 4 : 256);
         case GP_JACC: return j * g.neg * g.npc2;
@@ -163,22 +161,16 @@ void grouped_kernel(const GArgs a) {
                 g.Cp[t] = x;
                 g.Cp32[t] = (float)x;
             }
-        } else if constexpr (PHASE == GP_DKS) {
-            const int d = local / g.nlower, b = local % g.nlower;
-            ks_kernel_body<double>(g.Cp, g.N, g.OPAD, g.ioff[d], g.width[d], 1, 1, g.nlower,
-                                   g.Dpart + (long long)d * g.N * g.N, 0, b, g.nlower);
-        } else if constexpr (PHASE == GP_DRED || PHASE == GP_KRED) {
+        } else if constexpr (PHASE == GP_D) {
+            const int per = d_blocks(g.N), d = local / per;
+            d_body(g.Cp, g.N, g.OPAD, g.ioff[d], g.width[d], g.D + (long long)d * g.N * g.N, local % per);
+        } else if constexpr (PHASE == GP_KRED) {
             const int per = k_reduce_blocks(g.N), nb = gcdiv(g.N, 16);
             const int d = local / per, m4 = local % per / nb, n16 = local % per % nb;
             const long long NN = (long long)g.N * g.N;
-            if (n16 * 16 <= m4 * 4 + 3) {
-                if constexpr (PHASE == GP_DRED)
-                    k_reduce_body(g.Dpart + d * NN, 1, g.N, g.D + d * NN, m4, n16);
-                else
-                    k_reduce_body(g.Kpart + d * g.nsplit * NN,
-                                  PREC == F2JK_PREC_FP64 ? dtile_splits(g.dt, m4, n16) : g.nsplit, g.N, g.K[d], m4,
-                                  n16);
-            }
+            if (n16 * 16 <= m4 * 4 + 3)
+                k_reduce_body(g.Kpart + d * g.nsplit * NN,
+                              PREC == F2JK_PREC_FP64 ? dtile_splits(g.dt, m4, n16) : g.nsplit, g.N, g.K[d], m4, n16);
         } else if constexpr (PHASE == GP_GAMMA) {
             const int bx = local % g.neg, by = local / g.neg;
             const long long NN = (long long)g.N * g.N;
@@ -198,6 +190,7 @@ void grouped_kernel(const GArgs a) {
             if (t < (long long)g.nd * g.Q) {
                 const int dd = (int)(t / g.Q), P = (int)(t % g.Q);
                 double s = 0.0;
+#pragma unroll 8
                 for (int q = 0; q < g.neg; ++q) s += g.gpart[((long long)q * g.nd + dd) * g.Q + P];
                 g.gamma[t] = s;
             }

@@ -251,6 +251,7 @@ __global__ void j_gamma_reduce_kernel(const double* __restrict__ gpart, int ngro
     if (t >= (int64_t)ND * Q) return;
     const int dd = (int)(t / Q), P = (int)(t % Q);
     double s = 0.0;
+#pragma unroll 8
     for (int g = 0; g < ngroups; ++g) s += gpart[((int64_t)g * ND + dd) * Q + P];
     gamma[t] = s;
 }
@@ -988,21 +989,6 @@ __device__ __forceinline__ void split_bf16_from_double(double x, __bf16& hi, __b
     float f = (float)x;
     asm volatile("" : "+v"(f));
     split_bf16(f, hi, lo);
-}
-
-// CpT[c][k] (hi/lo) = Cp[k][c] for c < OPAD, k < N; zero for N <= k < KP.
-__global__ void pad_ct_bf16_kernel(const double* __restrict__ C, int64_t ldc, int N, int nocc,
-                                   int width, int ioff, int KP, u16* __restrict__ Th,
-                                   u16* __restrict__ Tl) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)width * KP) return;
-    const int i = (int)(t / KP), k = (int)(t % KP);
-    const double x = (i < nocc && k < N) ? C[(int64_t)k * ldc + i] : 0.0;
-    __bf16 h, l;
-    split_bf16_from_double(x, h, l);
-    const int64_t o = (int64_t)(ioff + i) * KP + k;
-    Th[o] = __builtin_bit_cast(u16, h);
-    Tl[o] = __builtin_bit_cast(u16, l);
 }
 
 // KX (bf16x3): X[r][c] = sum_k A[r][k] Ct[c][k]
@@ -1766,16 +1752,6 @@ __global__ __launch_bounds__(256) void k_reduce_kernel(const double* __restrict_
     const int nb = (N + 15) / 16, m4 = blockIdx.x / nb, n16 = blockIdx.x % nb;
     if (n16 * 16 > m4 * 4 + 3) return;
     k_reduce_body(Kpart + blockIdx.y * dstride, nsplit, N, K.p[blockIdx.y], m4, n16);
-}
-
-// Cp[n][ioff + i] = C[n][i] (i < nocc), zero for nocc <= i < width.
-template <typename T>
-__global__ void pad_c_kernel(const double* __restrict__ C, int64_t ldc, int N, int nocc,
-                             int width, int ioff, int OPAD, T* __restrict__ Cp) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)N * width) return;
-    const int n = (int)(t / width), i = (int)(t % width);
-    Cp[(int64_t)n * OPAD + ioff + i] = (i < nocc) ? (T)C[(int64_t)n * ldc + i] : T(0);
 }
 
 }  // namespace f2jk
