@@ -302,7 +302,7 @@ DTiles dtile_plan(int N, int64_t Pc, int width, int slots) {
     m.cnt[2] = m.nt - 1;
     m.cnt[3] = 1;
     const double cost[4] = {16, 1.6 * 9, 4.0 * ((m.rl + 1) / 2), 1.6 * ((m.rl * (m.rl + 1) / 2 + 3) / 4)};
-    const double unit_us = 0.225 * (double)cdiv(width, kDK);  // one block for one P, two workgroups on the CU
+    const double unit_us = 0.225 * (double)width / kDK;  // one block for one P, two workgroups on the CU
     double sum = 0;
     for (int k = 0; k < 4; ++k) sum += m.cnt[k] * cost[k];
     double best = -1;

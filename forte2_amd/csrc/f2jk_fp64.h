@@ -498,33 +498,35 @@ __device__ __forceinline__ void ksd_body(char* lds, const double* __restrict__ X
         const int lrow = qrow[q] + lr < N ? lr : N - 1 - qrow[q];
         qoff[q] = (uint32_t)(lrow * OPAD + 2 * lg) * 8;
     });
-    const int h0 = wid & 1;
-    const int nkp = (width + kDK - 1) / kDK;  // steps per P; the last one is half when width % 16 == 8
-    const bool tail = width % kDK != 0;
-    auto load = [&](int P, int kt, int stg) {
-        if (tail && kt == nkp - 1 && h0) return;
-        const double* XP = X + (int64_t)P * N * OPAD + ioff + kt * kDK + 8 * h0;
-        const uint32_t l0 = lds_addr(lds) + stg * STAGE;
-        static_for<0, 8>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            if (qon[q]) lds_load16(uniform_ptr(XP + (int64_t)qrow[q] * OPAD), qoff[q], l0 + (wid + 4 * q) * 1024);
-        });
+    // The k range runs in halves of 8 through the P of the split, one after the
+    // other, and a step is any two of them: with steps that ended with their P,
+    // an odd number of halves cost a half-empty step per P (nbf 318, 3 halves
+    // per density: 109 us, the matrix pipes 44% busy).
+    const int hp = width >> 3, nh = (Pb - Pa) * hp, nsteps = (nh + 1) >> 1;
+    int Pn = Pa, kn = wid & 1, ln = wid & 1;  // the half this wave loads next: its P, place in P, number
+    while (kn >= hp) kn -= hp, ++Pn;
+    auto load = [&](int stg) {
+        if (ln < nh) {
+            const double* XP = X + (int64_t)Pn * N * OPAD + ioff + 8 * kn;
+            const uint32_t l0 = lds_addr(lds) + stg * STAGE;
+            static_for<0, 8>([&](auto Q) {
+                constexpr int q = decltype(Q)::value;
+                if (qon[q]) lds_load16(uniform_ptr(XP + (int64_t)qrow[q] * OPAD), qoff[q], l0 + (wid + 4 * q) * 1024);
+            });
+        }
+        ln += 2;
+        kn += 2;
+        while (kn >= hp) kn -= hp, ++Pn;
     };
-
-    const int nsteps = (Pb - Pa) * nkp;
     // the steps of the P range, one after the other: compute(LDS of the step at
     // this lane's slot, halves of the step)
     auto sweep = [&](auto&& compute) {
-        int kt = 0;           // the step being computed, of its P
-        int Pn = Pa, kn = 0;  // the step being loaded
-        if (nsteps > 0) load(Pa, 0, 0);
+        load(0);
         drain_and_barrier();
         for (int st = 0; st < nsteps; ++st) {
             const int cur = st & 1;
-            if (++kn == nkp) kn = 0, ++Pn;
-            if (st + 1 < nsteps) load(Pn, kn, cur ^ 1);
-            compute(lds + cur * STAGE + lane * 16, tail && kt == nkp - 1 ? 1 : 2);
-            kt = kn;
+            if (st + 1 < nsteps) load(cur ^ 1);
+            compute(lds + cur * STAGE + lane * 16, min(2, nh - 2 * st));
             __builtin_amdgcn_sched_barrier(0);  // no MFMA moves past the drain
             drain_and_barrier();
         }
@@ -552,8 +554,8 @@ __device__ __forceinline__ void ksd_body(char* lds, const double* __restrict__ X
         for (int i = 0; i < NI; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc[i][j] = dx4{0, 0, 0, 0};
-        sweep([&](const char* L, int nh) {
-            for (int h = 0; h < nh; ++h) {
+        sweep([&](const char* L, int halves) {
+            for (int h = 0; h < halves; ++h) {
                 dx2 a[NI > 0 ? NI : 1], c[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) c[j] = frag(L, 8 + j0 + j, h);
@@ -591,8 +593,8 @@ __device__ __forceinline__ void ksd_body(char* lds, const double* __restrict__ X
         dx4 acc[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) acc[i] = dx4{0, 0, 0, 0};
-        sweep([&](const char* L, int nh) {
-            for (int h = 0; h < nh; ++h) {
+        sweep([&](const char* L, int halves) {
+            for (int h = 0; h < halves; ++h) {
                 static_for<0, 3>([&](auto U) {  // three blocks at a time: consecutive MFMAs on different ones
                     constexpr int u = 3 * decltype(U)::value;
                     dx2 a[3], c[3];
