@@ -713,8 +713,8 @@ def main():
         print(f"[bench] cpu baseline: {cpu['value']:.4f} builds/s on {cpu['cores']} cores",
               file=sys.stderr, flush=True)
     # the BF16x3 half-transform runs in 256-row tiles (kx_bf16x3_tall_kernel)
-    # unless the launch shape says 128 (the library's rule: 256 for nbf >= 768)
-    rows = fb.knobs.get("kx_rows", 0) or (256 if N >= 768 and N % 4 == 0 else 128)
+    # unless the launch shape says 128 (the library's rule: 256 for nbf >= 192)
+    rows = fb.knobs.get("kx_rows", 0) or (256 if N >= 192 and N % 4 == 0 else 128)
     kx_name = "kx_bf16x3_tall_kernel" if rows == 256 else "kx_bf16x3_kernel"
     if args.mixed != "bf16x3":
         # FP32: 320-column tiles above 128 occupied columns (the library's rule)
