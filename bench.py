@@ -701,7 +701,8 @@ def main():
     k_ms = ph_mix["kx"] + ph_mix["ks"] + ph_mix["k_reduce"]
     k64_ms = ph64["kx"] + ph64["ks"] + ph64["k_reduce"]
     j_ms = ph_mix["j_gamma"] + ph_mix["j_acc"]
-    j64_ms = ph64["j_gamma"] + ph64["j_acc"]
+    # FP64 J and K from C read B once for J: gamma comes with the half-transform
+    jb64, j64_ms = jb64 / 2, ph64["j_acc"]
 
     peaks = measured_peaks(read_buf=fb.B_fp32())
     mpeak = peaks["mfma_bf16_TFLOPs" if args.mixed == "bf16x3" else "mfma_fp32_TFLOPs"]
