@@ -46,6 +46,12 @@ constexpr int kEPT = 4;                 // vector elements per thread in the J k
 constexpr int kJ1PerBlock = 32;         // P values per block in J pass 1
 constexpr int kTargetBlocks = 2048;     // blocks wanted per launch to fill 256 CUs
 constexpr size_t kDefaultXChunkBytes = size_t(4) << 30;
+// The threads of a launch are counted in 32 bits per dimension, and one more
+// wraps around without an error.  The FP64 half-transform has four threads per
+// row (wider rows than one column tile's fit no card at this count), the sum of
+// its row sums a wave per P.
+constexpr int64_t kMaxLaunchRows = int64_t(1) << 29;
+constexpr int64_t kMaxLaunchP = int64_t(1) << 25;
 
 size_t align_up(size_t x, size_t a = 256) { return (x + a - 1) / a * a; }
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -461,7 +467,8 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         const size_t per_p = (size_t)N * p.OPAD * p.tk + grow_p;
         int64_t pc = (int64_t)(xchunk_bytes / std::max<size_t>(per_p, 1));
         pc = std::max<int64_t>(1, std::min<int64_t>(pc, Q));
-        pc = std::min<int64_t>(pc, INT32_MAX / N);  // rows of a chunk are numbered in 32 bits
+        // rows of a chunk are numbered in 32 bits; grouped launches walk their blocks
+        pc = std::min<int64_t>(pc, grouped ? INT32_MAX / N : std::min(kMaxLaunchP, kMaxLaunchRows / N));
         p.per_p = per_p;
         // as many chunks as the cap needs, of balanced size: no short last
         // chunk whose launches would be all set-up and Kpart traffic
@@ -555,6 +562,12 @@ int tim_mark(f2jk_ctx* ctx, int phase, hipStream_t st, bool start) {
     } while (0)
 
 // --------------------------------------------------------------------------- J
+dim3 j_reduce_grid(int nvec) {
+    const int64_t nb = cdiv(nvec, kJRedElems), x = std::min<int64_t>(nb, 1 << 22);
+    return dim3((unsigned)x, (unsigned)cdiv(nb, x));
+}
+dim3 k_reduce_grid(int N, int nd) { return dim3((unsigned)cdiv(N, 16), (unsigned)cdiv(N, 4), nd); }
+
 // densities d0 .. d0 + ND - 1; without D, gamma is there already
 template <typename TB, int VEC, int ND, bool NT>
 int launch_j(f2jk_ctx* ctx, const Plan& p, const TB* B, int d0, const double* const* D, int64_t ldd,
@@ -596,8 +609,7 @@ int launch_j(f2jk_ctx* ctx, const Plan& p, const TB* B, int d0, const double* co
     hipLaunchKernelGGL((j_accum_kernel<TB, VEC, kEPT, ND, NT>), dim3(p.neg, p.npc2), dim3(kJThreads), 0,
                        st, B, p.N, p.Q, gamma, rowoff, elist, (const TB*)p.jpacked, p.nvec, p.ppw2, jpart);
     F2JK_LAUNCHED("j_accum");
-    hipLaunchKernelGGL((j_reduce_kernel<VEC, ND>), dim3((unsigned)cdiv(p.jdense, kJRedElems)), dim3(kJThreads), 0,
-                       st, jpart, p.npc2, p.N, rowoff, p.jinv, p.nvec, p.jdense, jp);
+    hipLaunchKernelGGL((j_reduce_kernel<VEC, ND>), j_reduce_grid(p.jdense), dim3(kJThreads), 0, st, jpart, p.npc2, p.N, rowoff, p.jinv, p.nvec, p.jdense, jp);
     F2JK_LAUNCHED("j_reduce");
     TIM(F2JK_PH_JACC, false);
     return F2JK_OK;
@@ -807,7 +819,7 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const
         TIM(F2JK_PH_KX, false);
         if (p.gamma_x && !p.small) {
             TIM(F2JK_PH_JGAMMA, true);
-            hipLaunchKernelGGL(gamma_rows_kernel, dim3((unsigned)cdiv((int64_t)p.nd * pc, 4)), dim3(256), 0, st,
+            hipLaunchKernelGGL(gamma_rows_kernel, dim3((unsigned)cdiv(pc, 4), p.nd), dim3(256), 0, st,
                                (const double*)(ws + p.off_grow), (int64_t)p.Pc * p.N, p.nd, p.dncolt, p.N, pc,
                                (double*)(ws + p.off_gamma) + P0, p.Q);
             F2JK_LAUNCHED("gamma_rows");
@@ -844,11 +856,11 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const
                                        : (v2 ? launch_jkred<2, 1> : launch_jkred<1, 1>);
             red(ctx, p, (const double*)(ws + p.off_jpart), J, kpart, (int64_t)p.nsplit * NN, kp, st);
         } else {
-            hipLaunchKernelGGL(kred_kernel, dim3(k_reduce_blocks(p.N), p.nd), dim3(256), 0, st, kpart,
+            hipLaunchKernelGGL(kred_kernel, k_reduce_grid(p.N, p.nd), dim3(256), 0, st, kpart,
                                (int64_t)p.nsplit * NN, p.dt, p.N, kp);
         }
     } else
-        hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N), p.nd), dim3(256), 0, st, kpart,
+        hipLaunchKernelGGL(k_reduce_kernel, k_reduce_grid(p.N, p.nd), dim3(256), 0, st, kpart,
                            (int64_t)p.nsplit * NN, nsplit_used, p.N, kp);
     F2JK_LAUNCHED("k_reduce");
     TIM(F2JK_PH_KRED, false);
@@ -960,7 +972,7 @@ int run_k_bf16x3(f2jk_ctx* ctx, const Plan& p, double* const* K, char* ws, hipSt
     const int nsplit_used = std::min(p.nsplit, std::min(p.Pc, p.Q));
     KPtrs kp{};
     for (int d = 0; d < p.nd; ++d) kp.p[d] = K[d];
-    hipLaunchKernelGGL(k_reduce_kernel, dim3(k_reduce_blocks(p.N), p.nd), dim3(256), 0, st, kpart,
+    hipLaunchKernelGGL(k_reduce_kernel, k_reduce_grid(p.N, p.nd), dim3(256), 0, st, kpart,
                        (int64_t)p.nsplit * NN, nsplit_used, p.N, kp);
     F2JK_LAUNCHED("k_reduce");
     TIM(F2JK_PH_KRED, false);
@@ -1619,7 +1631,7 @@ int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ld
     const double* B = (const double*)ctx->B[F2JK_F64];
     const double* cq = (const double*)(w + p.off_cq);
     const int64_t NN = (int64_t)p.N * p.N;
-    const int64_t step = INT32_MAX / p.N;  // rows of a launch are numbered in 32 bits
+    const int64_t step = kMaxLaunchRows / p.N;
     for (int64_t P0 = p0; P0 < p1; P0 += step) {
         const int64_t R = std::min<int64_t>(step, p1 - P0) * p.N;
         launch_kxd(p, B + P0 * NN, R, cq, X + (P0 - p0) * p.N * ldx, ldx, (int)ncol, KxdGamma{}, st);

@@ -400,9 +400,8 @@ __global__ __launch_bounds__(256, 2) void kxt_kernel(const double* __restrict__ 
 
 // gamma[d][P] = sum over column tiles and rows m of grow[ct * nd + d][P * N + m], one wave per (d, P)
 __device__ __forceinline__ void gamma_rows_body(const double* __restrict__ grow, int64_t gstride, int nd, int ncolt,
-                                                int N, int pc, double* __restrict__ gamma, int Q, int64_t t) {
-    if (t >= (int64_t)nd * pc) return;
-    const int d = (int)(t / pc), P = (int)(t % pc), lane = threadIdx.x & 63;
+                                                int N, double* __restrict__ gamma, int Q, int d, int P) {
+    const int lane = threadIdx.x & 63;
     double s = 0.0;
     for (int ct = 0; ct < ncolt; ++ct) {
         const double* g = grow + (int64_t)(ct * nd + d) * gstride + (int64_t)P * N;
@@ -413,7 +412,8 @@ __device__ __forceinline__ void gamma_rows_body(const double* __restrict__ grow,
 }
 __global__ __launch_bounds__(256) void gamma_rows_kernel(const double* __restrict__ grow, int64_t gstride, int nd,
                                                          int ncolt, int N, int pc, double* __restrict__ gamma, int Q) {
-    gamma_rows_body(grow, gstride, nd, ncolt, N, pc, gamma, Q, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int P = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (P < pc) gamma_rows_body(grow, gstride, nd, ncolt, N, gamma, Q, blockIdx.y, P);
 }
 
 // ---------------------------------------------------------------------------
@@ -642,9 +642,9 @@ __device__ __forceinline__ int dtile_splits(const DTiles& m, int m4, int n16) {
 }
 __global__ __launch_bounds__(256) void kred_kernel(const double* __restrict__ Kpart, int64_t dstride, DTiles tm,
                                                    int N, KPtrs K) {
-    const int nb = (N + 15) / 16, m4 = blockIdx.x / nb, n16 = blockIdx.x % nb;
+    const int m4 = blockIdx.y, n16 = blockIdx.x;
     if (n16 * 16 > m4 * 4 + 3) return;
-    k_reduce_body(Kpart + blockIdx.y * dstride, dtile_splits(tm, m4, n16), N, K.p[blockIdx.y], m4, n16);
+    k_reduce_body(Kpart + blockIdx.z * dstride, dtile_splits(tm, m4, n16), N, K.p[blockIdx.z], m4, n16);
 }
 
 // both reductions of a small build in one launch: nbj blocks of J, the rest K

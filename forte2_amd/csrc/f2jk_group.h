@@ -183,8 +183,10 @@ void grouped_kernel(const GArgs a) {
                 j_gamma_kernel_body<TB, 2, 4, 1, true>(B, g.N, g.Q, dp, g.N, g.rowoff, g.nvec, 32, g.gpart, bx, by);
             }
         } else if constexpr (PHASE == GP_GRED && PREC == F2JK_PREC_FP64) {
-            gamma_rows_body(g.grow, (long long)g.Q * g.N, g.nd, g.dncolt, g.N, g.Q, g.gamma, g.Q,
-                            (long long)local * 4 + (tid >> 6));
+            const long long t = (long long)local * 4 + (tid >> 6);
+            if (t < (long long)g.nd * g.Q)
+                gamma_rows_body(g.grow, (long long)g.Q * g.N, g.nd, g.dncolt, g.N, g.gamma, g.Q, (int)(t / g.Q),
+                                (int)(t % g.Q));
         } else if constexpr (PHASE == GP_GRED) {
             const long long t = (long long)local * 256 + tid;
             if (t < (long long)g.nd * g.Q) {

@@ -422,7 +422,7 @@ __global__ __launch_bounds__(kJThreads) void j_reduce_kernel(const double* __res
                                                              const int* __restrict__ rowoff,
                                                              const int* __restrict__ jinv, int nlist, int nvec,
                                                              JPtrs<ND> J) {
-    j_reduce_body<VEC, ND>(jpart, nchunks, N, rowoff, jinv, nlist, nvec, J, blockIdx.x);
+    j_reduce_body<VEC, ND>(jpart, nchunks, N, rowoff, jinv, nlist, nvec, J, blockIdx.y * gridDim.x + blockIdx.x);
 }
 
 // flag[e] = 1 when B[P][m][c] != 0 for some P and some c <= m of vector
@@ -1746,12 +1746,12 @@ __host__ __device__ inline int k_reduce_blocks(int N) { return ((N + 3) / 4) * (
 struct KPtrs {
     double* p[8];
 };
-// grid (k_reduce_blocks(N), densities); the partials of one density are dstride doubles
+// grid (16-column blocks, 4-row blocks, densities); the partials of one density are dstride doubles
 __global__ __launch_bounds__(256) void k_reduce_kernel(const double* __restrict__ Kpart, int64_t dstride, int nsplit,
                                                        int N, KPtrs K) {
-    const int nb = (N + 15) / 16, m4 = blockIdx.x / nb, n16 = blockIdx.x % nb;
+    const int m4 = blockIdx.y, n16 = blockIdx.x;
     if (n16 * 16 > m4 * 4 + 3) return;
-    k_reduce_body(Kpart + blockIdx.y * dstride, nsplit, N, K.p[blockIdx.y], m4, n16);
+    k_reduce_body(Kpart + blockIdx.z * dstride, nsplit, N, K.p[blockIdx.z], m4, n16);
 }
 
 }  // namespace f2jk
