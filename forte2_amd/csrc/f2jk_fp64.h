@@ -251,9 +251,15 @@ __device__ __forceinline__ void kxd_body(char* lds, const double* __restrict__ A
 #pragma unroll
                 for (int j = 0; j < NB; ++j) {
                     const double x = cr[j * 16];
-                    if constexpr (decltype(masked)::value)
-                        s = fma(acc[i][j][r], c0 + j * 16 >= lo && c0 + j * 16 < hi ? x : 0.0, s);
-                    else
+                    if constexpr (decltype(masked)::value) {
+                        // the lanes of the density alone: its neighbour's sums may be
+                        // infinite, and zero times them is not zero.  Kept a branch: as
+                        // selects the copies of a whole row took up to 60 registers more
+                        if ((uint32_t)(c0 + j * 16 - lo) < (uint32_t)(hi - lo)) {
+                            s = fma(acc[i][j][r], x, s);
+                            asm volatile("" : "+v"(s));
+                        }
+                    } else
                         s = fma(acc[i][j][r], x, s);
                 }
 #pragma unroll
