@@ -192,6 +192,22 @@ int pack_jlist(f2jk_ctx* ctx, int dtype, const TB* B) {
     return F2JK_OK;
 }
 
+// the values of copy `dtype` into its packed elements
+int pack_elements(f2jk_ctx* ctx, int dtype) {
+    const int vec = ctx->jlist_vec[dtype];
+    int rc;
+    if (dtype == F2JK_F64)
+        rc = vec == 2 ? pack_jlist<double, 2>(ctx, dtype, (const double*)ctx->B[dtype])
+                      : pack_jlist<double, 1>(ctx, dtype, (const double*)ctx->B[dtype]);
+    else
+        rc = vec == 4 ? pack_jlist<float, 4>(ctx, dtype, (const float*)ctx->B[dtype])
+           : vec == 2 ? pack_jlist<float, 2>(ctx, dtype, (const float*)ctx->B[dtype])
+                      : pack_jlist<float, 1>(ctx, dtype, (const float*)ctx->B[dtype]);
+    if (rc) return rc;
+    F2JK_HIP(hipStreamSynchronize(nullptr));  // builds on any stream read it
+    return F2JK_OK;
+}
+
 // The packed elements of copy `dtype`, where they save bytes and a sixteenth of
 // the free memory holds them (a build that just fits the card keeps its room;
 // the passes give the same J, bitwise, either way).
@@ -209,17 +225,7 @@ int build_jpacked(f2jk_ctx* ctx, int dtype) {
         ctx->jpacked[dtype] = nullptr;
         return F2JK_OK;
     }
-    int rc;
-    if (dtype == F2JK_F64)
-        rc = vec == 2 ? pack_jlist<double, 2>(ctx, dtype, (const double*)ctx->B[dtype])
-                      : pack_jlist<double, 1>(ctx, dtype, (const double*)ctx->B[dtype]);
-    else
-        rc = vec == 4 ? pack_jlist<float, 4>(ctx, dtype, (const float*)ctx->B[dtype])
-           : vec == 2 ? pack_jlist<float, 2>(ctx, dtype, (const float*)ctx->B[dtype])
-                      : pack_jlist<float, 1>(ctx, dtype, (const float*)ctx->B[dtype]);
-    if (rc) return rc;
-    F2JK_HIP(hipStreamSynchronize(nullptr));  // builds on any stream read it
-    return F2JK_OK;
+    return pack_elements(ctx, dtype);
 }
 
 void free_jlist(f2jk_ctx* ctx, int dtype) {
@@ -1028,6 +1034,9 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
     }
     F2JK_HIP(hipSetDevice(ctx->device));
     hipStream_t st = (hipStream_t)stream;
+    // a captured build reads B itself: its replays see values written later, and
+    // do not depend on memory that "j_pack" may have given back by then
+    if (p.jpacked && capturing(st)) p.jpacked = nullptr;
     char* w = (char*)ws;
     tim_begin(ctx, flags & F2JK_TIMING);
     TIM(F2JK_PH_TOTAL, true);
@@ -1349,9 +1358,15 @@ int f2jk_set_tuning(f2jk_ctx* ctx, const char* key, int64_t value) {
         }
     } else if (!strcmp(key, "j_pack")) {
         ctx->j_pack = value != 0;
-        if (ctx->j_sparse) {
-            int rc = build_jlist(ctx, F2JK_F32);
+        F2JK_HIP(hipSetDevice(ctx->device));
+        if (ctx->j_pack && ctx->jlist[F2JK_F32]) {
+            F2JK_HIP(hipDeviceSynchronize());  // builds that read them, writes to B on any stream
+            int rc = ctx->jpacked[F2JK_F32] ? pack_elements(ctx, F2JK_F32) : build_jpacked(ctx, F2JK_F32);
             if (rc) return rc;
+        } else if (!ctx->j_pack && ctx->jpacked[F2JK_F32]) {
+            F2JK_HIP(hipDeviceSynchronize());
+            (void)hipFree(ctx->jpacked[F2JK_F32]);
+            ctx->jpacked[F2JK_F32] = nullptr;
         }
     } else if (!strcmp(key, "ks_dma")) {
         if (value < -1 || value > 1) return fail(F2JK_EINVAL, "ks_dma must be -1, 0 or 1");

@@ -59,6 +59,7 @@ class FockBuilder:
         self.device = _device_of(device)
         self._B64 = None
         self._B32 = None
+        self._B32_version = None  # writes to it that its packed elements include
         self._ctx = None
         self._ws = None
         self._manual = set()  # launch-shape knobs set by hand
@@ -113,11 +114,30 @@ class FockBuilder:
                                                     stats=self.B_stats))
         return self._B64
 
+    def _packable_version(self):
+        """torch's count of the writes to the FP32 copy; None where it keeps none
+        (a tensor made in inference mode): such a copy is not packed."""
+        return None if self._B32.is_inference() else self._B32._version
+
+    def _repack(self):
+        """Pack the listed elements again if the copy was written in place since
+        (captured builds read the copy itself)."""
+        v = self._packable_version()
+        if v != self._B32_version and not torch.cuda.is_current_stream_capturing():
+            self._B32_version = v
+            if self.knobs.get("j_pack"):
+                self._tune("j_pack", 1)
+
     def B_fp32(self):
-        """The FP32 copy of B used by the fp32/bf16x3 precision forms."""
+        """The FP32 copy of B used by the fp32/bf16x3 precision forms.  It may be
+        written in place with torch operations (its zero pattern stays): the next
+        build uses the new values."""
         if self._B32 is None:
             self._B32 = self.B_Pmn.to(torch.float32)
+            self._B32_version = self._packable_version()
             if self._ctx is not None:
+                if self.j_sparse and self._B32_version is None and "j_pack" not in self._manual:
+                    self._tune("j_pack", 0)
                 self._register(nat.F2JK_F32, self._B32)
         return self._B32
 
@@ -136,8 +156,9 @@ class FockBuilder:
             # fixed once formed; the scan happens here and when the FP32 copy
             # is registered)
             if self.j_sparse:
-                # the FP32 copy is this builder's own: its listed elements may be packed
-                self._tune("j_pack", 1)
+                # the listed elements of the FP32 copy are packed, and packed again
+                # after a write to it
+                self._tune("j_pack", int(self._B32 is None or self._B32_version is not None))
                 self._tune("j_sparse", 1)
         return self._ctx
 
@@ -200,6 +221,7 @@ class FockBuilder:
             raise ValueError(f"unknown precision {p!r}")
         if p != "fp64":
             self.B_fp32()
+            self._repack()
         self._apply_table(p)
         return nat.PREC[p]
 

@@ -124,8 +124,9 @@ int f2jk_get_shape(const f2jk_ctx* ctx, int64_t* naux, int64_t* nbf);
  * listed elements of the F32 copy are also kept one after the other in
  * memory of the library (where they are less than 85% of the lower triangle
  * and a sixteenth of the free device memory holds them), so that the J passes
- * read whole lines; the same J, bitwise.  The copy's values must then not
- * change while registered either.
+ * read whole lines; the same J, bitwise.  After writing to the copy's values,
+ * set "j_pack" to 1 again: that packs them anew in the same memory
+ * (synchronises the device).  Builds being captured read the copy itself.
  * Set by the autotuner. */
 int f2jk_set_tuning(f2jk_ctx* ctx, const char* key, int64_t value);
 
