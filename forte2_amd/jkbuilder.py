@@ -16,6 +16,7 @@ import ctypes
 
 import numpy as np
 import torch
+import torch.autograd.forward_ad as fwad
 
 from . import _native as nat
 
@@ -29,6 +30,11 @@ def _device_of(device):
     if d.index is None:
         d = torch.device("cuda", torch.cuda.current_device())
     return d
+
+
+def _traced(x):
+    """Whether torch records derivatives in x, backward or forward."""
+    return (torch.is_grad_enabled() and x.requires_grad) or fwad.unpack_dual(x).tangent is not None
 
 
 class FockBuilder:
@@ -424,12 +430,20 @@ class FockBuilder:
     def B_tensor_gen_block(self, C1, C2):
         """B[P, i, j] = sum_mn B_Pmn C1_mi C2_nj: the MO-basis B tensor
         (jkbuilder.py:521-552), both contractions on MFMA (f2jk_mo_block), the
-        narrower set first.  Real orbitals (conj is the identity)."""
+        narrower set first.  Real orbitals (conj is the identity).  Where torch
+        records derivatives in C1, they pass through (those in C2 do not)."""
         self.B_Pmn
         c1, to_np = self._as_dev(C1)
         c2, to_np2 = self._as_dev(C2)
         if c1.dim() != 2 or c2.dim() != 2 or c1.shape[0] != self.nbf or c2.shape[0] != self.nbf:
             raise ValueError(f"C1 and C2 must have {self.nbf} rows")
+        if _traced(c1):  # derivatives in C1: its product is torch's
+            out = torch.empty((self.naux, c1.shape[1], c2.shape[1]), dtype=torch.float64, device=self.device)
+            if out.numel():
+                c1t = c1.T.contiguous()
+                for P0, P1, X in self._x_blocks(c2):
+                    out[P0:P1] = torch.matmul(c1t, X)
+            return out.cpu().numpy() if to_np2 else out
         if c1.shape[1] > self.nbf:  # the kernels take at most nbf columns at a time
             out = torch.cat([self.B_tensor_gen_block(c1[:, i:i + self.nbf], c2)
                              for i in range(0, c1.shape[1], self.nbf)], 1)
