@@ -469,8 +469,10 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         off += p.jpart_bytes;
     }
     if (p.want_k) {
+        // the row sums come beside X and not out of its cap: J does not change the
+        // chunks of K, and a grouped job whose X fits stays one chunk
+        const size_t per_p = (size_t)N * p.OPAD * p.tk;
         const size_t grow_p = p.gamma_x ? (size_t)p.dncolt * ndens * N * 8 : 0;
-        const size_t per_p = (size_t)N * p.OPAD * p.tk + grow_p;
         int64_t pc = (int64_t)(xchunk_bytes / std::max<size_t>(per_p, 1));
         pc = std::max<int64_t>(1, std::min<int64_t>(pc, Q));
         // rows of a chunk are numbered in 32 bits; grouped launches walk their blocks
@@ -524,7 +526,7 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         else
             p.kva = (N % 4 == 0) ? 4 : ((N % 2 == 0) ? 2 : 1);
         p.off_x = off;
-        p.x_bytes = align_up((size_t)p.Pc * (per_p - grow_p));
+        p.x_bytes = align_up((size_t)p.Pc * per_p);
         off += p.x_bytes;
         p.off_grow = off;
         off += align_up((size_t)p.Pc * grow_p);
