@@ -1404,10 +1404,16 @@ int f2jk_set_tuning(f2jk_ctx* ctx, const char* key, int64_t value) {
 int f2jk_workspace_size(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision, int flags,
                         size_t* bytes) {
     if (!ctx || !bytes) return fail(F2JK_EINVAL, "null argument");
-    Plan p;
-    // a build_jk plan (J from C) is the largest; use it whenever C is known
+    Plan p, j;
     int rc = make_plan(ctx, ndens, nocc, precision, flags, nocc != nullptr, p);
     if (rc) return rc;
+    // J and K in FP64 keep neither D nor the partial gamma, which J alone has:
+    // the size is enough for that too (K alone needs less as it is)
+    if (p.gamma_x) {
+        rc = make_plan(ctx, ndens, nocc, precision, flags & ~F2JK_WANT_K, true, j);
+        if (rc) return rc;
+    }
+    p.total = std::max(p.total, j.total);
     *bytes = p.total;
     return F2JK_OK;
 }

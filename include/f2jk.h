@@ -130,7 +130,8 @@ int f2jk_get_shape(const f2jk_ctx* ctx, int64_t* naux, int64_t* nbf);
  * Set by the autotuner. */
 int f2jk_set_tuning(f2jk_ctx* ctx, const char* key, int64_t value);
 
-/* Scratch bytes needed by f2jk_build_jk / _j / _k for these arguments.
+/* Scratch bytes needed by f2jk_build_jk / _j / _k for these arguments.  The
+ * size of J and K together (both flags) is enough for either alone.
  * nocc may be NULL when flags has no F2JK_WANT_K and no F2JK_WANT_J with C. */
 int f2jk_workspace_size(const f2jk_ctx* ctx, int ndens, const int64_t* nocc,
                         int precision, int flags, size_t* bytes);
