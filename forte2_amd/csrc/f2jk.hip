@@ -11,6 +11,7 @@
 
 #include "f2jk.h"
 #include "f2jk_kernels.h"
+#include "f2jk_tiles.h"
 #include "f2jk_fp64.h"
 #include "f2jk_group.h"
 
@@ -502,17 +503,7 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
             p.kx_rows = 128;
             if (!grouped) p.kx_rows = ctx->kx_rows ? ctx->kx_rows : (N >= 192 ? 256 : 128);
             if (N % 4 || N < 32) p.kx_rows = 128;  // the tall kernel loads A rows 16 bytes at a time
-            // the tile width (in 32-column units) within the cap that computes
-            // the fewest column blocks; ties go to the wider tile
-            const int need = (int)cdiv(p.OPAD, 32);
-            int best = 0, cost = 0;
-            for (int w : {10, 8, 7, 6, 5, 4, 3, 2, 1}) {
-                if (w > ctx->bf16_nbw_max) continue;
-                if (p.kx_rows == 128 && (w == 7 || w == 3 || w == 1)) continue;
-                const int c = (int)cdiv(need, w) * w;
-                if (best == 0 || c < cost) best = w, cost = c;
-            }
-            p.nbw = best;
+            p.nbw = bf16_tile_units((int)cdiv(p.OPAD, 32), ctx->bf16_nbw_max, p.kx_rows);
             p.kx_waves = ctx->kx_waves;
             p.ncolt = (int)cdiv(p.OPAD, 32 * p.nbw);
         } else if (precision == F2JK_PREC_FP32) {
