@@ -1001,10 +1001,10 @@ bool capturing(hipStream_t st) {
     return status != hipStreamCaptureStatusNone;
 }
 
-int check_ws(const Plan& p, void* ws, size_t ws_bytes) {
+int check_ws(size_t need, void* ws, size_t ws_bytes) {
     if (!ws) return fail(F2JK_EINVAL, "workspace pointer is NULL");
-    if (ws_bytes < p.total)
-        return fail(F2JK_ENOMEM, "workspace too small: need " + std::to_string(p.total) + " bytes, got " +
+    if (ws_bytes < need)
+        return fail(F2JK_ENOMEM, "workspace too small: need " + std::to_string(need) + " bytes, got " +
                                      std::to_string(ws_bytes));
     if (((uintptr_t)ws) % 256) return fail(F2JK_EINVAL, "workspace must be 256-byte aligned");
     return F2JK_OK;
@@ -1019,7 +1019,7 @@ int build_common(f2jk_ctx* ctx, int ndens, const double* const* C, const int64_t
     int rc = make_plan(ctx, ndens, nocc, precision, flags, j_from_c, p, 0, false, caps);
     if (rc) return rc;
     p.no_alloc = no_alloc;
-    if ((rc = check_ws(p, ws, ws_bytes))) return rc;
+    if ((rc = check_ws(p.total, ws, ws_bytes))) return rc;
     for (int d = 0; d < ndens; ++d) {
         if (p.want_j && !J[d]) return fail(F2JK_EINVAL, "J output pointer is NULL");
         if (p.want_k && !K[d]) return fail(F2JK_EINVAL, "K output pointer is NULL");
@@ -1532,7 +1532,7 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
     int64_t k = 0;
     for (int j = 0; j < njobs; ++j) {
         const Plan& p = plans[j];
-        if ((rc = check_ws(p, ws[j], ws_bytes[j]))) return rc;
+        if ((rc = check_ws(p.total, ws[j], ws_bytes[j]))) return rc;
         if (want_j && (rc = ensure_rowoff(ctxs[j], p.jvec))) return rc;
         char* w = (char*)ws[j];
         GJob& g = jobs[j];
@@ -1625,6 +1625,18 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
     return F2JK_OK;
 }
 
+// The packed coefficients of a plan are all that the half-transform keeps in its
+// workspace (they come first): X goes to the caller's array.
+int f2jk_half_transform_workspace_size(const f2jk_ctx* ctx, int64_t ncol, size_t* bytes) {
+    if (!ctx || !bytes) return fail(F2JK_EINVAL, "null argument");
+    if (ncol < 1) return fail(F2JK_EINVAL, "ncol must be >= 1");
+    Plan p;
+    int rc = make_plan(ctx, 1, &ncol, F2JK_PREC_FP64, F2JK_WANT_K, false, p);
+    if (rc) return rc;
+    *bytes = p.off_x;
+    return F2JK_OK;
+}
+
 int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ldc, int64_t p0, int64_t p1,
                         double* X, int64_t ldx, int precision, void* ws, size_t ws_bytes, void* stream) {
     if (!ctx) return fail(F2JK_EINVAL, "null context");
@@ -1635,7 +1647,7 @@ int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ld
     int rc = make_plan(ctx, 1, &ncol, precision, F2JK_WANT_K, false, p);
     if (rc) return rc;
     if (p0 < 0 || p1 > p.Q || p0 >= p1) return fail(F2JK_EINVAL, "aux range [p0, p1) invalid");
-    if ((rc = check_ws(p, ws, ws_bytes))) return rc;
+    if ((rc = check_ws(p.off_x, ws, ws_bytes))) return rc;
     F2JK_HIP(hipSetDevice(ctx->device));
     hipStream_t st = (hipStream_t)stream;
     char* w = (char*)ws;
@@ -1706,9 +1718,7 @@ int f2jk_mo_block(f2jk_ctx* ctx, const double* C1, int64_t n1, int64_t ld1, cons
     MoPlan m;
     int rc = mo_plan(ctx, n1, n2, m);
     if (rc) return rc;
-    if (!ws) return fail(F2JK_EINVAL, "workspace pointer is NULL");
-    if (ws_bytes < m.total) return fail(F2JK_ENOMEM, "workspace too small");
-    if (((uintptr_t)ws) % 256) return fail(F2JK_EINVAL, "workspace must be 256-byte aligned");
+    if ((rc = check_ws(m.total, ws, ws_bytes))) return rc;
     F2JK_HIP(hipSetDevice(ctx->device));
     hipStream_t st = (hipStream_t)stream;
     const double* C[2] = {C1, C2};

@@ -409,8 +409,7 @@ class FockBuilder:
         elif tuple(out.shape) != shape or out.dtype != torch.float64 or not out.is_contiguous():
             raise ValueError(f"out must be a contiguous float64 tensor of shape {shape}")
         nbytes = ctypes.c_size_t()
-        nat.jk_check(lib.f2jk_workspace_size(self.ctx, 1, nat.i64_array([ncol]), nat.PREC["fp64"], nat.F2JK_WANT_K,
-                                             ctypes.byref(nbytes)), "workspace")
+        nat.jk_check(lib.f2jk_half_transform_workspace_size(self.ctx, ncol, ctypes.byref(nbytes)), "workspace")
         ws = self._workspace(nbytes.value)
         nat.jk_check(lib.f2jk_half_transform(self.ctx, ctypes.c_void_p(t.data_ptr()), ncol, ld, p0, p1,
                                              ctypes.c_void_p(out.data_ptr()), ncol, nat.PREC["fp64"],

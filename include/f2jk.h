@@ -217,11 +217,13 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens,
                         void* const* ws, const size_t* ws_bytes, void* stream);
 
 /* Half-transform X[P-p0][m][i] = sum_n B[P][m][n] C[n][i] for p0 <= P < p1,
- * i < ncol, into the caller's X ((p1-p0)*nbf rows, row stride ldx), FP64.  The first step of
- * FockBuilder.B_tensor_gen_block (forte2/jkbuilder/jkbuilder.py:521-552),
- * whose einsum "Pmn,mi,nj->Pij" f2jk_mo_block computes whole; two_electron_integrals_gen_block (:382-420) contracts two such blocks
- * over P.  Workspace: f2jk_workspace_size(ctx, 1, &ncol, FP64, F2JK_WANT_K).  With ldx equal
- * to ncol rounded up to 16 the kernel writes X in place (no copy). */
+ * i < ncol, straight into the caller's X ((p1-p0)*nbf rows, row stride ldx >=
+ * ncol), FP64.  The first step of FockBuilder.B_tensor_gen_block
+ * (forte2/jkbuilder/jkbuilder.py:521-552), whose einsum "Pmn,mi,nj->Pij"
+ * f2jk_mo_block computes whole; two_electron_integrals_gen_block (:382-420)
+ * contracts two such blocks over P.  Workspace (the packed coefficients):
+ * f2jk_half_transform_workspace_size. */
+int f2jk_half_transform_workspace_size(const f2jk_ctx* ctx, int64_t ncol, size_t* bytes);
 int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ldc, int64_t p0,
                         int64_t p1, double* X, int64_t ldx, int precision, void* ws, size_t ws_bytes,
                         void* stream);
