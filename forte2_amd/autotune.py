@@ -18,16 +18,19 @@ the launch shape:
     into LDS is bitwise the register-staged one and is used with the
     256-wide tiles, where it measured faster;
   * ``kx_rows`` (BF16x3, single-job): 128 or 256, the rows of a
-    half-transform tile (256: the tall kernel, 2 x 4 waves, even widths);
+    half-transform tile (256: the tall kernel, the library's choice from nbf
+    192 on);
   * ``ks_tile`` (BF16x3, single-job): 128 or 256, the lower-tile edge of the
     contraction.
 
 ``tune(shapes)`` times every candidate on synthetic B of each shape with HIP
-events and keeps the fastest; ``tune_grouped(shapes)`` does the same for a
+events around the build (its schedule as in a program) and keeps the fastest; ``tune_grouped(shapes)`` does the same for a
 grouped build of several jobs of one shape, timed through the serving layer's
 group path (the shapes the server batches).  ``save``/``load`` keep the table
 as JSON (``forte2_amd/data/tuning_gfx950.json`` ships the table measured on an
-MI355X).  ``apply(fb, precision, grouped=...)`` sets the entry of the nearest
+MI355X; its times are those of its settings with the present kernels, the
+settings themselves were ranked before the FP64 kernels of f2jk_fp64.h and
+before the 256-row half-transform ran below nbf 768).  ``apply(fb, precision, grouped=...)`` sets the entry of the nearest
 tuned size class on a FockBuilder.  Candidates change only the decomposition:
 every candidate gives the same J/K up to the reduction order (parity is tested
 separately), and a given table gives bitwise-stable results.
@@ -66,6 +69,7 @@ def _noccs(o):
 
 
 KS_TILE_MIN_NBF = 512  # below this a 256-wide contraction tile is mostly empty: not offered
+KX_ROWS_MIN_NBF = 192  # below this the library runs the 128-row half-transform
 
 
 def _candidates(precision, grouped, nbf=None):
@@ -75,7 +79,9 @@ def _candidates(precision, grouped, nbf=None):
         if not grouped:  # grouped builds use 4-wave half-transform and 128-wide contraction tiles
             names.append("kx_waves")
             if nbf is None or nbf >= KS_TILE_MIN_NBF:
-                names += ["ks_tile", "kx_rows"]
+                names.append("ks_tile")
+            if nbf is None or nbf >= KX_ROWS_MIN_NBF:
+                names.append("kx_rows")
     pools = {**CANDIDATES, "xchunk_bytes": XCHUNK_BF16 if precision == "bf16x3" else CANDIDATES["xchunk_bytes"]}
     for vals in itertools.product(*[pools[n] for n in names]):
         cand = dict(zip(names, vals))
@@ -87,6 +93,19 @@ def _candidates(precision, grouped, nbf=None):
 def _set(fb, cand):
     for k, v in cand.items():
         fb.set_tuning(k, v)
+
+
+def _build_ms(fb, Cs, prec):
+    """Time of one build as a program runs it: events around it, and not its own
+    phase events, which keep J off the side stream."""
+    import torch
+
+    t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    t0.record()
+    fb.build_JK(Cs, precision=prec)
+    t1.record()
+    t1.synchronize()
+    return t0.elapsed_time(t1)
 
 
 def tune(shapes, precisions=("fp64",), reps=3, device=None, log=print):
@@ -106,17 +125,11 @@ def tune(shapes, precisions=("fp64",), reps=3, device=None, log=print):
             best = None
             for cand in _candidates(prec, grouped=False, nbf=N):
                 _set(fb, cand)
-                fb.timing = False
                 fb.build_JK(Cs, precision=prec)  # warm-up (workspace of this plan)
-                fb.timing = True
-                ms = []
-                for _ in range(reps):
-                    fb.build_JK(Cs, precision=prec)
-                    ms.append(fb.last_timings["total"])
+                ms = [_build_ms(fb, Cs, prec) for _ in range(reps)]
                 t = sorted(ms)[len(ms) // 2]
                 if best is None or t < best["ms"]:
                     best = dict(cand, ms=t)
-            fb.timing = False
             table[_key(N, Q, prec)] = best
             if log:
                 log(f"[autotune] N={N} Q={Q} o={o} {prec}: {best}")
