@@ -1669,7 +1669,11 @@ int f2jk_half_transform(f2jk_ctx* ctx, const double* C, int64_t ncol, int64_t ld
 
 // Scratch of f2jk_mo_block: both coefficient sets, and the intermediate of one
 // block of P.  64 MB of it: what the first product writes the second one then
-// reads from the last-level cache.
+// reads from the last-level cache.  More where 64 MB give either launch less
+// than one round of workgroups (100 to 200 of the 512 for wide sets at nbf 500
+// and above), up to 512 MB: nbf 640 with 128 + 128 columns 4.52 ms with 64 MB,
+// 3.57 with this (4.02 with at most 256 MB), 320 + 320 13.96 and 10.7, 640 + 640
+// 35.8 and 28.9, nbf 499 with 99 + 99 2.46 and 1.77.
 namespace {
 struct MoPlan {
     Plan c[2];           // coefficient packing of C1 and C2
@@ -1677,7 +1681,7 @@ struct MoPlan {
     int64_t step;        // P per block
     size_t off_c[2], off_t, total;
 };
-constexpr size_t kMoBlockBytes = size_t(64) << 20;
+constexpr size_t kMoBlockBytes = size_t(64) << 20, kMoBlockMaxBytes = size_t(512) << 20;
 int mo_plan(const f2jk_ctx* ctx, int64_t n1, int64_t n2, MoPlan& m) {
     const int64_t n[2] = {n1, n2};
     size_t off = 0;
@@ -1692,7 +1696,14 @@ int mo_plan(const f2jk_ctx* ctx, int64_t n1, int64_t n2, MoPlan& m) {
     const int64_t N = m.c[0].N, Q = m.c[0].Q;
     m.rows_first = n1 < n2;  // the narrow set first: fewer products
     const int64_t per_p = 8 * N * std::min(n1, n2);
-    m.step = std::max<int64_t>(1, std::min<int64_t>({Q, (int64_t)kMoBlockBytes / per_p, INT32_MAX / std::max(N, std::max(n1, n2))}));
+    // workgroups per P of the transform of the row index and of the other one
+    const Plan &p1 = m.c[0], &p2 = m.c[1];
+    const int64_t cols = m.rows_first ? N : n2, rows = m.rows_first ? n1 : N;
+    const double wg = std::min((double)cdiv(cols, 16) / (4 * kxd_ib(p1.dnb)) * p1.dncolt,
+                               (double)rows / (64 * kxd_ib(p2.dnb)) * p2.dncolt);
+    const int64_t step = std::max((int64_t)kMoBlockBytes / per_p,
+                                  std::min((int64_t)(kDSlots / wg), (int64_t)kMoBlockMaxBytes / per_p));
+    m.step = std::max<int64_t>(1, std::min<int64_t>({Q, step, INT32_MAX / std::max(N, std::max(n1, n2))}));
     m.off_t = off;
     off += align_up((size_t)(m.step * per_p));
     m.total = off;
