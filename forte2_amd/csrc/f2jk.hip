@@ -1120,8 +1120,19 @@ int fit_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision,
         Plan p;
         int rc = make_plan(ctx, ndens, nocc, precision, flags, true, p, 0, false, &caps);
         if (rc) return rc;
-        if (p.total <= budget) return F2JK_OK;
         const size_t per_p = p.per_p;
+        if (p.total <= budget) {
+            // a chunk that was halved may have missed the array by little (nbf 384,
+            // 76 columns: 139 P at 67.3 of 67.1 MB, then 68 P at 46): three more tries
+            for (int q = 7; it > 0 && p.want_k && p.nchunks > 1 && q > 4; --q) {
+                const PlanCaps more{std::min(ctx->xchunk_bytes, per_p * ((size_t)p.Pc * q / 4)), caps.target_blocks};
+                Plan r;
+                if (make_plan(ctx, ndens, nocc, precision, flags, true, r, 0, false, &more) || r.total > budget) continue;
+                caps = more;
+                break;
+            }
+            return F2JK_OK;
+        }
         if (p.want_k && p.Pc > 1 && p.x_bytes >= p.jpart_bytes + p.kpart_bytes)
             caps.xchunk_bytes = per_p * (size_t)(p.Pc / 2);
         else if (caps.target_blocks > 1)
