@@ -34,6 +34,7 @@
 // with a full drain before its barrier; the loads have had the whole step.
 #pragma once
 #include "f2jk_kernels.h"
+#include "f2jk_tiles.h"
 
 namespace f2jk {
 
@@ -423,20 +424,12 @@ __global__ __launch_bounds__(256) void gamma_rows_kernel(const double* __restric
 }
 
 // ---------------------------------------------------------------------------
-// Contraction.  The lower triangle of K is cut into 128 x 128 tiles of 8 x 8
-// blocks; the last tile row has rl <= 8 blocks.  Four kinds of tiles, by the
-// blocks of their busiest wave (cost): 0 full (16), 1 diagonal (9), 2 last
-// row, 3 last diagonal.  Tiles of kind k split the P range in ns[k] parts.  Workgroups are numbered by the position
-// of their P range, so that those which read the same X run together.
+// Contraction.  The lower triangle of K is cut into 128 x 128 tiles (DTiles).
+// Tiles of kind k split the P range in ns[k] parts.  Workgroups are numbered by
+// the position of their P range, so that those which read the same X run
+// together.
 // ---------------------------------------------------------------------------
-struct DTiles {
-    int nt;        // tile rows
-    int rl;        // 16-row blocks of the last tile row
-    int cnt[4];    // tiles of each kind
-    int ns[4];     // P splits of each kind
-    int G;         // max ns of the kinds present
-    int total;     // workgroups: sum cnt * ns
-};
+static_assert(kDTileEdge == kTile, "one tile edge");
 __host__ __device__ inline int dtile_kind(const DTiles& m, int mt, int nt) {
     return (mt == m.nt - 1 ? 2 : 0) + (mt == nt ? 1 : 0);
 }
