@@ -70,10 +70,10 @@ struct f2jk_ctx {
     bool j_sparse = false;
     uint32_t* jlist[2] = {nullptr, nullptr};
     int* jinv[2] = {nullptr, nullptr};   // lower-triangle element -> place in the list, or -1
-    // the listed elements of a copy one after the other (P-major), when asked for
-    // ("j_pack") and there is room: the J passes then read whole lines
+    // the listed elements of the FP32 copy one after the other (P-major), when asked
+    // for ("j_pack") and there is room: the J passes then read whole lines
     bool j_pack = false;
-    void* jpacked[2] = {nullptr, nullptr};
+    void* jpacked = nullptr;
     int jlist_vec[2] = {0, 0};
     int jlist_n[2] = {0, 0};
     size_t xchunk_bytes = kDefaultXChunkBytes;
@@ -86,7 +86,7 @@ struct f2jk_ctx {
     int ks_tile = 0;                // BF16x3 contraction tile edge: 128, 256, 0 = by nbf
     int kx_rows = 0;                // BF16x3 half-transform tile rows: 128, 256, 0 = by nbf
     int ks_dma = -1;                // BF16x3 contraction tiles by direct-to-LDS loads: 0, 1, -1 = with 256 tiles
-    int kx_wide = -1;               // FP64/FP32 half-transform in 320-column tiles: 0, 1, -1 = above 128 columns
+    int kx_wide = -1;               // FP32 half-transform in 320-column tiles: 0, 1, -1 = above 128 columns
     hipStream_t side = nullptr;     // default priority, created with the context
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     std::mutex ev_mu;               // an event is recorded and waited on in one piece
@@ -182,55 +182,51 @@ int scan_jlist(f2jk_ctx* ctx, const TB* B, unsigned char* flag) {
     return F2JK_OK;
 }
 
-template <typename TB, int VEC>
-int pack_jlist(f2jk_ctx* ctx, int dtype, const TB* B) {
-    const int n = ctx->jlist_n[dtype];
+template <int VEC>
+int pack_jlist(f2jk_ctx* ctx) {
+    const int n = ctx->jlist_n[F2JK_F32];
     const unsigned ny = (unsigned)std::max<int64_t>(1, std::min<int64_t>(ctx->naux, 128));
-    hipLaunchKernelGGL((j_pack_kernel<TB, VEC>), dim3((unsigned)cdiv(n, 256), ny), dim3(256), 0, nullptr, B,
-                       (int)ctx->nbf, (int)ctx->naux, ctx->jlist[dtype], n, (TB*)ctx->jpacked[dtype]);
+    hipLaunchKernelGGL((j_pack_kernel<float, VEC>), dim3((unsigned)cdiv(n, 256), ny), dim3(256), 0, nullptr,
+                       (const float*)ctx->B[F2JK_F32], (int)ctx->nbf, (int)ctx->naux, ctx->jlist[F2JK_F32], n,
+                       (float*)ctx->jpacked);
     F2JK_LAUNCHED("j_pack");
     return F2JK_OK;
 }
 
-// the values of copy `dtype` into its packed elements
-int pack_elements(f2jk_ctx* ctx, int dtype) {
-    const int vec = ctx->jlist_vec[dtype];
-    int rc;
-    if (dtype == F2JK_F64)
-        rc = vec == 2 ? pack_jlist<double, 2>(ctx, dtype, (const double*)ctx->B[dtype])
-                      : pack_jlist<double, 1>(ctx, dtype, (const double*)ctx->B[dtype]);
-    else
-        rc = vec == 4 ? pack_jlist<float, 4>(ctx, dtype, (const float*)ctx->B[dtype])
-           : vec == 2 ? pack_jlist<float, 2>(ctx, dtype, (const float*)ctx->B[dtype])
-                      : pack_jlist<float, 1>(ctx, dtype, (const float*)ctx->B[dtype]);
+// the values of the FP32 copy into its packed elements
+int pack_elements(f2jk_ctx* ctx) {
+    const int vec = ctx->jlist_vec[F2JK_F32];
+    const int rc = vec == 4 ? pack_jlist<4>(ctx) : vec == 2 ? pack_jlist<2>(ctx) : pack_jlist<1>(ctx);
     if (rc) return rc;
     F2JK_HIP(hipStreamSynchronize(nullptr));  // builds on any stream read it
     return F2JK_OK;
 }
 
-// The packed elements of copy `dtype`, where they save bytes and a sixteenth of
+// The packed elements of the FP32 copy, where they save bytes and a sixteenth of
 // the free memory holds them (a build that just fits the card keeps its room;
 // the passes give the same J, bitwise, either way).
-int build_jpacked(f2jk_ctx* ctx, int dtype) {
-    const int64_t N = ctx->nbf, n = ctx->jlist_n[dtype];
-    const int vec = ctx->jlist_vec[dtype];
-    const double esize = dtype == F2JK_F64 ? 8.0 : 4.0;
-    const double bytes = (double)n * vec * esize * (double)ctx->naux;
-    if ((double)n * vec > 0.85 * (double)N * (N + 1) / 2) return F2JK_OK;
+int build_jpacked(f2jk_ctx* ctx) {
+    const int64_t N = ctx->nbf, elements = (int64_t)ctx->jlist_n[F2JK_F32] * ctx->jlist_vec[F2JK_F32];
+    const double bytes = (double)elements * 4.0 * (double)ctx->naux;
+    if ((double)elements > 0.85 * (double)N * (N + 1) / 2) return F2JK_OK;
     size_t free_b = 0, total_b = 0;
     F2JK_HIP(hipMemGetInfo(&free_b, &total_b));
     if (bytes > (double)free_b / 16) return F2JK_OK;
-    if (hipMalloc(&ctx->jpacked[dtype], (size_t)bytes) != hipSuccess) {
+    if (hipMalloc(&ctx->jpacked, (size_t)bytes) != hipSuccess) {
         (void)hipGetLastError();
-        ctx->jpacked[dtype] = nullptr;
+        ctx->jpacked = nullptr;
         return F2JK_OK;
     }
-    return pack_elements(ctx, dtype);
+    return pack_elements(ctx);
+}
+
+void free_jpacked(f2jk_ctx* ctx) {
+    if (ctx->jpacked) (void)hipFree(ctx->jpacked);
+    ctx->jpacked = nullptr;
 }
 
 void free_jlist(f2jk_ctx* ctx, int dtype) {
-    if (ctx->jpacked[dtype]) (void)hipFree(ctx->jpacked[dtype]);
-    ctx->jpacked[dtype] = nullptr;
+    if (dtype == F2JK_F32) free_jpacked(ctx);
     if (ctx->jlist[dtype]) (void)hipFree(ctx->jlist[dtype]);
     if (ctx->jinv[dtype]) (void)hipFree(ctx->jinv[dtype]);
     ctx->jlist[dtype] = nullptr;
@@ -278,7 +274,7 @@ int build_jlist(f2jk_ctx* ctx, int dtype) {
     F2JK_HIP(hipMemcpy(ctx->jinv[dtype], inv.data(), inv.size() * sizeof(int), hipMemcpyHostToDevice));
     ctx->jlist_vec[dtype] = vec;
     ctx->jlist_n[dtype] = (int)list.size();
-    if (ctx->j_pack && dtype == F2JK_F32) return build_jpacked(ctx, dtype);
+    if (ctx->j_pack && dtype == F2JK_F32) return build_jpacked(ctx);
     return F2JK_OK;
 }
 
@@ -382,7 +378,7 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
         if (!grouped && ctx->jlist[jdtype] && ctx->jlist_vec[jdtype] == p.jvec) {
             p.jlist = ctx->jlist[jdtype];
             p.jinv = ctx->jinv[jdtype];
-            p.jpacked = ctx->jpacked[jdtype];
+            if (jdtype == F2JK_F32) p.jpacked = ctx->jpacked;
             nvec = ctx->jlist_n[jdtype];
         }
         p.nvec = (int)nvec;
@@ -454,10 +450,7 @@ int make_plan(const f2jk_ctx* ctx, int ndens, const int64_t* nocc, int precision
             p.kx_wide = !grouped && (ctx->kx_wide < 0 ? p.OPAD > kTile : ctx->kx_wide == 1);
             p.ncolt = (int)cdiv(p.OPAD, p.kx_wide ? kWideCols : kTile);
         }
-        if (p.tk == 8)
-            p.kva = (N % 2 == 0) ? 2 : 1;
-        else
-            p.kva = (N % 4 == 0) ? 4 : ((N % 2 == 0) ? 2 : 1);
+        p.kva = (N % 4 == 0) ? 4 : ((N % 2 == 0) ? 2 : 1);
         p.off_x = off;
         p.x_bytes = align_up((size_t)p.Pc * per_p);
         off += p.x_bytes;
@@ -658,22 +651,22 @@ void launch_kx_fp32(const Plan& p, unsigned grid, const float* A, int64_t R, con
                     hipStream_t st) {
     if (p.kx_wide) {
         if (p.kva == 4)
-            hipLaunchKernelGGL((kx_wide_kernel<float, 4>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
+            hipLaunchKernelGGL((kx_wide_kernel<4>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
                                p.OPAD, X, p.ncolt);
         else if (p.kva == 2)
-            hipLaunchKernelGGL((kx_wide_kernel<float, 2>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
+            hipLaunchKernelGGL((kx_wide_kernel<2>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
                                p.OPAD, X, p.ncolt);
         else
-            hipLaunchKernelGGL((kx_wide_kernel<float, 1>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
+            hipLaunchKernelGGL((kx_wide_kernel<1>), dim3(grid), dim3(kWideThreads), 0, st, A, R, p.N, cp,
                                p.OPAD, X, p.ncolt);
     } else if (p.kva == 4) {
-        hipLaunchKernelGGL((kx_kernel<float, 4>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
+        hipLaunchKernelGGL((kx_kernel<4>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
                            p.ncolt);
     } else if (p.kva == 2) {
-        hipLaunchKernelGGL((kx_kernel<float, 2>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
+        hipLaunchKernelGGL((kx_kernel<2>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
                            p.ncolt);
     } else {
-        hipLaunchKernelGGL((kx_kernel<float, 1>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
+        hipLaunchKernelGGL((kx_kernel<1>), dim3(grid), dim3(kGThreads), 0, st, A, R, p.N, cp, p.OPAD, X,
                            p.ncolt);
     }
 }
@@ -778,7 +771,7 @@ int run_k_typed(f2jk_ctx* ctx, const Plan& p, const int64_t* nocc, double* const
             F2JK_LAUNCHED("ks");
         } else {
             for (int d = 0; d < p.nd; ++d) {
-                hipLaunchKernelGGL(ks_kernel<T>, dim3(p.nlower * nsplit), dim3(kGThreads), 0, st, X, p.N,
+                hipLaunchKernelGGL(ks_kernel, dim3(p.nlower * nsplit), dim3(kGThreads), 0, st, X, p.N,
                                    p.OPAD, p.ioff[d], p.width[d], pc, nsplit, p.nlower,
                                    kpart + (size_t)d * p.nsplit * NN, c > 0 ? 1 : 0);
                 F2JK_LAUNCHED("ks");
@@ -1307,12 +1300,11 @@ int f2jk_set_tuning(f2jk_ctx* ctx, const char* key, int64_t value) {
         F2JK_HIP(hipSetDevice(ctx->device));
         if (ctx->j_pack && ctx->jlist[F2JK_F32]) {
             F2JK_HIP(hipDeviceSynchronize());  // builds that read them, writes to B on any stream
-            int rc = ctx->jpacked[F2JK_F32] ? pack_elements(ctx, F2JK_F32) : build_jpacked(ctx, F2JK_F32);
+            int rc = ctx->jpacked ? pack_elements(ctx) : build_jpacked(ctx);
             if (rc) return rc;
-        } else if (!ctx->j_pack && ctx->jpacked[F2JK_F32]) {
+        } else if (!ctx->j_pack && ctx->jpacked) {
             F2JK_HIP(hipDeviceSynchronize());
-            (void)hipFree(ctx->jpacked[F2JK_F32]);
-            ctx->jpacked[F2JK_F32] = nullptr;
+            free_jpacked(ctx);
         }
     } else if (!strcmp(key, "ks_dma")) {
         if (value < -1 || value > 1) return fail(F2JK_EINVAL, "ks_dma must be -1, 0 or 1");
@@ -1538,9 +1530,6 @@ int f2jk_group_build_jk(f2jk_ctx* const* ctxs, int njobs, const int* ndens, cons
         g.nlower = p.nlower;
         g.nsplit = std::min(p.nsplit, std::min(p.Pc, p.Q));
         g.ncolt = (precision == F2JK_PREC_BF16X3) ? (int)cdiv(p.OPAD, 32 * nbw) : p.ncolt;
-        // the D-build tiles use the same lower-tile count as the K tiles
-        if (p.nlower != (int)(cdiv(p.N, kTile) * (cdiv(p.N, kTile) + 1) / 2))
-            return fail(F2JK_EINVAL, "inconsistent tile plan");
     }
     // the longest jobs first: a launch starts its blocks in this order and ends
     // with short ones

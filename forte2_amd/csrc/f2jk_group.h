@@ -104,8 +104,9 @@ struct GKxd {
     int N, nks, OPAD, ncolt;
     DCols2 dc;
 };
-// MAXNB 8: narrow jobs only, one row block per wave (114 registers and 32 KB
-// of LDS: four workgroups per CU); 20: every width (256 registers, two).
+// MAXNB 8: narrow jobs only, one row block per wave (116 registers and 32 KB of
+// LDS: four workgroups per CU); 20: every width (235 registers, two).  A group
+// with one job of more than 128 columns runs all its jobs in the second.
 constexpr int kGroupNarrowNB = 8;
 constexpr int grouped_kxd_ib(int maxnb, int nb) { return maxnb == kGroupNarrowNB ? 1 : kxd_ib(nb); }
 template <int MAXNB, int NB = 1>
@@ -221,7 +222,7 @@ void grouped_kernel(const GArgs a) {
                              DCols2{g.nd, g.ioff[0], g.ioff[0] + g.width[0], g.ioff[1], g.ioff[1] + g.width[1]}};
                 grouped_kxd<NBW>(lds, g.dnb, k, local, nb);
             } else if constexpr (PREC == F2JK_PREC_FP32) {
-                kx_kernel_body<float, 2>((const float*)g.B, R, g.N, g.Cp32, g.OPAD, (float*)g.X, g.ncolt, local, nb);
+                kx_kernel_body<2>((const float*)g.B, R, g.N, g.Cp32, g.OPAD, (float*)g.X, g.ncolt, local, nb);
             } else {
                 u16* xh = (u16*)g.X;
                 kx_bf16x3_kernel_body<NBW, VA>((const float*)g.B, R, g.N, g.KP, g.Cth, g.Ctl, g.OPAD, xh,
@@ -239,7 +240,7 @@ void grouped_kernel(const GArgs a) {
                 __shared__ __attribute__((aligned(16))) char lds[kDKsLds];
                 ksd_body(lds, (const double*)g.X, g.N, g.OPAD, g.ioff[d], g.width[d], g.Q, g.dt, kp, 0, b);
             } else {
-                ks_kernel_body<TB>((const TB*)g.X, g.N, g.OPAD, g.ioff[d], g.width[d], g.Q, g.nsplit, g.nlower,
+                ks_kernel_body((const float*)g.X, g.N, g.OPAD, g.ioff[d], g.width[d], g.Q, g.nsplit, g.nlower,
                                    kp, 0, b, per);
             }
         }

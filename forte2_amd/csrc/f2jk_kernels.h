@@ -495,37 +495,26 @@ __device__ __forceinline__ dx4 mfma4(double a, double b, dx4 c) {
 __device__ __forceinline__ fx4 mfma4(float a, float b, fx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-template <typename T>
-struct Acc;
-template <>
-struct Acc<double> {
-    typedef dx4 type;
-};
-template <>
-struct Acc<float> {
-    typedef fx4 type;
-};
 
 constexpr int kTile = 128;   // output tile edge (rows and columns)
 constexpr int kBK = 16;      // k extent of one LDS stage
 constexpr int kGThreads = 256;
 
 // ---------------------------------------------------------------------------
-// KX:  X[r][c] = sum_k A[r][k] Cp[k][c]
+// KX (FP32):  X[r][c] = sum_k A[r][k] Cp[k][c]
 //   A  = B of the chunk viewed as R x K row-major (R = Pc*N rows, K = N)
 //   Cp = K x OPAD row-major (zero-padded columns), X = R x OPAD row-major.
 // Tile 128 x 128, 4 waves as 2 x 2 blocks of 64 x 64 (4 x 4 MFMA blocks each).
 // VA: elements per global load of A (16 B when the row length allows).
 // ---------------------------------------------------------------------------
-template <typename T, int VA>
-__device__ __forceinline__ void kx_kernel_body(const T* __restrict__ A, int64_t R,
-                                                       int K, const T* __restrict__ Cp,
-                                                       int OPAD, T* __restrict__ X,
+template <int VA>
+__device__ __forceinline__ void kx_kernel_body(const float* __restrict__ A, int64_t R,
+                                                       int K, const float* __restrict__ Cp,
+                                                       int OPAD, float* __restrict__ X,
                                                        int ncolt, int b, int nblocks) {
-    typedef typename Acc<T>::type acc_t;
-    constexpr int VB = 16 / sizeof(T);       // B tile loads are always 16 B (OPAD % 16 == 0)
-    __shared__ T As[2][kTile][kBK + 1];  // two stages: MFMAs read one, the next k-step fills the other
-    __shared__ T Bs[2][kBK][kTile];
+    constexpr int VB = 4;       // B tile loads are always 16 B (OPAD % 16 == 0)
+    __shared__ float As[2][kTile][kBK + 1];  // two stages: MFMAs read one, the next k-step fills the other
+    __shared__ float Bs[2][kBK][kTile];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
@@ -539,8 +528,8 @@ __device__ __forceinline__ void kx_kernel_body(const T* __restrict__ A, int64_t 
 
     constexpr int A_LD = (kTile * kBK) / (kGThreads * VA);  // loads per thread
     constexpr int B_LD = (kTile * kBK) / (kGThreads * VB);
-    Vec<T, VA> ra[A_LD];
-    Vec<T, VB> rb[B_LD];
+    Vec<float, VA> ra[A_LD];
+    Vec<float, VB> rb[B_LD];
 
     auto load_tiles = [&](int k0) {
 #pragma unroll
@@ -550,10 +539,10 @@ __device__ __forceinline__ void kx_kernel_body(const T* __restrict__ A, int64_t 
             const int64_t gr = r0 + row;
             const int gk = k0 + kc;
             if (gr < R && gk < K) {
-                ra[s] = load_vec<T, VA>(A + gr * K + gk);
+                ra[s] = load_vec<float, VA>(A + gr * K + gk);
             } else {
 #pragma unroll
-                for (int v = 0; v < VA; ++v) ra[s].v[v] = T(0);
+                for (int v = 0; v < VA; ++v) ra[s].v[v] = 0.0f;
             }
         }
 #pragma unroll
@@ -562,10 +551,10 @@ __device__ __forceinline__ void kx_kernel_body(const T* __restrict__ A, int64_t 
             const int kr = idx / (kTile / VB), cc = (idx % (kTile / VB)) * VB;
             const int gk = k0 + kr, gc = c0 + cc;
             if (gk < K && gc < OPAD) {
-                rb[s] = load_vec<T, VB>(Cp + (int64_t)gk * OPAD + gc);
+                rb[s] = load_vec<float, VB>(Cp + (int64_t)gk * OPAD + gc);
             } else {
 #pragma unroll
-                for (int v = 0; v < VB; ++v) rb[s].v[v] = T(0);
+                for (int v = 0; v < VB; ++v) rb[s].v[v] = 0.0f;
             }
         }
     };
@@ -586,11 +575,11 @@ __device__ __forceinline__ void kx_kernel_body(const T* __restrict__ A, int64_t 
         }
     };
 
-    acc_t acc[4][4];
+    fx4 acc[4][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+        for (int j = 0; j < 4; ++j) acc[i][j] = fx4{0, 0, 0, 0};
 
     const int nk = (K + kBK - 1) / kBK;
     load_tiles(0);
@@ -601,7 +590,7 @@ __device__ __forceinline__ void kx_kernel_body(const T* __restrict__ A, int64_t 
         const int cur = kt & 1;
 #pragma unroll
         for (int kk = 0; kk < kBK; kk += 4) {
-            T a[4], b[4];
+            float a[4], b[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) a[i] = As[cur][wr * 64 + i * 16 + (lane & 15)][kk + (lane >> 4)];
 #pragma unroll
@@ -626,38 +615,36 @@ __device__ __forceinline__ void kx_kernel_body(const T* __restrict__ A, int64_t 
             const int col = wcol0 + j * 16 + (lane & 15);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int64_t row = r0 + wr * 64 + i * 16 + acc_row<T>(lane, r);
+                const int64_t row = r0 + wr * 64 + i * 16 + acc_row<float>(lane, r);
                 if (row < R) X[row * OPAD + col] = acc[i][j][r];
             }
         }
 }
-template <typename T, int VA>
-__global__ __launch_bounds__(kGThreads) void kx_kernel(const T* __restrict__ A, int64_t R,
-                                                       int K, const T* __restrict__ Cp,
-                                                       int OPAD, T* __restrict__ X,
+template <int VA>
+__global__ __launch_bounds__(kGThreads) void kx_kernel(const float* __restrict__ A, int64_t R,
+                                                       int K, const float* __restrict__ Cp,
+                                                       int OPAD, float* __restrict__ X,
                                                        int ncolt) {
-    kx_kernel_body<T, VA>(A, R, K, Cp, OPAD, X, ncolt, blockIdx.x, gridDim.x);
+    kx_kernel_body<VA>(A, R, K, Cp, OPAD, X, ncolt, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
-// KX, wide tiles (FP64 / FP32): the product of kx_kernel with 128 x 320
-// output tiles, so that a 128-row block of B is read once for up to 320
-// occupied columns (the 128-column kernel reads it once per column tile: 3x
-// at 320 columns).  8 waves as 2 x 4, each 64 x 80 (4 x 5 MFMA blocks, 160
-// accumulator registers in FP64), one workgroup per CU.  The k loop, the
-// MFMA and each output element's accumulation order are those of kx_kernel,
-// so X is bitwise the same.  The k-major coefficient tile is padded by 16
+// KX, wide tiles: the product of kx_kernel with 128 x 320 output tiles, so that
+// a 128-row block of B is read once for up to 320 occupied columns (the
+// 128-column kernel reads it once per column tile: 3x at 320 columns).  8 waves
+// as 2 x 4, each 64 x 80 (4 x 5 MFMA blocks), one workgroup per CU.  The k
+// loop, the MFMA and each output element's accumulation order are those of
+// kx_kernel, so X is bitwise the same.  The k-major coefficient tile is padded by 16
 // elements per row: its fragment reads (4 k rows x 16 columns per wave
 // instruction) then fall in distinct LDS banks.
 // ---------------------------------------------------------------------------
 constexpr int kWideCols = 320;
 constexpr int kWideThreads = 512;
 
-template <typename T, int VA>
-__device__ __forceinline__ void kx_wide_body(const T* __restrict__ A, int64_t R, int K,
-                                             const T* __restrict__ Cp, int OPAD, T* __restrict__ X,
+template <int VA>
+__device__ __forceinline__ void kx_wide_body(const float* __restrict__ A, int64_t R, int K,
+                                             const float* __restrict__ Cp, int OPAD, float* __restrict__ X,
                                              int ncolt, int b, int nblocks) {
-    typedef typename Acc<T>::type acc_t;
     constexpr int TN = kWideCols, BS = TN + 16;
     constexpr int WC = 4, NB = TN / WC / 16;       // 5 column blocks per wave
     constexpr int VB = 2;                          // coefficient loads: 2 elements each
@@ -665,8 +652,8 @@ __device__ __forceinline__ void kx_wide_body(const T* __restrict__ A, int64_t R,
     constexpr int B_LD = (kBK * TN) / (kWideThreads * VB);
     static_assert(A_LD * kWideThreads * VA == kTile * kBK && B_LD * kWideThreads * VB == kBK * TN,
                   "tiles must split evenly over the threads");
-    __shared__ T As[2][kTile][kBK + 1];
-    __shared__ T Bs[2][kBK][BS];
+    __shared__ float As[2][kTile][kBK + 1];
+    __shared__ float Bs[2][kBK][BS];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -678,8 +665,8 @@ __device__ __forceinline__ void kx_wide_body(const T* __restrict__ A, int64_t R,
     int nbv = (OPAD - wcol0) / 16;
     nbv = nbv < 0 ? 0 : (nbv > NB ? NB : nbv);
 
-    Vec<T, VA> ra[A_LD];
-    Vec<T, VB> rb[B_LD];
+    Vec<float, VA> ra[A_LD];
+    Vec<float, VB> rb[B_LD];
     auto load_tiles = [&](int k0) {
 #pragma unroll
         for (int s = 0; s < A_LD; ++s) {
@@ -688,10 +675,10 @@ __device__ __forceinline__ void kx_wide_body(const T* __restrict__ A, int64_t R,
             const int64_t gr = r0 + row;
             const int gk = k0 + kc;
             if (gr < R && gk < K) {
-                ra[s] = load_vec<T, VA>(A + gr * K + gk);
+                ra[s] = load_vec<float, VA>(A + gr * K + gk);
             } else {
 #pragma unroll
-                for (int v = 0; v < VA; ++v) ra[s].v[v] = T(0);
+                for (int v = 0; v < VA; ++v) ra[s].v[v] = 0.0f;
             }
         }
 #pragma unroll
@@ -700,10 +687,10 @@ __device__ __forceinline__ void kx_wide_body(const T* __restrict__ A, int64_t R,
             const int kr = idx / (TN / VB), cc = (idx % (TN / VB)) * VB;
             const int gk = k0 + kr, gc = c0 + cc;
             if (gk < K && gc < OPAD) {
-                rb[s] = load_vec<T, VB>(Cp + (int64_t)gk * OPAD + gc);
+                rb[s] = load_vec<float, VB>(Cp + (int64_t)gk * OPAD + gc);
             } else {
 #pragma unroll
-                for (int v = 0; v < VB; ++v) rb[s].v[v] = T(0);
+                for (int v = 0; v < VB; ++v) rb[s].v[v] = 0.0f;
             }
         }
     };
@@ -724,11 +711,11 @@ __device__ __forceinline__ void kx_wide_body(const T* __restrict__ A, int64_t R,
         }
     };
 
-    acc_t acc[4][NB];
+    fx4 acc[4][NB];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+        for (int j = 0; j < NB; ++j) acc[i][j] = fx4{0, 0, 0, 0};
 
     const int nk = (K + kBK - 1) / kBK;
     load_tiles(0);
@@ -739,7 +726,7 @@ __device__ __forceinline__ void kx_wide_body(const T* __restrict__ A, int64_t R,
         const int cur = kt & 1;
 #pragma unroll
         for (int kk = 0; kk < kBK; kk += 4) {
-            T a[4], bv[NB];
+            float a[4], bv[NB];
 #pragma unroll
             for (int i = 0; i < 4; ++i) a[i] = As[cur][wr * 64 + i * 16 + (lane & 15)][kk + (lane >> 4)];
 #pragma unroll
@@ -764,33 +751,31 @@ __device__ __forceinline__ void kx_wide_body(const T* __restrict__ A, int64_t R,
             const int col = wcol0 + j * 16 + (lane & 15);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int64_t row = r0 + wr * 64 + i * 16 + acc_row<T>(lane, r);
+                const int64_t row = r0 + wr * 64 + i * 16 + acc_row<float>(lane, r);
                 if (row < R) X[row * OPAD + col] = acc[i][j][r];
             }
         }
 }
-template <typename T, int VA>
-__global__ __launch_bounds__(kWideThreads) void kx_wide_kernel(const T* __restrict__ A, int64_t R, int K,
-                                                               const T* __restrict__ Cp, int OPAD,
-                                                               T* __restrict__ X, int ncolt) {
-    kx_wide_body<T, VA>(A, R, K, Cp, OPAD, X, ncolt, blockIdx.x, gridDim.x);
+template <int VA>
+__global__ __launch_bounds__(kWideThreads) void kx_wide_kernel(const float* __restrict__ A, int64_t R, int K,
+                                                               const float* __restrict__ Cp, int OPAD,
+                                                               float* __restrict__ X, int ncolt) {
+    kx_wide_body<VA>(A, R, K, Cp, OPAD, X, ncolt, blockIdx.x, gridDim.x);
 }
 
 
 // ---------------------------------------------------------------------------
-// KS:  Kpart[s][m][n] (+)= sum_{P in split s} sum_{i < width} X[P][m][ioff+i] X[P][n][ioff+i]
+// KS (FP32):  Kpart[s][m][n] (+)= sum_{P in split s} sum_{i < width} X[P][m][ioff+i] X[P][n][ioff+i]
 // Only lower tiles (mt >= nt) are computed.  grid = nlower * nsplit.
-// FP32 inputs accumulate each P in FP32 and fold it into FP64 registers.
+// Each P is accumulated in FP32 and folded into FP64 registers.
 // ---------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ void ks_kernel_body(const T* __restrict__ X, int N, int OPAD,
+__device__ __forceinline__ void ks_kernel_body(const float* __restrict__ X, int N, int OPAD,
                                                        int ioff, int width, int Pc, int nsplit,
                                                        int nlower, double* __restrict__ Kpart,
                                                        int accumulate, int b, int nblocks) {
-    typedef typename Acc<T>::type acc_t;
-    constexpr int VA = 16 / sizeof(T);
-    __shared__ T As[2][kTile][kBK + 1];  // two LDS stages
-    __shared__ T Bs[2][kTile][kBK + 1];
+    constexpr int VA = 4;
+    __shared__ float As[2][kTile][kBK + 1];  // two LDS stages
+    __shared__ float Bs[2][kTile][kBK + 1];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
@@ -806,25 +791,25 @@ __device__ __forceinline__ void ks_kernel_body(const T* __restrict__ X, int N, i
     const int Pb = (int)(((int64_t)Pc * (s + 1)) / nsplit);
 
     constexpr int LD = (kTile * kBK) / (kGThreads * VA);
-    Vec<T, VA> ra[LD], rb[LD];
+    Vec<float, VA> ra[LD], rb[LD];
 
     auto load_tiles = [&](int P, int i0) {
-        const T* XP = X + (int64_t)P * N * OPAD + ioff + i0;
+        const float* XP = X + (int64_t)P * N * OPAD + ioff + i0;
 #pragma unroll
         for (int q = 0; q < LD; ++q) {
             const int idx = tid + kGThreads * q;
             const int row = idx / (kBK / VA), kc = (idx % (kBK / VA)) * VA;
             if (m0 + row < N) {
-                ra[q] = load_vec<T, VA>(XP + (int64_t)(m0 + row) * OPAD + kc);
+                ra[q] = load_vec<float, VA>(XP + (int64_t)(m0 + row) * OPAD + kc);
             } else {
 #pragma unroll
-                for (int v = 0; v < VA; ++v) ra[q].v[v] = T(0);
+                for (int v = 0; v < VA; ++v) ra[q].v[v] = 0.0f;
             }
             if (n0 + row < N) {
-                rb[q] = load_vec<T, VA>(XP + (int64_t)(n0 + row) * OPAD + kc);
+                rb[q] = load_vec<float, VA>(XP + (int64_t)(n0 + row) * OPAD + kc);
             } else {
 #pragma unroll
-                for (int v = 0; v < VA; ++v) rb[q].v[v] = T(0);
+                for (int v = 0; v < VA; ++v) rb[q].v[v] = 0.0f;
             }
         }
     };
@@ -842,13 +827,13 @@ __device__ __forceinline__ void ks_kernel_body(const T* __restrict__ X, int N, i
     };
 
     dx4 acc64[4][4];
-    acc_t acc[4][4];
+    fx4 acc[4][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             acc64[i][j] = dx4{0, 0, 0, 0};
-            acc[i][j] = acc_t{0, 0, 0, 0};
+            acc[i][j] = fx4{0, 0, 0, 0};
         }
 
     const int nkp = width / kBK;  // k steps per P (width % 16 == 0)
@@ -864,7 +849,7 @@ __device__ __forceinline__ void ks_kernel_body(const T* __restrict__ X, int N, i
         const int cur = st & 1;
 #pragma unroll
         for (int kk = 0; kk < kBK; kk += 4) {
-            T a[4], b[4];
+            float a[4], b[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) a[i] = As[cur][wr * 64 + i * 16 + (lane & 15)][kk + (lane >> 4)];
 #pragma unroll
@@ -877,25 +862,17 @@ __device__ __forceinline__ void ks_kernel_body(const T* __restrict__ X, int N, i
         if (st + 1 < nsteps) store_tiles(cur ^ 1);
         if (st + 2 < nsteps) load_step(st + 2);
         __syncthreads();
-        if constexpr (sizeof(T) == 4) {
-            if ((st + 1) % nkp == 0) {  // end of one P: fold FP32 partials into FP64
+        if ((st + 1) % nkp == 0) {  // end of one P: fold FP32 partials into FP64
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
+                for (int j = 0; j < 4; ++j) {
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) acc64[i][j][r] += (double)acc[i][j][r];
-                        acc[i][j] = acc_t{0, 0, 0, 0};
-                    }
-            }
+                    for (int r = 0; r < 4; ++r) acc64[i][j][r] += (double)acc[i][j][r];
+                    acc[i][j] = fx4{0, 0, 0, 0};
+                }
         }
     }
-    auto outval = [&](int i, int j, int r) -> double {
-        if constexpr (sizeof(T) == 8)
-            return acc[i][j][r];
-        else
-            return acc64[i][j][r];
-    };
     double* Ks = Kpart + (int64_t)s * N * N;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -905,22 +882,21 @@ __device__ __forceinline__ void ks_kernel_body(const T* __restrict__ X, int N, i
             if (col >= N) continue;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = m0 + wr * 64 + i * 16 + acc_row<T>(lane, r);
+                const int row = m0 + wr * 64 + i * 16 + acc_row<float>(lane, r);
                 if (row >= N) continue;
                 double* dst = Ks + (int64_t)row * N + col;
-                const double v = outval(i, j, r);
+                const double v = acc64[i][j][r];
                 *dst = accumulate ? (*dst + v) : v;
             }
         }
 }
 // two workgroups per CU: 4 waves of one workgroup leave each SIMD idle at the
 // k-step barrier and the LDS-read latency
-template <typename T>
-__global__ __launch_bounds__(kGThreads, 2) void ks_kernel(const T* __restrict__ X, int N, int OPAD,
+__global__ __launch_bounds__(kGThreads, 2) void ks_kernel(const float* __restrict__ X, int N, int OPAD,
                                                        int ioff, int width, int Pc, int nsplit,
                                                        int nlower, double* __restrict__ Kpart,
                                                        int accumulate) {
-    ks_kernel_body<T>(X, N, OPAD, ioff, width, Pc, nsplit, nlower, Kpart, accumulate, blockIdx.x, gridDim.x);
+    ks_kernel_body(X, N, OPAD, ioff, width, Pc, nsplit, nlower, Kpart, accumulate, blockIdx.x, gridDim.x);
 }
 
 
