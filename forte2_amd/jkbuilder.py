@@ -50,7 +50,8 @@ class FockBuilder:
         (forte2/jkbuilder/jkbuilder.py:46-50).  The device kernels read the
         (P, m, n) layout directly, so no transposed copy is ever made.
     B : array or tensor (naux, nbf, nbf), optional
-        A ready B tensor (e.g. from a previous run); copied to the device.
+        A ready B tensor (e.g. from a previous run), symmetric in its last two
+        indices; copied to the device.
     precision : {"fp64", "fp32", "bf16x3"}
         Arithmetic of ``build_*`` calls (see include/f2jk.h).  fp32/bf16x3
         create an FP32 copy of B next to the FP64 one.

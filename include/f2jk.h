@@ -81,7 +81,10 @@ int f2jk_ctx_destroy(f2jk_ctx* ctx);
 
 /* Register a resident copy of B (borrowed device pointer) of the given dtype.
  * A context may hold one F64 and one F32 copy of the same tensor; both must
- * have the same naux and nbf.  Replaces FockBuilder.B_Pmn
+ * have the same naux and nbf.  B[P] is symmetric for every P, as a fitted B is:
+ * the passes of J read its lower triangle, the half-transform (K, the MO
+ * blocks, and in FP64 the gamma of J that comes with K) all of it.  Replaces
+ * FockBuilder.B_Pmn
  * (forte2/jkbuilder/jkbuilder.py:52-72) and B_nPm (:74-80); the transposed
  * copy is not needed. */
 int f2jk_set_B(f2jk_ctx* ctx, int dtype, const void* B, int64_t naux, int64_t nbf);
@@ -97,10 +100,10 @@ int f2jk_get_shape(const f2jk_ctx* ctx, int64_t* naux, int64_t* nbf);
  * -1; default -1 = FP64 J and K from C, and BF16x3 with 256-wide contraction
  * tiles, when a J pass reads 128 MB or more, F2JK_TIMING is not asked for and
  * the stream is not being captured) runs the J passes of a build_jk on the
- * context's side stream concurrently with K (joined back before the call returns its work to the
- * caller's stream); "bf16_nbw_max" (2, 4, 5, 6, 8, 10) caps the BF16x3
- * half-transform tile at 32 * value occupied columns (tiles of up to 5 run two
- * workgroups per CU); "kx_waves" (4 or 8, default 8) is the number of waves of
+ * context's side stream concurrently with K (joined back before the call
+ * returns its work to the caller's stream); "bf16_nbw_max" (2, 4, 5, 6, 8, 10) caps the BF16x3
+ * half-transform tile at 32 * value occupied columns (128-row tiles of up to 5
+ * run two workgroups per CU); "kx_waves" (4 or 8, default 8) is the number of waves of
  * a BF16x3 half-transform workgroup (8: two per SIMD sharing the tile; tiles
  * of an even number of 32-column units); "ks_tile" (0, 128, 256; default 0 =
  * 256 when nbf >= 768) is the lower-tile edge of the single-job BF16x3
