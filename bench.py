@@ -47,7 +47,8 @@ HBM_PEAK_GBS = 8000.0
 # the kernel sources it was measured on: a table measured on other sources is
 # not reported (traffic null).
 TRAFFIC_TABLE = os.path.join(ROOT, "forte2_amd", "data", "traffic_gfx950.json")
-KERNEL_SOURCES = ("forte2_amd/csrc/f2jk.hip", "forte2_amd/csrc/f2jk_kernels.h", "forte2_amd/csrc/f2jk_group.h")
+KERNEL_SOURCES = tuple(f"forte2_amd/csrc/{f}" for f in ("f2jk.hip", "f2jk_kernels.h", "f2jk_fp64.h", "f2jk_tiles.h",
+                                                        "f2jk_group.h"))
 
 
 def kernel_sources_sha256():

@@ -499,8 +499,8 @@ __device__ __forceinline__ void ksd_body(char* lds, const double* __restrict__ X
     });
     // The k range runs in halves of 8 through the P of the split, one after the
     // other, and a step is any two of them: with steps that ended with their P,
-    // an odd number of halves cost a half-empty step per P (nbf 318, 3 halves
-    // per density: 109 us, the matrix pipes 44% busy).
+    // an odd number of halves cost a half-empty step per P (nbf 318, two
+    // densities of 3 halves: 109 us for both, the matrix pipes 44% busy).
     const int hp = width >> 3, nh = (Pb - Pa) * hp, nsteps = (nh + 1) >> 1;
     int Pn = Pa, kn = wid & 1, ln = wid & 1;  // the half this wave loads next: its P, place in P, number
     while (kn >= hp) kn -= hp, ++Pn;
