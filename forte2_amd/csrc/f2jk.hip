@@ -543,7 +543,8 @@ int launch_j(f2jk_ctx* ctx, const Plan& p, const TB* B, int d0, const double* co
     hipLaunchKernelGGL((j_accum_kernel<TB, VEC, kEPT, ND, NT>), dim3(p.neg, p.npc2), dim3(kJThreads), 0,
                        st, B, p.N, p.Q, gamma, rowoff, elist, (const TB*)p.jpacked, p.nvec, p.ppw2, jpart);
     F2JK_LAUNCHED("j_accum");
-    hipLaunchKernelGGL((j_reduce_kernel<VEC, ND>), j_reduce_grid(p.jdense), dim3(kJThreads), 0, st, jpart, p.npc2, p.N, rowoff, p.jinv, p.nvec, p.jdense, jp);
+    hipLaunchKernelGGL((j_reduce_kernel<VEC, ND>), j_reduce_grid(p.jdense), dim3(kJThreads), 0, st, jpart, p.npc2,
+                       p.N, rowoff, p.jinv, p.nvec, p.jdense, jp);
     F2JK_LAUNCHED("j_reduce");
     TIM(F2JK_PH_JACC, false);
     return F2JK_OK;
